@@ -343,7 +343,6 @@ int pms_source_extraction(const float* planes, int n_planes, int h, int w, doubl
   return guarded([&] {
     PMS_REQUIRE(planes && extracted_out && mask_out && work, "NULL buffer");
     PMS_REQUIRE(n_planes >= 1 && h >= 1 && w >= 1, "bad plane stack shape");
-    extract_work_init(work, n_planes, h, w, S(stream));
     source_extract(planes, n_planes, h, w, tolerance, neg_comp, mask_out, extracted_out, labels_out, work, nullptr,
                    S(stream));
   });

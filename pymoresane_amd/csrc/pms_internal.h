@@ -294,7 +294,6 @@ void max_final(const float* pmax, int nb, int S, float* out_max, const double* e
 void max_final(const double* pmax, int nb, int S, double* out_max, const double* energy, double* nsm,
                const int* pred, hipStream_t st);
 size_t extract_work_bytes(int S, int h, int w);
-void extract_work_init(void* work, int S, int h, int w, hipStream_t st);
 void source_extract(const float* w, int S, int h, int wd, double tol, int neg_comp, uint8_t* mask, float* extracted,
                     int* labels_out, void* work, const int* pred, hipStream_t st);
 void source_extract(const double* w, int S, int h, int wd, double tol, int neg_comp, uint8_t* mask,

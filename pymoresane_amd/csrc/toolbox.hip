@@ -421,15 +421,28 @@ __global__ __launch_bounds__(kT) void k_max_final(const T* pmax, int nb, T* out_
 }
 
 // ----------------------------------------------------------------------------- connected components
+// A label word holds the index of the pixel's parent; in a root's own word the top bit is the keep
+// rule's mark (planes hold fewer than 2^31 pixels).  Only set pixels have a label: which pixels are
+// set is kept as one 64-bit word per row and 64 columns (layout (scale, row, word)), an eighth of a
+// byte per pixel, so that every pass after the first reads 1/32 of the planes and touches labels and
+// values of set pixels alone.
+using u64 = unsigned long long;
+constexpr int kMark = (int)0x80000000u;
+constexpr int kCclW = 64, kCclH = 32;  // tile: one row is one wave's ballot
+
+__host__ __device__ __forceinline__ int ccl_words(int wd) { return (wd + kCclW - 1) / kCclW; }
+__host__ __device__ __forceinline__ int ccl_tiles(int h, int wd) { return ccl_words(wd) * ((h + kCclH - 1) / kCclH); }
+
 __device__ __forceinline__ int ccl_find(const int* lab, int x) {
-  int p = lab[x];
+  int p = lab[x] & ~kMark;
   while (p != x) {
     x = p;
-    p = lab[x];
+    p = lab[x] & ~kMark;
   }
   return x;
 }
 
+// before any mark is set
 __device__ __forceinline__ void ccl_union(int* lab, int a, int b) {
   while (true) {
     a = ccl_find(lab, a);
@@ -445,14 +458,6 @@ __device__ __forceinline__ void ccl_union(int* lab, int a, int b) {
     a = old;
   }
 }
-
-// Two-level labelling: each 32x32 tile is labelled in LDS (row runs linked to their first pixel,
-// then union-find with LDS atomicMin links between rows, so every tile component's root is its
-// smallest raster index), the tile roots are written as global
-// raster indices, then only pixels on tile borders union across tiles in global memory.  The final
-// forest, and so the roots, are those of a global union-find: every component's root is its
-// smallest raster index.
-constexpr int kCclTile = 32;
 
 __device__ __forceinline__ int lds_find(const int* L, int x) {
   int p = L[x];
@@ -479,154 +484,244 @@ __device__ __forceinline__ void lds_union(int* L, int a, int b) {
   }
 }
 
-template <class V>
-__global__ __launch_bounds__(kT) void k_ccl_tile(const V* __restrict__ w, int* __restrict__ lab, int h, int wd,
-                                                 const int* pred) {
+// Which unions with the row above a set pixel takes part in, given that its row neighbours are joined
+// already: with the pixel above it, or the one above to the left, only where its run of set pixels
+// starts (otherwise the pixel to the left has made that union), and with the one above to the right
+// only where the pixel above is not set (otherwise both are one run).  m and u are the row's and the
+// upper row's bits, the others those shifted by one pixel.
+__device__ __forceinline__ void ccl_rules(u64 m, u64 left, u64 u, u64 ul, u64 ur, u64* up, u64* upl, u64* upr) {
+  const u64 start = m & ~left;
+  *up = start & u;
+  *upl = start & ~u & ul;
+  *upr = m & ~u & ur;
+}
+
+// Two-level labelling, first level: one block labels a 64 x 32 tile in LDS (row runs linked to their
+// first pixel by bit arithmetic on the row's ballot, then union-find with LDS atomicMin links between
+// rows, so every tile component's root is its smallest raster index), and writes the rows' bit words
+// and, for set pixels, the tile roots as global raster indices; tiles without a set pixel end after
+// the words.  The pass also takes the tile's maximum (of |w| with use_abs), so the planes are read
+// once: eight loads per thread are issued before the first is used.  Bound: reading the planes.  A
+// 32 x 32 tile that wrote a label (or -1) for every pixel took 297 us on seven 4096^2 planes, and the
+// separate maximum pass 111 us more.
+template <class T>
+__global__ __launch_bounds__(kT) void k_ccl_tile(const T* __restrict__ w, int* __restrict__ lab, u64* __restrict__ bits,
+                                                 int h, int wd, int use_abs, T* __restrict__ pmax, const int* pred) {
   if (pred_off(pred)) return;
-  constexpr int T = kCclTile, TT = kCclTile * kCclTile;
-  __shared__ int L[TT];
+  constexpr int TW = kCclW, TH = kCclH, PER = TH / (kT / 64);
+  __shared__ int L[TH * TW];
+  __shared__ u64 rows[TH];
   const int s = blockIdx.y;
-  const int tiles_x = (wd + T - 1) / T;
-  const int r0 = (blockIdx.x / tiles_x) * T, c0 = (blockIdx.x % tiles_x) * T;
+  const int nw = ccl_words(wd);
+  const int cw = blockIdx.x % nw;
+  const int r0 = (blockIdx.x / nw) * TH, c0 = cw * TW;
   const size_t plane = (size_t)h * wd;
-  const V* x = w + (size_t)s * plane;
+  const T* x = w + (size_t)s * plane;
   int* l = lab + (size_t)s * plane;
-  // A tile row is half a wave: one ballot gives each pixel the unset pixels left of it in its row, so
-  // every run of set pixels starts as a tree one link deep under its first pixel (its smallest index)
-  // and row neighbours need no union.
-  static_assert(T == 32 && TT % kT == 0 && kT % 64 == 0, "one tile row per half wave, uniform loop");
-  for (int i = threadIdx.x; i < TT; i += kT) {
-    const int r = r0 + i / T, c = c0 + i % T;
-    const bool on = r < h && c < wd && x[(size_t)r * wd + c] != (V)0;
-    const unsigned long long m = __ballot(on);
-    const int lo = i & 31;  // == this lane's position within its half wave
-    const unsigned gaps = ~(unsigned)(m >> (threadIdx.x & 32)) & ((1u << lo) - 1u);
-    L[i] = on ? i - lo + (gaps ? 32 - __clz(gaps) : 0) : -1;
+  const int lane = threadIdx.x & 63, row0 = (threadIdx.x >> 6) * PER;
+  const int col = c0 + lane;
+  const bool col_ok = col < wd;
+  T v[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int r = r0 + row0 + i;
+    v[i] = x[(size_t)min(r, h - 1) * wd + (col_ok ? col : wd - 1)];
   }
-  __syncthreads();
-  // 8-connected unions with the row above: the pixel above alone when it is set (the diagonal ones
-  // are then in its run), otherwise each diagonal pixel that is set
-  for (int i = threadIdx.x; i < TT; i += kT) {
-    if (L[i] < 0) continue;
-    const int tr = i / T, tc = i % T;
-    if (tr > 0) {
-      const int up = i - T;
-      if (L[up] >= 0) {
-        lds_union(L, i, up);
-      } else {
-        if (tc > 0 && L[up - 1] >= 0) lds_union(L, i, up - 1);
-        if (tc + 1 < T && L[up + 1] >= 0) lds_union(L, i, up + 1);
-      }
+  T m = -INFINITY;
+  u64 any = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int r = r0 + row0 + i;
+    const T a = use_abs ? (T)fabs(v[i]) : v[i];
+    m = a > m ? a : m;  // a dead lane repeats a pixel of the tile
+    const u64 word = __ballot(col_ok && r < h && v[i] != (T)0);
+    any |= word;
+    if (lane == 0) {
+      rows[row0 + i] = word;
+      if (r < h) bits[((size_t)s * h + r) * nw + cw] = word;
+    }
+    if ((word >> lane) & 1) {
+      const u64 gaps = ~word & (((u64)1 << lane) - 1);
+      L[(row0 + i) * TW + lane] = (row0 + i) * TW + (gaps ? 64 - __clzll(gaps) : 0);
     }
   }
+  m = block_max_t<T>(m);
+  if (threadIdx.x == 0) pmax[(size_t)s * gridDim.x + blockIdx.x] = m;
+  if (!__syncthreads_or(any != 0)) return;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int tr = row0 + i;
+    const u64 word = rows[tr];
+    if (tr == 0 || !((word >> lane) & 1)) continue;
+    const u64 u = rows[tr - 1];
+    u64 up, upl, upr;
+    ccl_rules(word, word << 1, u, u << 1, u >> 1, &up, &upl, &upr);
+    const int me = tr * TW + lane;
+    if ((up >> lane) & 1) lds_union(L, me, me - TW);
+    if ((upl >> lane) & 1) lds_union(L, me, me - TW - 1);
+    if ((upr >> lane) & 1) lds_union(L, me, me - TW + 1);
+  }
   __syncthreads();
-  for (int i = threadIdx.x; i < TT; i += kT) {
-    const int r = r0 + i / T, c = c0 + i % T;
-    if (r >= h || c >= wd) continue;
-    int v = L[i];
-    if (v >= 0) {
-      v = lds_find(L, i);
-      v = (r0 + v / T) * wd + (c0 + v % T);
-    }
-    l[(size_t)r * wd + c] = v;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int tr = row0 + i;
+    if (!((rows[tr] >> lane) & 1)) continue;
+    const int root = lds_find(L, tr * TW + lane);
+    l[(size_t)(r0 + tr) * wd + col] = (r0 + root / TW) * wd + c0 + root % TW;
   }
 }
 
-// unions across tile borders (first row, first and last column of each tile)
-// Unions across tile borders.  Only border pixels take part -- every pixel of a row that starts a
-// tile row (r % T == 0, r > 0), and on the other rows the first and last column of each tile -- so
-// one block walks one row at a time and its threads take that row's border pixels, with 32-bit
-// indices (planes hold fewer than 2^29 pixels).  Unions commute: the forest's roots, each
-// component's smallest index, do not depend on their order.
-__global__ __launch_bounds__(kT) void k_ccl_border(int* __restrict__ lab, int h, int wd, const int* pred) {
+// Second level: unions across tile borders, one thread per bit word (a word spans a tile's width), so
+// that pixels without a set neighbour across a border cost no label access.  On the rows that start a
+// tile every pixel looks at the row above; on the others only the word's first and last pixel look at
+// the neighbouring words, and not where the neighbour above or beside them makes the same union.  Unions
+// commute: the roots, each component's smallest index, do not depend on their order.  The last
+// block of a plane reduces the plane's tile maxima instead (smax).  Reading the labels of every tile
+// border took 502 us on seven 4096^2 planes: with 32-pixel tiles that is every line of them.
+template <class T>
+__global__ __launch_bounds__(kT) void k_ccl_border(int* __restrict__ lab, const u64* __restrict__ bits, int h, int wd,
+                                                   const T* __restrict__ pmax, int n_pmax, T* __restrict__ smax,
+                                                   const int* pred) {
   if (pred_off(pred)) return;
-  constexpr int T = kCclTile;
   const int s = blockIdx.y;
+  if (blockIdx.x == gridDim.x - 1) {
+    T m = -INFINITY;
+    for (int i = threadIdx.x; i < n_pmax; i += kT) {
+      const T v = pmax[(size_t)s * n_pmax + i];
+      m = v > m ? v : m;
+    }
+    m = block_max_t<T>(m);
+    if (threadIdx.x == 0) smax[s] = m;
+    return;
+  }
+  const unsigned nw = ccl_words(wd);
+  const unsigned n = (unsigned)h * nw;
   int* l = lab + (size_t)s * h * wd;
-  const int edge_cols = 2 * ((wd + T - 1) / T);  // columns tT and tT + T - 1 of every tile t
-  for (int r = blockIdx.x; r < h; r += gridDim.x) {
-    const bool top = r > 0 && r % T == 0;
-    const int n = top ? wd : edge_cols;
-    for (int k = threadIdx.x; k < n; k += kT) {
-      const int c = top ? k : (k >> 1) * T + ((k & 1) ? T - 1 : 0);
-      if (c >= wd) continue;
-      const int cr = c % T;
-      const bool left = c > 0 && cr == 0, right = cr == T - 1;
-      const int me = r * wd + c;
-      if (!(top || left || right) || l[me] < 0) continue;
-      if (left && l[me - 1] >= 0) ccl_union(l, me, me - 1);
-      if (r > 0) {
-        const int up = me - wd;
-        if (c > 0 && (top || left) && l[up - 1] >= 0) ccl_union(l, me, up - 1);
-        if (top && l[up] >= 0) ccl_union(l, me, up);
-        if (c + 1 < wd && (top || right) && l[up + 1] >= 0) ccl_union(l, me, up + 1);
+  const u64* b = bits + (size_t)s * n;
+  for (unsigned i = blockIdx.x * kT + threadIdx.x; i < n; i += (gridDim.x - 1) * kT) {
+    const u64 m = b[i];
+    if (m == 0) continue;
+    const int r = (int)(i / nw), cw = (int)(i - (unsigned)r * nw);
+    const int me = r * wd + cw * kCclW;  // the word's first pixel
+    const bool has_l = cw > 0, has_r = cw + 1 < (int)nw;
+    const u64 lw = has_l ? b[i - 1] >> 63 : 0;  // the pixel left of the word
+    if (lw & m & 1) ccl_union(l, me, me - 1);
+    if (r == 0) continue;
+    const u64 u = b[i - nw];
+    const u64 ulw = has_l ? b[i - nw - 1] >> 63 : 0;
+    const u64 urw = has_r ? b[i - nw + 1] & 1 : 0;
+    if (r % kCclH == 0) {
+      u64 up, upl, upr;
+      ccl_rules(m, (m << 1) | lw, u, (u << 1) | ulw, (u >> 1) | (urw << 63), &up, &upl, &upr);
+      for (; up; up &= up - 1) {
+        const int c = me + __ffsll(up) - 1;
+        ccl_union(l, c, c - wd);
       }
+      for (; upl; upl &= upl - 1) {
+        const int c = me + __ffsll(upl) - 1;
+        ccl_union(l, c, c - wd - 1);
+      }
+      for (; upr; upr &= upr - 1) {
+        const int c = me + __ffsll(upr) - 1;
+        ccl_union(l, c, c - wd + 1);
+      }
+    } else {
+      if (m & 1 & ulw & ~u & ~lw) ccl_union(l, me, me - wd - 1);
+      if ((m >> 63) & urw & ~(u >> 63)) ccl_union(l, me + 63, me + 63 - wd + 1);
     }
   }
 }
 
-__global__ __launch_bounds__(kT) void k_ccl_compress(int* __restrict__ lab, size_t plane, const int* pred) {
-  if (pred_off(pred)) return;
+// labels for the caller: every set pixel's root without its mark, -1 for the others
+__global__ __launch_bounds__(kT) void k_ccl_flatten(int* __restrict__ lab, const u64* __restrict__ bits, int h, int wd) {
   const int s = blockIdx.y;
+  const size_t plane = (size_t)h * wd;
+  const int nw = ccl_words(wd);
   int* l = lab + (size_t)s * plane;
-  const size_t stride = (size_t)gridDim.x * kT;
-  size_t tail = 0;
-  if ((reinterpret_cast<uintptr_t>(l) & 15) == 0) {  // four labels per load; roots found per element
-    const int4* l4 = reinterpret_cast<const int4*>(l);
-    const size_t n4 = plane >> 2;
-    for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n4; i += stride) {
-      const int4 v = l4[i];
-      const int b = (int)(4 * i);
-      if (v.x >= 0) l[b] = ccl_find(l, b);
-      if (v.y >= 0) l[b + 1] = ccl_find(l, b + 1);
-      if (v.z >= 0) l[b + 2] = ccl_find(l, b + 2);
-      if (v.w >= 0) l[b + 3] = ccl_find(l, b + 3);
-    }
-    tail = 4 * n4;
+  for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < plane; i += (size_t)gridDim.x * kT) {
+    const int r = (int)(i / wd), c = (int)(i % wd);
+    const bool on = (bits[((size_t)s * h + r) * nw + (c >> 6)] >> (c & 63)) & 1;
+    l[i] = on ? ccl_find(l, (int)i) : -1;
   }
-  for (size_t i = tail + blockIdx.x * (size_t)kT + threadIdx.x; i < plane; i += stride)
-    if (l[i] >= 0) l[i] = ccl_find(l, (int)i);
 }
+
+// four plane elements, stored together where the rows' alignment allows
+template <class T>
+struct alignas(16) Quad {
+  T a[4];
+};
 
 // One step of the per-scale keep rule, coarsest scale first, in one pass over the pixels: applies
 // scale sa's marks (mask = pixel's object kept, extracted = mask * w) and marks the roots of scale
 // sm = sa - 1's objects that hold a seed pixel (value >= tol * max) inside sa's kept mask.  sa < 0:
-// mark only (the coarsest scale, which has no coarser mask); sm < 0: apply only.  A mark is the
-// scale's number plus one, in one of two flag planes by the scale's parity, so a launch reads the
-// marks of one plane while it writes the other's and no plane needs clearing between scales.
-template <class T>
-__global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, const int* __restrict__ lab, int sa, int sm,
-                                                  const T* __restrict__ smax, double tol, int neg_comp, size_t plane,
-                                                  uint8_t* __restrict__ keep2, size_t kstride,
+// mark only (the coarsest scale, which has no coarser mask); sm < 0: apply only.  A thread takes four
+// pixels of a row: their bits come from the scales' words, labels and values are read at set pixels
+// alone, and VEC (sides and buffers that keep quads aligned) writes the four extracted values and the
+// four mask bytes as one store each.  Roots are found by walking from the tile's root, so no pass
+// compresses the labels beforehand (162 us on seven 4096^2 planes).  Bound: the two outputs' stores.
+template <class T, bool VEC>
+__global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, int* __restrict__ lab,
+                                                  const u64* __restrict__ bits, int sa, int sm,
+                                                  const T* __restrict__ smax, double tol, int neg_comp, int h, int wd,
                                                   uint8_t* __restrict__ mask, T* __restrict__ extracted,
                                                   const int* pred) {
   if (pred_off(pred)) return;
   const double lim = sm >= 0 ? tol * (double)smax[sm] : 0.0;
-  const uint8_t* ka = keep2 + (size_t)(sa & 1) * kstride;
-  uint8_t* km = keep2 + (size_t)(sm & 1) * kstride;
-  for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < plane; i += (size_t)gridDim.x * kT) {
-    bool coarse_kept = true;
+  const int nw = ccl_words(wd);
+  const unsigned nq = (unsigned)(wd + 3) / 4;
+  const size_t plane = (size_t)h * wd;
+  const size_t oa = (size_t)(sa < 0 ? 0 : sa) * plane, om = (size_t)(sm < 0 ? 0 : sm) * plane;
+  const int* la = lab + oa;
+  int* lm = lab + om;
+  const unsigned total = (unsigned)h * nq;
+  for (unsigned i = blockIdx.x * kT + threadIdx.x; i < total; i += gridDim.x * kT) {
+    const int r = (int)(i / nq), c = 4 * (int)(i - (unsigned)r * nq);
+    const int px = r * wd + c;
+    const int word = r * nw + (c >> 6), shift = c & 63;
+    unsigned kept = 15u;
     if (sa >= 0) {
-      const size_t o = (size_t)sa * plane + i;
-      const int root = lab[o];
-      const bool k = root >= 0 && ka[root] == (uint8_t)(sa + 1);
-      mask[o] = k;
-      if (extracted) extracted[o] = k ? w[o] : (T)0;
-      coarse_kept = k;
+      const unsigned on = (unsigned)(bits[(size_t)sa * h * nw + word] >> shift) & 15u;
+      kept = 0;
+      Quad<T> e;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        e.a[k] = 0;
+        if ((on >> k) & 1) {
+          if (la[ccl_find(la, px + k)] < 0) {
+            kept |= 1u << k;
+            e.a[k] = w[oa + px + k];
+          }
+        }
+      }
+      uint8_t* mo = mask + oa + px;
+      T* eo = extracted ? extracted + oa + px : nullptr;
+      if constexpr (VEC) {
+        *reinterpret_cast<uint32_t*>(mo) =
+            (kept & 1u) | ((kept & 2u) << 7) | ((kept & 4u) << 14) | ((kept & 8u) << 21);
+        if (eo) *reinterpret_cast<Quad<T>*>(eo) = e;
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (c + k >= wd) break;
+          mo[k] = (kept >> k) & 1u;
+          if (eo) eo[k] = e.a[k];
+        }
+      }
     }
-    if (sm >= 0 && coarse_kept) {
-      const size_t o = (size_t)sm * plane + i;
-      const int root = lab[o];
-      if (root < 0) continue;
-      const T v = neg_comp ? (T)fabs(w[o]) : w[o];
-      if ((double)v >= lim) km[root] = (uint8_t)(sm + 1);
+    if (sm >= 0 && kept) {
+      const unsigned on = (unsigned)(bits[(size_t)sm * h * nw + word] >> shift) & kept;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (!((on >> k) & 1)) continue;
+        const T x = w[om + px + k];
+        const T v = neg_comp ? (T)fabs(x) : x;
+        if ((double)v >= lim) {
+          const int root = ccl_find(lm, px + k);
+          lm[root] = root | kMark;
+        }
+      }
     }
   }
-}
-
-__global__ void k_clear_u8(uint8_t* p, size_t n, const int* pred) {
-  if (pred_off(pred)) return;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0;
 }
 
 // raster-order label numbering: count roots per block, scan, write ranks
@@ -1032,24 +1127,19 @@ void max_final(const double* pmax, int nb, int S, double* out_max, const double*
   max_final_t(pmax, nb, S, out_max, energy, nsm, pred, st);
 }
 
-// workspace layout: [keep flags: two planes of bytes][maxima: 64 values][partial maxima: 16 x 2048
-// values][labels: S planes of int]; everything before the labels sits at fixed offsets (values sized
-// for double, so one layout serves both element types).
-static size_t keep_bytes(size_t plane) { return ((plane + 255) / 256) * 256; }
-static size_t ext_labels_offset(size_t plane) {
-  return 2 * keep_bytes(plane) + 64 * sizeof(double) + (size_t)kMaxPlanes * 2048 * sizeof(double);
+// workspace layout: [maxima: 64 values][tile maxima: S x tiles values][set-pixel words: S x h x words]
+// [labels: S planes of int], values sized for double so that one layout serves both element types.
+// Nothing in it has to be prepared: every part is written before it is read.
+static size_t ext_round(size_t bytes) { return ((bytes + 255) / 256) * 256; }
+static size_t ext_bits_offset(int S, int h, int wd) {
+  return ext_round((64 + (size_t)S * ccl_tiles(h, wd)) * sizeof(double));
+}
+static size_t ext_labels_offset(int S, int h, int wd) {
+  return ext_bits_offset(S, h, wd) + ext_round((size_t)S * h * ccl_words(wd) * sizeof(u64));
 }
 
 size_t extract_work_bytes(int S, int h, int w) {
-  const size_t plane = (size_t)h * w;
-  return ext_labels_offset(plane) + (size_t)S * plane * sizeof(int);
-}
-
-void extract_work_init(void* work, int, int h, int w, hipStream_t st) {
-  const size_t plane = (size_t)h * w;
-  hipLaunchKernelGGL(k_clear_u8, dim3(ew_grid(2 * plane)), dim3(kT), 0, st, (uint8_t*)work, 2 * keep_bytes(plane),
-                     (const int*)nullptr);
-  PMS_LAUNCH_CHECK();
+  return ext_labels_offset(S, h, w) + (size_t)S * h * w * sizeof(int);
 }
 
 template <class T>
@@ -1058,33 +1148,34 @@ static void source_extract_t(const T* w, int S, int h, int wd, double tol, int n
   PMS_REQUIRE((size_t)h * wd < (size_t)1 << 31, "plane too large for int labels");
   PMS_REQUIRE(S >= 1 && S <= kMaxPlanes, "source extraction handles 1..16 planes per call");
   const size_t plane = (size_t)h * wd;
-  uint8_t* keep = (uint8_t*)work;
-  const size_t kstride = keep_bytes(plane);
-  T* smax = (T*)((char*)work + 2 * kstride);
-  T* pmax = (T*)((char*)work + 2 * kstride + 64 * sizeof(double));
-  int* lab = (int*)((char*)work + ext_labels_offset(plane));
-  const int gx = threshold_grid(plane);
-  // keep flags start cleared whatever the workspace held before
-  hipLaunchKernelGGL(k_clear_u8, dim3(ew_grid(2 * plane)), dim3(kT), 0, st, keep, 2 * kstride, pred);
+  T* smax = (T*)work;
+  T* pmax = (T*)((char*)work + 64 * sizeof(double));
+  u64* bits = (u64*)((char*)work + ext_bits_offset(S, h, wd));
+  int* lab = (int*)((char*)work + ext_labels_offset(S, h, wd));
+  const int tiles = ccl_tiles(h, wd);
+  hipLaunchKernelGGL(k_ccl_tile<T>, dim3(tiles, S), dim3(kT), 0, st, w, lab, bits, h, wd, neg_comp, pmax, pred);
   PMS_LAUNCH_CHECK();
-  plane_max_t(w, S, plane, neg_comp, pmax, pred, st);
-  max_final_t(pmax, gx, S, smax, (const double*)nullptr, (double*)nullptr, pred, st);
-  const int gl = std::min(ew_grid(plane), 1024);
-  const int tiles = ceil_div(h, kCclTile) * ceil_div(wd, kCclTile);
-  hipLaunchKernelGGL(k_ccl_tile<T>, dim3(tiles, S), dim3(kT), 0, st, w, lab, h, wd, pred);
-  PMS_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_ccl_border, dim3(std::min(h, 4096), S), dim3(kT), 0, st, lab, h, wd, pred);
-  PMS_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_ccl_compress, dim3(gl, S), dim3(kT), 0, st, lab, plane, pred);
+  const int gb = std::min(ceil_div(h * ccl_words(wd), kT), 1024);
+  hipLaunchKernelGGL(k_ccl_border<T>, dim3(gb + 1, S), dim3(kT), 0, st, lab, (const u64*)bits, h, wd, (const T*)pmax,
+                     tiles, smax, pred);
   PMS_LAUNCH_CHECK();
   // keep rule from the coarsest scale down: mark S-1; apply s and mark s-1; ...; apply 0
+  const int gk = std::min(ceil_div(h * ceil_div(wd, 4), kT), 4096);
+  const bool vec = wd % 4 == 0 && aligned16(extracted) && (reinterpret_cast<uintptr_t>(mask) & 3) == 0;
   for (int sa = S; sa >= 0; --sa) {
-    hipLaunchKernelGGL(k_keep_step<T>, dim3(gl), dim3(kT), 0, st, w, (const int*)lab, sa < S ? sa : -1, sa - 1,
-                       (const T*)smax, tol, neg_comp, plane, keep, kstride, mask, extracted, pred);
+    if (vec)
+      hipLaunchKernelGGL((k_keep_step<T, true>), dim3(gk), dim3(kT), 0, st, w, lab, (const u64*)bits, sa < S ? sa : -1,
+                         sa - 1, (const T*)smax, tol, neg_comp, h, wd, mask, extracted, pred);
+    else
+      hipLaunchKernelGGL((k_keep_step<T, false>), dim3(gk), dim3(kT), 0, st, w, lab, (const u64*)bits,
+                         sa < S ? sa : -1, sa - 1, (const T*)smax, tol, neg_comp, h, wd, mask, extracted, pred);
     PMS_LAUNCH_CHECK();
   }
   if (labels_out) {
     // rank roots in raster order (scipy.ndimage.label numbering)
+    const int gl = std::min(ew_grid(plane), 1024);
+    hipLaunchKernelGGL(k_ccl_flatten, dim3(gl, S), dim3(kT), 0, st, lab, (const u64*)bits, h, wd);
+    PMS_LAUNCH_CHECK();
     const int chunk = 4096;
     const int nb = (int)((plane + chunk - 1) / chunk);
     uint32_t* counts = nullptr;
