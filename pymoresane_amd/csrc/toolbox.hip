@@ -496,21 +496,33 @@ __device__ __forceinline__ void ccl_rules(u64 m, u64 left, u64 u, u64 ul, u64 ur
   *upr = m & ~u & ur;
 }
 
+// this lane's bit of a mask that is the same in all lanes: the mask goes to the lanes' predicate as it is
+__device__ __forceinline__ bool lane_bit(u64 mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+__device__ __forceinline__ u64 first_lane(u64 v) {
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)(unsigned)v);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((int)(unsigned)(v >> 32));
+  return (u64)hi << 32 | lo;
+}
+
 // Two-level labelling, first level: one block labels a 64 x 32 tile in LDS (row runs linked to their
 // first pixel by bit arithmetic on the row's ballot, then union-find with LDS atomicMin links between
 // rows, so every tile component's root is its smallest raster index), and writes the rows' bit words
-// and, for set pixels, the tile roots as global raster indices; tiles without a set pixel end after
+// and, for set pixels, the tile roots as global raster indices; a tile without a set pixel ends after
 // the words.  The pass also takes the tile's maximum (of |w| with use_abs), so the planes are read
-// once: eight loads per thread are issued before the first is used.  Bound: reading the planes.  A
-// 32 x 32 tile that wrote a label (or -1) for every pixel took 297 us on seven 4096^2 planes, and the
-// separate maximum pass 111 us more.
-template <class T>
-__global__ __launch_bounds__(kT) void k_ccl_tile(const T* __restrict__ w, int* __restrict__ lab, u64* __restrict__ bits,
-                                                 int h, int wd, int use_abs, T* __restrict__ pmax, const int* pred) {
+// once.  Bound: instruction issue and reading the planes in sparse tiles, the chains of dependent LDS
+// reads in dense ones; a row is one wave's ballot, so the rows' words and union rules are scalar arithmetic; a
+// wave unions its rows from the top down, which links each run straight to its component's root.
+// NT threads (128 or 512) share a tile: four rows a wave end a tile soonest, sixteen spend the fewest
+// instructions per pixel (source_extract_t chooses).  Seven 4096^2 planes take 144 / 161 / 241 us with
+// 128 / 256 / 512 threads, five 500^2 planes 21.9 / 15.7 / 12.2 us.
+template <class T, int NT>
+__global__ __launch_bounds__(NT) void k_ccl_tile(const T* __restrict__ w, int* __restrict__ lab,
+                                                    u64* __restrict__ bits, int h, int wd, int use_abs,
+                                                    T* __restrict__ pmax, const int* pred) {
   if (pred_off(pred)) return;
-  constexpr int TW = kCclW, TH = kCclH, PER = TH / (kT / 64);
+  constexpr int TW = kCclW, TH = kCclH, PER = TH / (NT / 64);
   __shared__ int L[TH * TW];
-  __shared__ u64 rows[TH];
+  __shared__ u64 last_rows[NT / 64];  // each wave's last row
   const int s = blockIdx.y;
   const int nw = ccl_words(wd);
   const int cw = blockIdx.x % nw;
@@ -518,56 +530,60 @@ __global__ __launch_bounds__(kT) void k_ccl_tile(const T* __restrict__ w, int* _
   const size_t plane = (size_t)h * wd;
   const T* x = w + (size_t)s * plane;
   int* l = lab + (size_t)s * plane;
-  const int lane = threadIdx.x & 63, row0 = (threadIdx.x >> 6) * PER;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row0 = wave * PER;
   const int col = c0 + lane;
   const bool col_ok = col < wd;
   T v[PER];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int r = r0 + row0 + i;
-    v[i] = x[(size_t)min(r, h - 1) * wd + (col_ok ? col : wd - 1)];
-  }
+  for (int i = 0; i < PER; ++i)  // a lane or row outside the plane repeats a pixel of the tile
+    v[i] = (x + (size_t)min(r0 + row0 + i, h - 1) * wd)[col_ok ? col : wd - 1];
   T m = -INFINITY;
+  u64 word[PER];
   u64 any = 0;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int r = r0 + row0 + i;
     const T a = use_abs ? (T)fabs(v[i]) : v[i];
-    m = a > m ? a : m;  // a dead lane repeats a pixel of the tile
-    const u64 word = __ballot(col_ok && r < h && v[i] != (T)0);
-    any |= word;
-    if (lane == 0) {
-      rows[row0 + i] = word;
-      if (r < h) bits[((size_t)s * h + r) * nw + cw] = word;
-    }
-    if ((word >> lane) & 1) {
-      const u64 gaps = ~word & (((u64)1 << lane) - 1);
-      L[(row0 + i) * TW + lane] = (row0 + i) * TW + (gaps ? 64 - __clzll(gaps) : 0);
+    m = a > m ? a : m;
+    word[i] = r < h ? __ballot(col_ok && v[i] != (T)0) : 0;
+    any |= word[i];
+    if (word[i] != 0) {
+      const u64 gaps = ~word[i] & (((u64)1 << lane) - 1);
+      if (lane_bit(word[i])) L[(row0 + i) * TW + lane] = (row0 + i) * TW + (gaps ? 64 - __clzll(gaps) : 0);
     }
   }
+  // lane i stores row i's word
+  u64 mine = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) mine = lane == i ? word[i] : mine;
+  if (lane < PER && r0 + row0 + lane < h) bits[((size_t)s * h + r0 + row0 + lane) * nw + cw] = mine;
+  if (lane == PER - 1) last_rows[wave] = mine;
   m = block_max_t<T>(m);
   if (threadIdx.x == 0) pmax[(size_t)s * gridDim.x + blockIdx.x] = m;
   if (!__syncthreads_or(any != 0)) return;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int tr = row0 + i;
-    const u64 word = rows[tr];
-    if (tr == 0 || !((word >> lane) & 1)) continue;
-    const u64 u = rows[tr - 1];
+    if (word[i] == 0) continue;
+    u64 u;
+    if (i > 0)
+      u = word[i > 0 ? i - 1 : 0];
+    else
+      u = wave > 0 ? first_lane(last_rows[wave > 0 ? wave - 1 : 0]) : 0;
     u64 up, upl, upr;
-    ccl_rules(word, word << 1, u, u << 1, u >> 1, &up, &upl, &upr);
-    const int me = tr * TW + lane;
-    if ((up >> lane) & 1) lds_union(L, me, me - TW);
-    if ((upl >> lane) & 1) lds_union(L, me, me - TW - 1);
-    if ((upr >> lane) & 1) lds_union(L, me, me - TW + 1);
+    ccl_rules(word[i], word[i] << 1, u, u << 1, u >> 1, &up, &upl, &upr);
+    const int me = (row0 + i) * TW + lane;
+    if (up && lane_bit(up)) lds_union(L, me, me - TW);
+    if (upl && lane_bit(upl)) lds_union(L, me, me - TW - 1);
+    if (upr && lane_bit(upr)) lds_union(L, me, me - TW + 1);
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int tr = row0 + i;
-    if (!((rows[tr] >> lane) & 1)) continue;
-    const int root = lds_find(L, tr * TW + lane);
-    l[(size_t)(r0 + tr) * wd + col] = (r0 + root / TW) * wd + c0 + root % TW;
+    if (word[i] == 0 || !lane_bit(word[i])) continue;
+    const int root = lds_find(L, (row0 + i) * TW + lane);
+    (l + (size_t)(r0 + row0 + i) * wd)[col] = (r0 + root / TW) * wd + c0 + root % TW;
   }
 }
 
@@ -605,12 +621,12 @@ __global__ __launch_bounds__(kT) void k_ccl_border(int* __restrict__ lab, const 
     const int me = r * wd + cw * kCclW;  // the word's first pixel
     const bool has_l = cw > 0, has_r = cw + 1 < (int)nw;
     const u64 lw = has_l ? b[i - 1] >> 63 : 0;  // the pixel left of the word
-    if (lw & m & 1) ccl_union(l, me, me - 1);
-    if (r == 0) continue;
-    const u64 u = b[i - nw];
-    const u64 ulw = has_l ? b[i - nw - 1] >> 63 : 0;
-    const u64 urw = has_r ? b[i - nw + 1] & 1 : 0;
-    if (r % kCclH == 0) {
+    const u64 u = r > 0 ? b[i - nw] : 0;
+    const u64 ulw = r > 0 && has_l ? b[i - nw - 1] >> 63 : 0;
+    const u64 urw = r > 0 && has_r ? b[i - nw + 1] & 1 : 0;
+    const bool top = r % kCclH == 0;
+    if ((lw & m & 1) && (top || !(u & ulw & 1))) ccl_union(l, me, me - 1);
+    if (top) {
       u64 up, upl, upr;
       ccl_rules(m, (m << 1) | lw, u, (u << 1) | ulw, (u >> 1) | (urw << 63), &up, &upl, &upr);
       for (; up; up &= up - 1) {
@@ -651,50 +667,84 @@ struct alignas(16) Quad {
   T a[4];
 };
 
+// Roots of the set ones (bits `on`) of four pixels from px on, walked side by side so that a step costs
+// one memory latency for all of them; returns which of the roots carry the keep mark.
+__device__ __forceinline__ unsigned ccl_find4(const int* lab, int px, unsigned on, int (&root)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) root[k] = (on >> k) & 1 ? lab[px + k] & ~kMark : 0;
+  unsigned marked = 0, more = on;
+  while (more) {
+    int p[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) p[k] = (more >> k) & 1 ? lab[root[k]] : 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (!((more >> k) & 1)) continue;
+      if ((p[k] & ~kMark) == root[k]) {
+        more &= ~(1u << k);
+        marked |= p[k] < 0 ? 1u << k : 0u;
+      }
+      root[k] = p[k] & ~kMark;
+    }
+  }
+  return marked;
+}
+
 // One step of the per-scale keep rule, coarsest scale first, in one pass over the pixels: applies
 // scale sa's marks (mask = pixel's object kept, extracted = mask * w) and marks the roots of scale
 // sm = sa - 1's objects that hold a seed pixel (value >= tol * max) inside sa's kept mask.  sa < 0:
-// mark only (the coarsest scale, which has no coarser mask); sm < 0: apply only.  A thread takes four
-// pixels of a row: their bits come from the scales' words, labels and values are read at set pixels
+// mark only (the coarsest scale, which has no coarser mask); sm < 0: apply only.  A thread takes U times four
+// pixels of a row: their bits come from the scales' words, requested for all of them first, labels
+// and values are read at set pixels
 // alone, and VEC (sides and buffers that keep quads aligned) writes the four extracted values and the
 // four mask bytes as one store each.  Roots are found by walking from the tile's root, so no pass
-// compresses the labels beforehand (162 us on seven 4096^2 planes).  Bound: the two outputs' stores.
-template <class T, bool VEC>
+// compresses the labels beforehand (162 us on seven 4096^2 planes).  Bound: the two outputs' stores:
+// 31 us a scale at 4096^2 (64 us on label planes with separate flags; 33 us with one quad a thread).
+template <class T, bool VEC, int U>
 __global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, int* __restrict__ lab,
                                                   const u64* __restrict__ bits, int sa, int sm,
                                                   const T* __restrict__ smax, double tol, int neg_comp, int h, int wd,
                                                   uint8_t* __restrict__ mask, T* __restrict__ extracted,
                                                   const int* pred) {
   if (pred_off(pred)) return;
-  const double lim = sm >= 0 ? tol * (double)smax[sm] : 0.0;
   const int nw = ccl_words(wd);
   const unsigned nq = (unsigned)(wd + 3) / 4;
   const size_t plane = (size_t)h * wd;
   const size_t oa = (size_t)(sa < 0 ? 0 : sa) * plane, om = (size_t)(sm < 0 ? 0 : sm) * plane;
   const int* la = lab + oa;
   int* lm = lab + om;
+  const u64* ba = bits + (size_t)(sa < 0 ? 0 : sa) * h * nw;
+  const u64* bm = bits + (size_t)(sm < 0 ? 0 : sm) * h * nw;
   const unsigned total = (unsigned)h * nq;
-  for (unsigned i = blockIdx.x * kT + threadIdx.x; i < total; i += gridDim.x * kT) {
-    const int r = (int)(i / nq), c = 4 * (int)(i - (unsigned)r * nq);
-    const int px = r * wd + c;
-    const int word = r * nw + (c >> 6), shift = c & 63;
+  const unsigned i0 = blockIdx.x * (unsigned)(kT * U) + threadIdx.x;
+  int px[U], c[U];
+  unsigned on_a[U], on_m[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const unsigned i = min(i0 + u * kT, total - 1);
+    const int r = (int)(i / nq);
+    c[u] = 4 * (int)(i - (unsigned)r * nq);
+    px[u] = r * wd + c[u];
+    const int word = r * nw + (c[u] >> 6), shift = c[u] & 63;
+    on_a[u] = (unsigned)(ba[word] >> shift) & 15u;
+    on_m[u] = (unsigned)(bm[word] >> shift) & 15u;
+  }
+  const double lim = sm >= 0 ? tol * (double)smax[sm] : 0.0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (i0 + u * kT >= total) return;
     unsigned kept = 15u;
+    int root[4];
     if (sa >= 0) {
-      const unsigned on = (unsigned)(bits[(size_t)sa * h * nw + word] >> shift) & 15u;
-      kept = 0;
+      const unsigned on = on_a[u];
       Quad<T> e;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        e.a[k] = 0;
-        if ((on >> k) & 1) {
-          if (la[ccl_find(la, px + k)] < 0) {
-            kept |= 1u << k;
-            e.a[k] = w[oa + px + k];
-          }
-        }
-      }
-      uint8_t* mo = mask + oa + px;
-      T* eo = extracted ? extracted + oa + px : nullptr;
+      for (int k = 0; k < 4; ++k) e.a[k] = (on >> k) & 1 ? w[oa + px[u] + k] : (T)0;
+      kept = on ? ccl_find4(la, px[u], on, root) : 0u;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) e.a[k] = (kept >> k) & 1 ? e.a[k] : (T)0;
+      uint8_t* mo = mask + oa + px[u];
+      T* eo = extracted ? extracted + oa + px[u] : nullptr;
       if constexpr (VEC) {
         *reinterpret_cast<uint32_t*>(mo) =
             (kept & 1u) | ((kept & 2u) << 7) | ((kept & 4u) << 14) | ((kept & 8u) << 21);
@@ -702,25 +752,28 @@ __global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, int* 
       } else {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          if (c + k >= wd) break;
+          if (c[u] + k >= wd) break;
           mo[k] = (kept >> k) & 1u;
           if (eo) eo[k] = e.a[k];
         }
       }
     }
-    if (sm >= 0 && kept) {
-      const unsigned on = (unsigned)(bits[(size_t)sm * h * nw + word] >> shift) & kept;
+    if (sm < 0) continue;
+    unsigned seeds = on_m[u] & kept;
+    if (!seeds) continue;
+    T x[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (!((on >> k) & 1)) continue;
-        const T x = w[om + px + k];
-        const T v = neg_comp ? (T)fabs(x) : x;
-        if ((double)v >= lim) {
-          const int root = ccl_find(lm, px + k);
-          lm[root] = root | kMark;
-        }
-      }
+    for (int k = 0; k < 4; ++k) x[k] = (seeds >> k) & 1 ? w[om + px[u] + k] : (T)0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const T v = neg_comp ? (T)fabs(x[k]) : x[k];
+      if (!((double)v >= lim)) seeds &= ~(1u << k);
     }
+    if (!seeds) continue;
+    (void)ccl_find4(lm, px[u], seeds, root);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if ((seeds >> k) & 1) lm[root[k]] = root[k] | kMark;
   }
 }
 
@@ -1153,22 +1206,31 @@ static void source_extract_t(const T* w, int S, int h, int wd, double tol, int n
   u64* bits = (u64*)((char*)work + ext_bits_offset(S, h, wd));
   int* lab = (int*)((char*)work + ext_labels_offset(S, h, wd));
   const int tiles = ccl_tiles(h, wd);
-  hipLaunchKernelGGL(k_ccl_tile<T>, dim3(tiles, S), dim3(kT), 0, st, w, lab, bits, h, wd, neg_comp, pmax, pred);
+  // While every tile's block is resident at once (1024 blocks of 512 threads), the time is that of one
+  // tile; beyond, it is the instructions of all.
+  if ((size_t)tiles * S <= 1024)
+    hipLaunchKernelGGL((k_ccl_tile<T, 512>), dim3(tiles, S), dim3(512), 0, st, w, lab, bits, h, wd, neg_comp, pmax,
+                       pred);
+  else
+    hipLaunchKernelGGL((k_ccl_tile<T, 128>), dim3(tiles, S), dim3(128), 0, st, w, lab, bits, h, wd, neg_comp, pmax,
+                       pred);
   PMS_LAUNCH_CHECK();
   const int gb = std::min(ceil_div(h * ccl_words(wd), kT), 1024);
   hipLaunchKernelGGL(k_ccl_border<T>, dim3(gb + 1, S), dim3(kT), 0, st, lab, (const u64*)bits, h, wd, (const T*)pmax,
                      tiles, smax, pred);
   PMS_LAUNCH_CHECK();
   // keep rule from the coarsest scale down: mark S-1; apply s and mark s-1; ...; apply 0
-  const int gk = std::min(ceil_div(h * ceil_div(wd, 4), kT), 4096);
   const bool vec = wd % 4 == 0 && aligned16(extracted) && (reinterpret_cast<uintptr_t>(mask) & 3) == 0;
+  const unsigned quads = (unsigned)h * (unsigned)ceil_div(wd, 4);
+  // four quads a thread once that still leaves eight blocks per CU (from about 2900^2 pixels on); below, a thread's chain
+  // of dependent reads sets the time and more threads hide it
+  const bool four = quads >= 4u * kT * 2048;
+  const unsigned per = kT * (four ? 4 : 1);
+  auto keep = vec ? (four ? k_keep_step<T, true, 4> : k_keep_step<T, true, 1>)
+                  : (four ? k_keep_step<T, false, 4> : k_keep_step<T, false, 1>);
   for (int sa = S; sa >= 0; --sa) {
-    if (vec)
-      hipLaunchKernelGGL((k_keep_step<T, true>), dim3(gk), dim3(kT), 0, st, w, lab, (const u64*)bits, sa < S ? sa : -1,
-                         sa - 1, (const T*)smax, tol, neg_comp, h, wd, mask, extracted, pred);
-    else
-      hipLaunchKernelGGL((k_keep_step<T, false>), dim3(gk), dim3(kT), 0, st, w, lab, (const u64*)bits,
-                         sa < S ? sa : -1, sa - 1, (const T*)smax, tol, neg_comp, h, wd, mask, extracted, pred);
+    hipLaunchKernelGGL(keep, dim3((quads + per - 1) / per), dim3(kT), 0, st, w, lab, (const u64*)bits,
+                       sa < S ? sa : -1, sa - 1, (const T*)smax, tol, neg_comp, h, wd, mask, extracted, pred);
     PMS_LAUNCH_CHECK();
   }
   if (labels_out) {
