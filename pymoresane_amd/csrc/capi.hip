@@ -287,9 +287,7 @@ int pms_fft_convolve(const float* in, int n, int p, const void* spectrum, float*
 // ------------------------------------------------------------------- threshold
 size_t pms_threshold_work_bytes(int n_planes, int h, int w) {
   if (n_planes <= 0 || h <= 0 || w <= 0) return 0;
-  (void)h;
-  (void)w;
-  return ((mad_work_bytes(n_planes) + 255) / 256) * 256 + (size_t)n_planes * 256 * sizeof(float);
+  return std::max(mad_work_bytes(n_planes, (size_t)h * w, sizeof(float)), (size_t)n_planes * 256 * sizeof(float));
 }
 
 int pms_estimate_threshold(const float* planes, int n_planes, int h, int w, int edge_excl, int int_excl,
@@ -298,7 +296,6 @@ int pms_estimate_threshold(const float* planes, int n_planes, int h, int w, int 
     PMS_REQUIRE(planes && thresholds_out && work, "NULL buffer");
     PMS_REQUIRE(n_planes >= 1 && h >= 1 && w >= 1, "bad plane stack shape");
     NoiseMask nm = noise_mask(h, w, edge_excl, int_excl);
-    mad_work_init(work, n_planes, S(stream));
     mad_thresholds(planes, n_planes, h, w, nm, thresholds_out, work, nullptr, S(stream));
   });
 }
@@ -315,11 +312,7 @@ int pms_estimate_threshold_noalloc(const float* planes, int n_planes, int h, int
     NoiseMask nm = noise_mask(h, w, edge_excl, int_excl);
     PMS_REQUIRE(nm.count < (1L << 32), "pms_estimate_threshold_noalloc: more than 2^32 - 1 pixels per plane");
     void* work = noalloc_mad_scratch();
-    PMS_REQUIRE(mad_work_bytes(n_planes) <= noalloc_mad_bytes(), "median workspace larger than the device array");
-    // the array keeps the previous call's contents: clear the histograms (the select state is
-    // rewritten by the first kernel of every call)
-    mad_work_init(work, n_planes, S(stream));
-    mad_thresholds(planes, n_planes, h, w, nm, thresholds_out, work, nullptr, S(stream));
+    mad_thresholds_noalloc(planes, n_planes, h, w, nm, thresholds_out, work, nullptr, S(stream));
   });
 }
 
@@ -327,8 +320,7 @@ int pms_apply_threshold(const float* planes, int n_planes, int h, int w, const d
                         double sigma_level, float* out, void* work, void* stream) {
   return guarded([&] {
     PMS_REQUIRE(planes && thresholds && out && work, "NULL buffer");
-    float* pmax = (float*)((char*)work + ((mad_work_bytes(n_planes) + 255) / 256) * 256);
-    apply_threshold(planes, out, n_planes, h, w, thresholds, sigma_level, nullptr, pmax, nullptr, S(stream));
+    apply_threshold(planes, out, n_planes, h, w, thresholds, sigma_level, nullptr, (float*)work, nullptr, S(stream));
   });
 }
 

@@ -67,7 +67,7 @@ Geometry make_geometry(int n, int psf_n, const MoresaneParams& prm, int scale_co
 
 // byte sizes of the per-job device buffers
 struct JobSizes {
-  size_t s2, S_s2, mask, iuwt, N2, spec_sub, spec_full, fft, psf, ext, partial, pmax;
+  size_t s2, S_s2, mask, iuwt, N2, spec_sub, spec_full, fft, psf, ext, mad, partial, pmax;
   bool f64;
 };
 

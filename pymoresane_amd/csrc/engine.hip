@@ -531,6 +531,7 @@ static JobSizes job_sizes(const Geometry& g, int S) {
           2 * e;
   z.psf = (size_t)g.psf_n * g.psf_n * e;
   z.ext = extract_work_bytes(S, g.sub, g.sub);
+  z.mad = mad_work_bytes(S, s2, e);
   const long dec_partials = g.f64 ? iuwt_decompose_partials_f64(g.sub, g.sub, S, 0)
                                   : iuwt_decompose_partials(g.sub, g.sub, S, 0);
   z.partial = (size_t)std::max<long>({dec_partials, (long)reduce_grid(N2) * 2, (long)reduce_grid(s2) * S, 4096L}) *
@@ -542,7 +543,7 @@ static JobSizes job_sizes(const Geometry& g, int S) {
 static bool fits(const JobSizes& need, const JobSizes& have) {
   return need.f64 == have.f64 && need.s2 <= have.s2 && need.S_s2 <= have.S_s2 && need.mask <= have.mask &&
          need.iuwt <= have.iuwt && need.N2 <= have.N2 && need.spec_sub <= have.spec_sub &&
-         need.spec_full <= have.spec_full && need.fft <= have.fft && need.psf <= have.psf && need.ext <= have.ext &&
+         need.spec_full <= have.spec_full && need.fft <= have.fft && need.psf <= have.psf && need.ext <= have.ext && need.mad <= have.mad &&
          need.partial <= have.partial && need.pmax <= have.pmax;
 }
 
@@ -559,6 +560,7 @@ static JobSizes max_sizes(const JobSizes& a, const JobSizes& b) {
   z.fft = std::max(a.fft, b.fft);
   z.psf = std::max(a.psf, b.psf);
   z.ext = std::max(a.ext, b.ext);
+  z.mad = std::max(a.mad, b.mad);
   z.partial = std::max(a.partial, b.partial);
   z.pmax = std::max(a.pmax, b.pmax);
   return z;
@@ -567,7 +569,7 @@ static JobSizes max_sizes(const JobSizes& a, const JobSizes& b) {
 size_t job_footprint_bytes(const Geometry& g) {
   const JobSizes z = job_sizes(g, std::max(g.S, (int)std::log2((double)g.n) - 1));
   const size_t by_scale = z.N2;  // moresane_by_scale's private dirty copy
-  return z.s2 * 10 + z.S_s2 * 4 + z.mask + z.iuwt + z.N2 * 3 + z.spec_sub + z.spec_full + z.fft + z.psf + z.ext +
+  return z.s2 * 10 + z.S_s2 * 4 + z.mask + z.iuwt + z.N2 * 3 + z.spec_sub + z.spec_full + z.fft + z.psf + z.ext + z.mad +
          z.partial + z.pmax + by_scale + 64 * 8 + 64 * 4 + 12 * 256;
 }
 
@@ -639,8 +641,7 @@ bool Job::ensure(const Geometry& g, hipStream_t st) {
   else
     carve(f, z, arena_);
   M = (uint8_t*)arena_.alloc(z.mask);
-  mad_work = arena_.alloc(mad_work_bytes(16));
-  mad_work_init(mad_work, 16, st);
+  mad_work = arena_.alloc(z.mad);
   ext_work = arena_.alloc(z.ext);
   partial = (double*)arena_.alloc(z.partial);
   have_ = true;

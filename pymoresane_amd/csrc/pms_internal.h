@@ -272,15 +272,17 @@ struct NoiseMask {
   long count;
 };
 NoiseMask noise_mask(int h, int w, int edge_excl, int int_excl);
-size_t mad_work_bytes(int S);
+size_t mad_work_bytes(int S, size_t plane, size_t real_bytes);  // for S planes of `plane` elements
 // the allocation-free median workspace of the current device (looked up once per device) and its size
 void* noalloc_mad_scratch();
 size_t noalloc_mad_bytes();
-void mad_work_init(void* work, int S, hipStream_t st);  // once per workspace (histograms start at 0)
 void mad_thresholds(const float* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
                     const int* pred, hipStream_t st);
 void mad_thresholds(const double* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
                     const int* pred, hipStream_t st);
+// the same medians from a workspace of noalloc_mad_bytes(), which a call reads a plane several times for
+void mad_thresholds_noalloc(const float* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
+                            const int* pred, hipStream_t st);
 // out = in where |in| > sigma*thr[s] else 0, zeroing a per-scale border (border may be null);
 // pmax receives threshold_grid(plane) partial maxima per plane.
 void apply_threshold(const float* in, float* out, int S, int h, int w, const double* thr, double sigma,

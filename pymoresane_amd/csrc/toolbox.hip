@@ -343,6 +343,619 @@ __global__ void k_mad_finish(const SelStateT<typename MadKey<T>::K>* st, int S, 
   thr[s] = med / 0.6745;
 }
 
+// four plane elements, read or stored together where the alignment allows
+template <class T>
+struct alignas(16) Quad {
+  T a[4];
+};
+
+// ---- median in one reading of the planes -------------------------------------------------------
+// The radix select above reads a plane once per digit.  With a workspace for it, a plane is read once:
+//   * planes of at most 32768 noise pixels are selected by one block with the keys in registers;
+//   * larger ones are sampled (k_mad_pivot: one block a plane, a radix select on the sample) for a range of
+//     keys [lo, lo + range] around the median.  The sample is groups of four neighbours; were the four
+//     always alike, the range would still reach four standard deviations of the median's rank to
+//     either side.  One pass over the plane (k_mad_scan) counts the keys below the range, counts those in
+//     it in 64 bins and sets them aside (6 to 9% of the plane), and one block a plane (k_mad_pick) takes the
+//     bin of the median's rank and selects in it (from a list of that bin, k_mad_collect, on large planes).
+// Nothing is estimated in the result: when the range misses the median's rank or more keys fall in it
+// than there is room for, k_mad_pick selects from the plane itself.  The result is the same key, and
+// for even counts the same pair of keys, as the radix select's.
+constexpr int kMT = 1024;            // threads of the one-block kernels
+constexpr int kMadOne = 32 * kMT;    // noise pixels that one block holds in registers
+constexpr int kMadBins = 64;         // bins of the range
+
+template <class K>
+struct alignas(16) MadRange {
+  K lo, range;      // keys lo .. lo + range (inclusive)
+  K least2;         // k_mad_collect: least key of the successor's bin
+  uint32_t shift;   // bin = (key - lo) >> shift, below kMadBins
+  uint32_t below;   // keys below lo
+  uint32_t n;       // keys of the range set aside (counted beyond the room for them)
+  uint32_t listed;  // k_mad_collect: keys of the median's bin (counted beyond the room for them)
+};
+constexpr size_t kRangeBytes = 64;
+static_assert(sizeof(MadRange<uint32_t>) <= kRangeBytes && sizeof(MadRange<unsigned long long>) <= kRangeBytes,
+              "median range exceeds its slot");
+
+// keys set aside per plane at most (a multiple of 16: each plane's buffer starts 64-byte aligned)
+__host__ __device__ __forceinline__ size_t mad_room(size_t plane) { return (plane / 8 / 16 + 64) * 16; }
+// keys of the median's bin listed per plane at most
+__host__ __device__ __forceinline__ size_t mad_list_room(size_t plane) { return plane / 128 + 4096; }
+
+template <class K>
+__device__ __forceinline__ int bit_length(K v) {
+  if constexpr (sizeof(K) == 8)
+    return v ? 64 - __clzll((long long)v) : 0;
+  else
+    return v ? 32 - __clz((int)v) : 0;
+}
+
+// Where a block finds ranks in the 2048 counts of h (LDS): the bin, the counts before it and its own.
+// All threads of a kMT block call it; the result is the same in all of them.  A rank beyond the total
+// gives the last bin.
+struct BinHit {
+  int bin;
+  uint32_t before, count;
+};
+struct BinScratch {
+  uint32_t part[kMT / 64];
+  BinHit hit[2];
+};
+__device__ __forceinline__ void find_bins(const uint32_t* h, uint32_t r0, uint32_t r1, BinScratch& sc, BinHit* a,
+                                          BinHit* b) {
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const uint32_t c0 = h[2 * t], c1 = h[2 * t + 1], local = c0 + c1;
+  uint32_t inc = local;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t v = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += v;
+  }
+  __syncthreads();  // the scratch of an earlier call has been read
+  if (lane == 63) sc.part[wid] = inc;
+  __syncthreads();
+  uint32_t before = lane < wid ? sc.part[lane & (kMT / 64 - 1)] : 0;  // lanes 0 .. 15 hold the waves before
+#pragma unroll
+  for (int o = kMT / 128; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+  inc += (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
+  const uint32_t exc = inc - local;
+  auto put = [&](uint32_t r, BinHit* to) {
+    if ((r >= exc && r < inc) || (t == kMT - 1 && r >= inc)) {
+      const bool second = r >= exc + c0;
+      *to = BinHit{2 * t + (second ? 1 : 0), second ? exc + c0 : exc, second ? c1 : c0};
+    }
+  };
+  put(r0, &sc.hit[0]);
+  put(r1, &sc.hit[1]);
+  __syncthreads();
+  *a = sc.hit[0];
+  *b = sc.hit[1];
+}
+__device__ __forceinline__ BinHit find_bin(const uint32_t* h, uint32_t r, BinScratch& sc) {
+  BinHit a, b;
+  find_bins(h, r, r, sc, &a, &b);
+  return a;
+}
+
+__device__ __forceinline__ void clear_bins(uint32_t* h) {
+  h[threadIdx.x] = 0;
+  h[threadIdx.x + kMT] = 0;
+}
+
+// minimum over a kMT block, the same in all threads
+template <class K>
+__device__ __forceinline__ K block_min_key(K v, K* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const K u = __shfl_xor(v, o, 64);
+    v = u < v ? u : v;
+  }
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  for (int k = 0; k < kMT / 64; ++k) v = red[k] < v ? red[k] : v;
+  return v;
+}
+
+template <class T>
+__device__ __forceinline__ double mad_of(typename MadKey<T>::K lo, typename MadKey<T>::K hi, bool even) {
+  const double a = (double)MadKey<T>::val(lo);
+  return (even ? (a + (double)MadKey<T>::val(hi)) * 0.5 : a) / 0.6745;
+}
+
+// The key of noise pixel j of a plane in the order of the included rectangle's rows (the whole plane
+// without a mask); false for a pixel of the excluded rectangle.
+template <class T, bool MASKED>
+__device__ __forceinline__ bool noise_key(const T* x, int w, Rect inc, Rect exc, uint32_t j,
+                                          typename MadKey<T>::K* key) {
+  if constexpr (!MASKED) {
+    *key = MadKey<T>::key(x[j]);
+    return true;
+  } else {
+    const uint32_t wr = (uint32_t)(inc.c1 - inc.c0);
+    const uint32_t q = j / wr;
+    const int r = inc.r0 + (int)q, c = inc.c0 + (int)(j - q * wr);
+    *key = MadKey<T>::key(x[(size_t)r * w + c]);
+    return !(r >= exc.r0 && r < exc.r1 && c >= exc.c0 && c < exc.c1);
+  }
+}
+
+// Every noise pixel's key of a plane, dealt over `nthr` threads, to f(key).
+template <class T, bool MASKED, class F>
+__device__ __forceinline__ void each_noise_key(const T* x, size_t plane, int w, Rect inc, Rect exc, size_t thr,
+                                               size_t nthr, F f) {
+  if constexpr (!MASKED) {
+    constexpr int V = 16 / sizeof(T);
+    struct alignas(16) Vec {
+      T a[V];
+    };
+    size_t done = 0;
+    if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+      const Vec* xv = reinterpret_cast<const Vec*>(x);
+      const size_t nv = plane / V;
+      size_t i = thr;
+      for (; i + 3 * nthr < nv; i += 4 * nthr) {  // four loads in flight
+        const Vec a = xv[i], b = xv[i + nthr], c = xv[i + 2 * nthr], d = xv[i + 3 * nthr];
+#pragma unroll
+        for (int k = 0; k < V; ++k) f(MadKey<T>::key(a.a[k]));
+#pragma unroll
+        for (int k = 0; k < V; ++k) f(MadKey<T>::key(b.a[k]));
+#pragma unroll
+        for (int k = 0; k < V; ++k) f(MadKey<T>::key(c.a[k]));
+#pragma unroll
+        for (int k = 0; k < V; ++k) f(MadKey<T>::key(d.a[k]));
+      }
+      for (; i < nv; i += nthr) {
+        const Vec a = xv[i];
+#pragma unroll
+        for (int k = 0; k < V; ++k) f(MadKey<T>::key(a.a[k]));
+      }
+      done = nv * V;
+    }
+    for (size_t i = done + thr; i < plane; i += nthr) f(MadKey<T>::key(x[i]));
+  } else {
+    // 64 threads a row: no division per pixel
+    const int lane = (int)(thr & 63);
+    for (size_t r = inc.r0 + (thr >> 6); r < (size_t)inc.r1; r += nthr >> 6) {
+      const T* row = x + r * w;
+      const bool cut = (int)r >= exc.r0 && (int)r < exc.r1;
+      for (int c = inc.c0 + lane; c < inc.c1; c += 64) {
+        if (cut && c >= exc.c0 && c < exc.c1) continue;
+        f(MadKey<T>::key(row[c]));
+      }
+    }
+  }
+}
+
+// Whole planes of at most kMadOne noise pixels (area: pixels of the included rectangle): a radix select
+// in LDS over keys held in registers, 11 bits a digit; then the successor of an even count.
+template <class T, bool MASKED, int PT>
+__global__ __launch_bounds__(kMT) void k_mad_one(const T* __restrict__ planes, size_t plane, int w, Rect inc, Rect exc,
+                                                 uint32_t area, uint32_t count, double* __restrict__ thr,
+                                                 const int* pred) {
+  using K = typename MadKey<T>::K;
+  if (pred_off(pred)) return;
+  __shared__ uint32_t h[kBins];
+  __shared__ BinScratch scratch;
+  __shared__ K red[kMT / 64];
+  const T* x = planes + (size_t)blockIdx.x * plane;
+  K key[PT];
+  uint32_t have = 0;
+#pragma unroll
+  for (int i = 0; i < PT; ++i) {
+    const uint32_t j = threadIdx.x + i * kMT;
+    const bool in = noise_key<T, MASKED>(x, w, inc, exc, min(j, area - 1), &key[i]);
+    if (in && j < area) have |= 1u << i;
+  }
+  uint32_t rank = (count - 1) / 2;  // of the low median among the keys that share the digits found so far
+  K v = 0;
+  int top = 8 * (int)sizeof(K) - 1;  // the sign bit is clear
+  uint32_t equal = count;
+  while (top > 0) {
+    const int nd = min(11, top), shift = top - nd;
+    clear_bins(h);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+      if ((have >> i) & 1 && (key[i] >> top) == (v >> top))
+        atomicAdd(&h[(uint32_t)(key[i] >> shift) & ((1u << nd) - 1)], 1u);
+    __syncthreads();
+    const BinHit b = find_bin(h, rank, scratch);
+    v |= (K)b.bin << shift;
+    rank -= b.before;
+    equal = b.count;
+    top = shift;
+  }
+  const bool even = (count & 1) == 0;
+  K hi = v;
+  if (even && rank + 1 >= equal) {
+    K m = ~(K)0;
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+      if ((have >> i) & 1 && key[i] > v && key[i] < m) m = key[i];
+    hi = block_min_key(m, red);
+  }
+  if (threadIdx.x == 0) thr[blockIdx.x] = mad_of<T>(v, hi, even);
+}
+
+// Sampled range of keys around the median; also clears the plane's counters and bins.  PT keys a
+// thread, four neighbours from each of the sample's strata (one cache line each) at a place that a
+// hash picks, so that a pattern in the plane does not line up with them.
+template <class T, bool MASKED, int PT>
+__global__ __launch_bounds__(kMT) void k_mad_pivot(const T* __restrict__ planes, size_t plane, int w, Rect inc,
+                                                   Rect exc, uint32_t area, MadRange<typename MadKey<T>::K>* st,
+                                                   uint32_t* __restrict__ hist, const int* pred) {
+  using K = typename MadKey<T>::K;
+  if (pred_off(pred)) return;
+  constexpr int kKeyBits = 8 * sizeof(K) - 1;
+  __shared__ uint32_t h0[kBins], h1[kBins];
+  __shared__ BinScratch scratch;
+  __shared__ uint32_t taken;
+  const int s = blockIdx.x, t = threadIdx.x;
+  const T* x = planes + (size_t)s * plane;
+  if (t < kMadBins) hist[(size_t)s * kMadBins + t] = 0;
+  if (t == 0) taken = 0;
+  const uint32_t stratum = area / (PT / 4 * kMT);  // at least 16 (area > kMadOne)
+  K key[PT];
+  uint32_t have = 0;
+  const bool vec = !MASKED && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < PT / 4; ++i) {
+    const uint32_t c = t + i * kMT;
+    const uint32_t at = c * stratum + ((c * 2654435761u) >> 8) % (stratum - 3);
+    if (vec) {
+      const Quad<T> q = reinterpret_cast<const Quad<T>*>(x)[at / 4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) key[4 * i + k] = MadKey<T>::key(q.a[k]);
+      have |= 15u << (4 * i);
+      continue;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (noise_key<T, MASKED>(x, w, inc, exc, at + k, &key[4 * i + k])) have |= 1u << (4 * i + k);
+  }
+  __syncthreads();
+  atomicAdd(&taken, (uint32_t)__popc(have));
+  __syncthreads();
+  const uint32_t m = taken;
+  const uint32_t half = (uint32_t)(4.f * sqrtf((float)m)) + 8;
+  uint32_t r0 = m / 2 > half ? m / 2 - half : 0, r1 = m / 2 + half;
+  const bool open0 = m / 2 <= half, open1 = r1 >= m;
+  // Digits of both ends: two, which is a range's width to better than a tenth, or three (a float32 key)
+  // where both ends share two, as where many keys are equal.
+  K lo = 0, hi = 0;
+  int rest = kKeyBits;
+  for (int top = kKeyBits, pass = 0; top > 0 && (pass < 2 || (pass < 3 && lo == hi)); ++pass) {
+    const int nd = min(11, top), shift = top - nd;
+    const bool apart = lo != hi;
+    clear_bins(h0);
+    clear_bins(h1);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      if (!((have >> i) & 1)) continue;
+      const uint32_t d = (uint32_t)(key[i] >> shift) & ((1u << nd) - 1);
+      if ((key[i] >> top) == (lo >> top)) atomicAdd(&h0[d], 1u);
+      if (apart && (key[i] >> top) == (hi >> top)) atomicAdd(&h1[d], 1u);
+    }
+    __syncthreads();
+    BinHit a, b;
+    find_bins(h0, r0, r1, scratch, &a, &b);
+    if (apart) b = find_bin(h1, r1, scratch);
+    lo |= (K)a.bin << shift;
+    hi |= (K)b.bin << shift;
+    r0 -= a.before;
+    r1 -= b.before;
+    top = shift;
+    rest = top;
+  }
+  if (t == 0) {
+    hi |= ((K)1 << rest) - 1;
+    MadRange<K> z{};
+    if (open0) lo = 0;
+    if (open1) hi = ((K)1 << kKeyBits) - 1;
+    z.lo = lo;
+    z.range = hi - lo;
+    z.least2 = ~(K)0;
+    const int bits = bit_length<K>(z.range);
+    z.shift = bits > 6 ? bits - 6 : 0;
+    st[s] = z;
+  }
+}
+
+// The pass over the planes, eight keys (four float64) a thread at a time: keys below the range are
+// counted, keys in it go to an LDS bin and to the wave's part of an LDS list (slots from a prefix sum
+// over the wave, no atomic), which the wave appends to the plane's buffer with one reservation when it fills
+// and at the end.  Bound: reading the
+// planes (137 us for seven of 4096^2, against 95 us for each of the radix select's three passes); what
+// stands above that is the prefix sums and bins.  A reservation for every few hundred keys of a wave made it
+// 279 us: atomics on one address follow one another.
+template <class T, bool MASKED>
+__global__ __launch_bounds__(kT) void k_mad_scan(const T* __restrict__ planes, size_t plane, int w, Rect inc, Rect exc,
+                                                 MadRange<typename MadKey<T>::K>* __restrict__ st,
+                                                 uint32_t* __restrict__ hist,
+                                                 typename MadKey<T>::K* __restrict__ aside, size_t room,
+                                                 const int* pred) {
+  using K = typename MadKey<T>::K;
+  if (pred_off(pred)) return;
+  constexpr int V = 16 / sizeof(T), G = 2 * V;  // keys of a vector, of a group
+  constexpr int kStage = 64 * G + 768;          // room for a large plane's share of a wave: one reservation a block
+  __shared__ uint32_t h[kMadBins];
+  __shared__ K stage[kT / 64][kStage];
+  __shared__ uint32_t counts[kT / 64], belows[kT / 64], base_all;
+  const int s = blockIdx.y;
+  MadRange<K>* S = st + s;
+  const K lo = S->lo, range = S->range;
+  const uint32_t shift = S->shift;
+  K* out = aside + (size_t)s * room;
+  if (threadIdx.x < kMadBins) h[threadIdx.x] = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  K* mine = stage[threadIdx.x >> 6];
+  uint32_t below = 0;
+  int n = 0;  // keys in the wave's part, the same in all its lanes
+  auto flush = [&] {
+    __builtin_amdgcn_wave_barrier();  // the other lanes' LDS writes precede the reads below (one wave: in order)
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(&S->n, (uint32_t)n);
+    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+    for (int i = lane; i < n; i += 64)
+      if ((size_t)base + i < room) out[base + i] = mine[i];
+    n = 0;
+    __builtin_amdgcn_wave_barrier();
+  };
+  // `live`: which of the lane's keys are noise pixels; every lane of a wave takes every group
+  auto take = [&](const K (&key)[G], uint32_t live) {
+    uint32_t in = 0;
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      below += (live >> k) & (key[k] < lo ? 1u : 0u);
+      in |= key[k] - lo <= range ? 1u << k : 0u;
+    }
+    in &= live;
+    uint32_t at = __popc(in);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t v = __shfl_up(at, o, 64);
+      if (lane >= o) at += v;
+    }
+    const int total = __builtin_amdgcn_readlane((int)at, 63);
+    if (total == 0) return;
+    at += (uint32_t)n - __popc(in);
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      if (!((in >> k) & 1)) continue;
+      atomicAdd(&h[(uint32_t)((key[k] - lo) >> shift)], 1u);
+      mine[at + __popc(in & ((1u << k) - 1))] = key[k];
+    }
+    if (shift != 0) n += total;  // otherwise a bin is one key and the bins say all
+    if (n > kStage - 64 * G) flush();
+  };
+  const T* x = planes + (size_t)s * plane;
+  const size_t thr = blockIdx.x * (size_t)kT + threadIdx.x, nthr = (size_t)gridDim.x * kT;
+  K key[G];
+  if constexpr (!MASKED) {
+    struct alignas(16) Vec {
+      T a[V];
+    };
+    const size_t nv = (reinterpret_cast<uintptr_t>(x) & 15) == 0 ? plane / V : 0;
+    const Vec* xv = reinterpret_cast<const Vec*>(x);
+    for (size_t i0 = thr - lane; i0 < nv; i0 += 2 * nthr) {  // the wave's first vector
+      uint32_t live = 0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const size_t i = i0 + u * nthr + lane;
+        const Vec v = xv[min(i, nv - 1)];
+        live |= i < nv ? ((1u << V) - 1) << (u * V) : 0u;
+#pragma unroll
+        for (int k = 0; k < V; ++k) key[u * V + k] = MadKey<T>::key(v.a[k]);
+      }
+      take(key, live);
+    }
+    for (size_t i0 = nv * V + thr - lane; i0 < plane; i0 += G * nthr) {
+      uint32_t live = 0;
+#pragma unroll
+      for (int k = 0; k < G; ++k) {
+        const size_t i = i0 + k * nthr + lane;
+        key[k] = MadKey<T>::key(x[min(i, plane - 1)]);
+        live |= i < plane ? 1u << k : 0u;
+      }
+      take(key, live);
+    }
+  } else {
+    // a wave takes two rows by G / 2 columns a lane: no division per pixel
+    const int rstep = (int)(nthr >> 6);
+    for (int r = inc.r0 + (int)(thr >> 6); r < inc.r1; r += 2 * rstep) {
+      for (int c0 = inc.c0 + lane; c0 - lane < inc.c1; c0 += 32 * G) {
+        uint32_t live = 0;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int y = r + u * rstep;
+          const T* row = x + (size_t)min(y, inc.r1 - 1) * w;
+          const bool cut = y >= exc.r0 && y < exc.r1;
+#pragma unroll
+          for (int k = 0; k < G / 2; ++k) {
+            const int c = c0 + 64 * k;
+            key[u * (G / 2) + k] = MadKey<T>::key(row[min(c, inc.c1 - 1)]);
+            if (y < inc.r1 && c < inc.c1 && !(cut && c >= exc.c0 && c < exc.c1)) live |= 1u << (u * (G / 2) + k);
+          }
+        }
+        take(key, live);
+      }
+    }
+  }
+  // the block's remainder in one reservation: atomics on one address cost more than the copy
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o, 64);
+  if (lane == 0) {
+    counts[threadIdx.x >> 6] = (uint32_t)n;
+    belows[threadIdx.x >> 6] = below;
+  }
+  __syncthreads();
+  uint32_t before = 0, all = 0, low = 0;
+  for (int k = 0; k < kT / 64; ++k) {
+    before += k < (int)(threadIdx.x >> 6) ? counts[k] : 0;
+    all += counts[k];
+    low += belows[k];
+  }
+  if (threadIdx.x == 0) {
+    base_all = all ? atomicAdd(&S->n, all) : 0;
+    if (low) atomicAdd(&S->below, low);
+  }
+  if (threadIdx.x < kMadBins && h[threadIdx.x])
+    atomicAdd(&hist[(size_t)s * kMadBins + threadIdx.x], h[threadIdx.x]);
+  __syncthreads();
+  const size_t to = (size_t)base_all + before;
+  for (int i = lane; i < n; i += 64)
+    if (to + i < room) out[to + i] = mine[i];
+}
+
+// the 64 bins of a plane as the counts that find_bins takes
+__device__ __forceinline__ void load_bins(uint32_t* h, const uint32_t* __restrict__ hist, int s) {
+  clear_bins(h);
+  if (threadIdx.x < kMadBins) h[threadIdx.x] = hist[(size_t)s * kMadBins + threadIdx.x];
+  __syncthreads();
+}
+
+// Large planes: the keys of the median's bin and the least key of its successor's, by many blocks.
+template <class K>
+__global__ __launch_bounds__(kMT) void k_mad_collect(uint32_t count, MadRange<K>* __restrict__ st,
+                                                     const uint32_t* __restrict__ hist, const K* __restrict__ aside,
+                                                     size_t room, K* __restrict__ lists, size_t list_room,
+                                                     const int* pred) {
+  if (pred_off(pred)) return;
+  __shared__ uint32_t h[kBins];
+  __shared__ BinScratch scratch;
+  constexpr int V = 16 / sizeof(K);
+  __shared__ K stage[V * kMT];
+  __shared__ uint32_t n_stage, base;
+  const int s = blockIdx.y, t = threadIdx.x;
+  MadRange<K>* S = st + s;
+  const K lo = S->lo;
+  const uint32_t shift = S->shift, below = S->below, n = S->n, k = (count - 1) / 2;
+  if (shift == 0 || n > room || k < below) return;
+  load_bins(h, hist, s);
+  BinHit b, b2;  // of ranks in the range; k_mad_pick finds out if they are not
+  find_bins(h, k - below, k - below + ((count & 1) == 0 ? 1 : 0), scratch, &b, &b2);
+  struct alignas(16) Vec {
+    K a[V];
+  };
+  const Vec* bv = reinterpret_cast<const Vec*>(aside + (size_t)s * room);
+  K* list = lists + (size_t)s * list_room;
+  const uint32_t nv = (n + V - 1) / V;
+  K least2 = ~(K)0;
+  for (uint32_t i0 = blockIdx.x * kMT; i0 < nv; i0 += gridDim.x * kMT) {
+    const uint32_t i = i0 + t;
+    const Vec v = bv[min(i, nv - 1)];
+    if (t == 0) n_stage = 0;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      if (i >= nv || i * V + e >= n) break;
+      const int bin = (int)((v.a[e] - lo) >> shift);
+      if (bin == b.bin)
+        stage[atomicAdd(&n_stage, 1u)] = v.a[e];
+      else if (bin == b2.bin)
+        least2 = v.a[e] < least2 ? v.a[e] : least2;
+    }
+    __syncthreads();
+    const uint32_t m = n_stage;
+    if (t == 0 && m) base = atomicAdd(&S->listed, m);
+    __syncthreads();
+    for (uint32_t q = t; q < m; q += kMT)
+      if ((size_t)base + q < list_room) list[base + q] = stage[q];
+  }
+  __shared__ K red[kMT / 64];
+  least2 = block_min_key(least2, red);
+  if (t == 0 && least2 != ~(K)0) atomicMin(&S->least2, least2);
+}
+
+// The median's rank in the bins, then digits of 11 bits of its bin's keys: from the list that
+// k_mad_collect left (lists, large planes), from the keys set aside, or from the plane where the range
+// missed the rank or its keys found no room.
+template <class T, bool MASKED>
+__global__ __launch_bounds__(kMT) void k_mad_pick(const T* __restrict__ planes, size_t plane, int w, Rect inc, Rect exc,
+                                                  uint32_t count,
+                                                  const MadRange<typename MadKey<T>::K>* __restrict__ st,
+                                                  const uint32_t* __restrict__ hist,
+                                                  const typename MadKey<T>::K* __restrict__ aside, size_t room,
+                                                  const typename MadKey<T>::K* __restrict__ lists, size_t list_room,
+                                                  double* __restrict__ thr, const int* pred) {
+  using K = typename MadKey<T>::K;
+  if (pred_off(pred)) return;
+  __shared__ uint32_t h[kBins];
+  __shared__ BinScratch scratch;
+  __shared__ K red[kMT / 64];
+  const int s = blockIdx.x, t = threadIdx.x;
+  const T* x = planes + (size_t)s * plane;
+  const MadRange<K> S = st[s];
+  const bool even = (count & 1) == 0;
+  const uint32_t k = (count - 1) / 2;
+  load_bins(h, hist, s);
+  const BinHit last = find_bin(h, 0xffffffffu, scratch);
+  const uint32_t total = last.before + last.count;
+  const bool found = k >= S.below && k - S.below + (even ? 1 : 0) < total;
+  const bool listed = found && lists && S.n <= room && S.listed <= list_room;
+  // key - lo of every key that can be the median, and of at least all keys of the range up to its successor
+  const K lo = found ? S.lo : 0;
+  K v = 0;
+  K least2 = ~(K)0;
+  uint32_t rank = k, equal = 0;
+  int top = 8 * (int)sizeof(K) - 1;
+  if (found) {
+    BinHit b, b2;
+    find_bins(h, k - S.below, k - S.below + (even ? 1 : 0), scratch, &b, &b2);
+    v = (K)b.bin << S.shift;
+    rank = k - S.below - b.before;
+    equal = b.count;
+    top = (int)S.shift;
+    if (top == 0)
+      least2 = (K)b2.bin;
+    else if (listed && b2.bin != b.bin)
+      least2 = S.least2 - lo;
+  }
+  auto each = [&](auto f) {
+    if (listed || (found && S.n <= room)) {
+      const K* from = listed ? lists + (size_t)s * list_room : aside + (size_t)s * room;
+      const uint32_t n = listed ? S.listed : S.n;
+      for (uint32_t i0 = t; i0 < n; i0 += 8 * kMT) {
+        K q[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) q[u] = from[min(i0 + u * kMT, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (i0 + u * kMT < n) f(q[u] - lo);
+      }
+    } else {
+      each_noise_key<T, MASKED>(x, plane, w, inc, exc, t, kMT, [&](K key) {
+        if (!found || key - lo <= S.range) f(key - lo);
+      });
+    }
+  };
+  while (top > 0) {
+    const int nd = min(11, top), shift = top - nd;
+    clear_bins(h);
+    __syncthreads();
+    each([&](K rel) {
+      if ((rel >> top) == (v >> top)) atomicAdd(&h[(uint32_t)(rel >> shift) & ((1u << nd) - 1)], 1u);
+    });
+    __syncthreads();
+    const BinHit b = find_bin(h, rank, scratch);
+    v |= (K)b.bin << shift;
+    rank -= b.before;
+    equal = b.count;
+    top = shift;
+  }
+  K hi = v;
+  if (even && rank + 1 >= equal) {
+    K m = least2;
+    if (!(found && S.shift == 0)) each([&](K rel) { m = rel > v && rel < m ? rel : m; });
+    hi = block_min_key(m, red);
+  }
+  if (t == 0) thr[s] = mad_of<T>(lo + v, lo + hi, even);
+}
+
 // ----------------------------------------------------------------------------- threshold + maxima
 template <class T>
 __global__ __launch_bounds__(kT) void k_threshold(const T* __restrict__ in, T* __restrict__ out, size_t plane, int w,
@@ -660,12 +1273,6 @@ __global__ __launch_bounds__(kT) void k_ccl_flatten(int* __restrict__ lab, const
     l[i] = on ? ccl_find(l, (int)i) : -1;
   }
 }
-
-// four plane elements, stored together where the rows' alignment allows
-template <class T>
-struct alignas(16) Quad {
-  T a[4];
-};
 
 // Roots of the set ones (bits `on`) of four pixels from px on, walked side by side so that a step costs
 // one memory latency for all of them; returns which of the roots carry the keep mark.
@@ -1040,9 +1647,12 @@ NoiseMask noise_mask(int h, int w, int edge_excl, int int_excl) {
   return m;
 }
 
-// workspace layout is independent of the plane count and element type of a call:
-// [select state: 16 slots of 32 bytes][histograms 16 x 2048]
-size_t mad_work_bytes(int) { return (size_t)kMaxPlanes * (kSelBytes + kBins * sizeof(uint32_t)); }
+// workspace layout: [ranges: 16 slots][bins: 16 x kMadBins][keys set aside: S planes of mad_room keys]
+// [keys of the median's bin: S planes of mad_list_room keys].  Nothing in it has to be prepared.
+static size_t mad_aside_offset() { return (size_t)kMaxPlanes * (kRangeBytes + kMadBins * sizeof(uint32_t)); }
+size_t mad_work_bytes(int S, size_t plane, size_t real_bytes) {
+  return mad_aside_offset() + (size_t)S * (mad_room(plane) + mad_list_room(plane)) * real_bytes;
+}
 
 // Allocation-free median workspace: one file-scope device array per GPU, holding the select state
 // and histograms of one call of up to kMaxPlanes planes (131,584 bytes).  Host code never names
@@ -1071,7 +1681,7 @@ void* noalloc_mad_scratch() {
   return ptr;
 }
 
-void mad_work_init(void* work, int, hipStream_t st) {
+static void mad_select_init(void* work, hipStream_t st) {
   uint32_t* hist = (uint32_t*)((char*)work + (size_t)kMaxPlanes * kSelBytes);
   fill_u32(hist, (size_t)kMaxPlanes * kBins, 0u, st);
 }
@@ -1079,13 +1689,20 @@ void mad_work_init(void* work, int, hipStream_t st) {
 // Exact median per plane: radix select over the key bits in digits of at most 11 bits, one
 // histogram pass and one select step per digit; for even counts the last pass and select also find
 // the successor of the low median.
-template <class T>
-static void mad_thresholds_t(const T* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
-                             const int* pred, hipStream_t st) {
-  using K = typename MadKey<T>::K;
+static void check_mad(int S, const NoiseMask& nm) {
   PMS_REQUIRE(nm.count > 0, "noise mask selects no pixels");
   PMS_REQUIRE(nm.count < (1L << 32), "plane too large for the median");
   PMS_REQUIRE(S >= 1 && S <= kMaxPlanes, "the median handles 1..16 planes per call");
+}
+
+// the form for a workspace of kNoAllocMadBytes
+void mad_thresholds_noalloc(const float* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
+                            const int* pred, hipStream_t st) {
+  using T = float;
+  using K = typename MadKey<T>::K;
+  check_mad(S, nm);
+  // the histograms hold the previous call's contents (the select state is rewritten by the first kernel)
+  mad_select_init(work, st);
   SelStateT<K>* sst = (SelStateT<K>*)work;
   uint32_t* hist = (uint32_t*)((char*)work + (size_t)kMaxPlanes * kSelBytes);
   const size_t plane = (size_t)h * w;
@@ -1124,13 +1741,68 @@ static void mad_thresholds_t(const T* planes, int S, int h, int w, const NoiseMa
   hipLaunchKernelGGL(k_mad_finish<T>, dim3(ceil_div(S, 64)), dim3(64), 0, st, (const SelStateT<K>*)sst, S, thr, pred);
   PMS_LAUNCH_CHECK();
 }
+// Exact median per plane in one reading of it (k_mad_one, or k_mad_pivot / k_mad_scan / k_mad_pick).
+// The sample has 8192 keys below 2^20 noise pixels and 16384 above: a range of 8.8 and 6.3% of the
+// plane (32768: 4.4%, 35 instead of 20 us in k_mad_pivot for 4 us less in k_mad_scan).  From 2^20 pixels on the
+// median's bin is collected by many blocks: one block alone needs 45 us to look at what a 4096^2 plane sets
+// aside.  Seven 4096^2 planes take 190 us (340 us with the radix select), five 500^2 planes with an edge
+// mask 39 us (50 us), four 256^2 planes 26 us (33 us).
+template <class T, bool MASKED>
+static void mad_thresholds_t(const T* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
+                             const int* pred, hipStream_t st) {
+  using K = typename MadKey<T>::K;
+  check_mad(S, nm);
+  const size_t plane = (size_t)h * w;
+  const Rect inc{nm.inc_r0, nm.inc_r1, nm.inc_c0, nm.inc_c1};
+  const Rect exc{nm.exc_r0, nm.exc_r1, nm.exc_c0, nm.exc_c1};
+  const size_t area = (size_t)(inc.r1 - inc.r0) * (inc.c1 - inc.c0);
+  const uint32_t n = (uint32_t)nm.count;
+  PMS_REQUIRE(area < ((size_t)1 << 32), "plane too large for the median");
+  if (area <= (size_t)kMadOne) {
+    auto one = area <= (size_t)8 * kMT ? k_mad_one<T, MASKED, 8> : k_mad_one<T, MASKED, 32>;
+    hipLaunchKernelGGL(one, dim3(S), dim3(kMT), 0, st, planes, plane, w, inc, exc, (uint32_t)area, n, thr, pred);
+    PMS_LAUNCH_CHECK();
+    return;
+  }
+  MadRange<K>* range = (MadRange<K>*)work;
+  uint32_t* hist = (uint32_t*)((char*)work + (size_t)kMaxPlanes * kRangeBytes);
+  const size_t room = mad_room(plane), list_room = mad_list_room(plane);
+  K* aside = (K*)((char*)work + mad_aside_offset());
+  K* lists = aside + (size_t)S * room;
+  const bool large = area >= (size_t)1 << 20;
+  auto pivot = large ? k_mad_pivot<T, MASKED, 16> : k_mad_pivot<T, MASKED, 8>;
+  hipLaunchKernelGGL(pivot, dim3(S), dim3(kMT), 0, st, planes, plane, w, inc, exc, (uint32_t)area, range, hist, pred);
+  PMS_LAUNCH_CHECK();
+  // one group of keys a thread until 512 blocks a plane
+  const int gx = (int)std::min<size_t>((area + kT * (32 / sizeof(T)) - 1) / (kT * (32 / sizeof(T))), 512);
+  hipLaunchKernelGGL((k_mad_scan<T, MASKED>), dim3(gx, S), dim3(kT), 0, st, planes, plane, w, inc, exc, range, hist,
+                     aside, room, pred);
+  PMS_LAUNCH_CHECK();
+  if (large) {
+    hipLaunchKernelGGL((k_mad_collect<K>), dim3(32, S), dim3(kMT), 0, st, n, range, (const uint32_t*)hist,
+                       (const K*)aside, room, lists, list_room, pred);
+    PMS_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL((k_mad_pick<T, MASKED>), dim3(S), dim3(kMT), 0, st, planes, plane, w, inc, exc, n,
+                     (const MadRange<K>*)range, (const uint32_t*)hist, (const K*)aside, room,
+                     large ? (const K*)lists : (const K*)nullptr, list_room, thr, pred);
+  PMS_LAUNCH_CHECK();
+}
+template <class T>
+static void mad_thresholds_any(const T* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
+                               const int* pred, hipStream_t st) {
+  if (nm.masked)
+    mad_thresholds_t<T, true>(planes, S, h, w, nm, thr, work, pred, st);
+  else
+    mad_thresholds_t<T, false>(planes, S, h, w, nm, thr, work, pred, st);
+}
 void mad_thresholds(const float* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
                     const int* pred, hipStream_t st) {
-  mad_thresholds_t(planes, S, h, w, nm, thr, work, pred, st);
+  mad_thresholds_any(planes, S, h, w, nm, thr, work, pred, st);
 }
 void mad_thresholds(const double* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
                     const int* pred, hipStream_t st) {
-  mad_thresholds_t(planes, S, h, w, nm, thr, work, pred, st);
+  mad_thresholds_any(planes, S, h, w, nm, thr, work, pred, st);
 }
 
 int threshold_grid(size_t plane) { return std::min(ew_grid(plane), 256); }
@@ -1222,8 +1894,8 @@ static void source_extract_t(const T* w, int S, int h, int wd, double tol, int n
   // keep rule from the coarsest scale down: mark S-1; apply s and mark s-1; ...; apply 0
   const bool vec = wd % 4 == 0 && aligned16(extracted) && (reinterpret_cast<uintptr_t>(mask) & 3) == 0;
   const unsigned quads = (unsigned)h * (unsigned)ceil_div(wd, 4);
-  // four quads a thread once that still leaves eight blocks per CU (from about 2900^2 pixels on); below, a thread's chain
-  // of dependent reads sets the time and more threads hide it
+  // four quads a thread once that still leaves eight blocks per CU (from about 2900^2 pixels on);
+  // below, a thread's chain of dependent reads sets the time and more threads hide it
   const bool four = quads >= 4u * kT * 2048;
   const unsigned per = kT * (four ? 4 : 1);
   auto keep = vec ? (four ? k_keep_step<T, true, 4> : k_keep_step<T, true, 1>)
