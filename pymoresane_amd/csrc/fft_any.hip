@@ -5,10 +5,9 @@
 // PSF product, inverse) -> rows c2r with scale and crop, the image at the frame origin and the
 // P/2 roll folded into the PSF frame.  Differences: the transforms are mixed radix (2, 3, 4, 5,
 // 7, 8, 11, 13) with the radix plan chosen at run time, and every kernel is templated on the
-// arithmetic type, so this file serves
-//   * float32 frames whose side is not a power of two (the reference's numpy rfft2 takes any
-//     size, iuwt_convolution.py:64-73), and
-//   * the float64 path of every frame side (the deconvolution's float64 precision mode).
+// arithmetic type, so this file serves frames whose side is not a power of two (the reference's
+// numpy rfft2 takes any size, iuwt_convolution.py:64-73) in float32 and in float64 (the
+// deconvolution's float64 precision mode).
 //
 // Each transform of length L runs in LDS as in-place decimation-in-frequency stages (forward,
 // output in mixed-radix digit-reversed order) or their exact mirror (inverse, decimation in time,
@@ -526,6 +525,12 @@ void gfft_psf_spectrum(const TIN* psf, int q, int p, Cx<T>* spec, Cx<T>* work,
                        hipStream_t st) {
   check_g_frame<T>(p);
   PMS_REQUIRE(q >= 1 && q <= p, "PSF larger than the FFT frame");
+  if constexpr (sizeof(T) == 8) {
+    if (is_pow2(p)) {
+      pow2_psf_spectrum_f64(psf, q, p, spec, work, st);
+      return;
+    }
+  }
   set_g_attrs<T>();
   const auto* tw = g_twiddles<T>(p);
   GR2cBatch<T> rb{};
@@ -542,6 +547,12 @@ template <class T>
 void gfft_conv_batch(const GConvJob<T>* jobs, int count, int n, int p, hipStream_t st) {
   check_g_frame<T>(p);
   PMS_REQUIRE(p == n || p == 2 * n, "fft_conv: frame must be N (circular) or 2N (linear)");
+  if constexpr (sizeof(T) == 8) {
+    if (is_pow2(p)) {
+      pow2_conv_batch_f64(jobs, count, n, p, st);
+      return;
+    }
+  }
   set_g_attrs<T>();
   const auto* tw = g_twiddles<T>(p);
   const int L = p / 2;

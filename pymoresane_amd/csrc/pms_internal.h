@@ -193,11 +193,10 @@ void iuwt_recompose_batch(const IuwtRecompJobT<double>* jobs, int count, int h, 
 long iuwt_decompose_partials_f64(int h, int w, int scale_count, int scale_adjust);
 
 // ------------------------------------------------------------------------ FFT
-// Device twiddle table exp(-2 pi i k / kFftMaxLen), k in [0, kFftMaxLen).
+// Length of the device twiddle tables exp(-2 pi i k / kFftMaxLen), k in [0, kFftMaxLen).
 constexpr int kFftMaxLog2 = 14;
 constexpr int kFftMaxLen = 1 << kFftMaxLog2;
 void fft_init_device(int device);
-const float2* fft_twiddles();
 
 // Spectrum layout: (P/2+1) frequency columns, each holding P values along the
 // other axis in the library's digit-reversed FFT order, already carrying the
@@ -223,8 +222,8 @@ void fft_spectrum_from_numpy_host(const float* re_im, int p, float2* spec_host);
 int fft_perm(int k, int p);  // storage position of frequency k in a length-p column
 
 // Mixed-radix FFT convolution (fft_any.hip) for any even frame side with prime factors up to 13,
-// in float32 or float64; spectra and scratch in the library complex type Cx<T>.  The float32
-// power-of-two frames keep the kernels above; the float32 entry points above route other frames
+// in float32 or float64; spectra and scratch in the library complex type Cx<T>.  Power-of-two
+// frames have kernels of their own (fft_pow2.h); the float32 entry points above route other frames
 // here.  Layout as above ((P/2+1) columns of P values in the transform's digit-reversed order).
 template <class T>
 struct alignas(2 * sizeof(T)) Cx {
@@ -245,6 +244,11 @@ template <class T, class TIN>
 void gfft_psf_spectrum(const TIN* psf, int q, int p, Cx<T>* spec, Cx<T>* work, hipStream_t st);
 template <class T>
 void gfft_conv_batch(const GConvJob<T>* jobs, int count, int n, int p, hipStream_t st);
+// the same in float64 for power-of-two frames up to 8192 (fft_f64.hip), which the two functions above route
+// there; such spectra are in the power-of-two kernels' order
+template <class TIN>
+void pow2_psf_spectrum_f64(const TIN* psf, int q, int p, Cx<double>* spec, Cx<double>* work, hipStream_t st);
+void pow2_conv_batch_f64(const GConvJob<double>* jobs, int count, int n, int p, hipStream_t st);
 
 // ------------------------------------------------------------------- toolbox
 // Element-typed helpers take float or double planes (the float64 precision mode of the driver).
