@@ -66,9 +66,9 @@ struct CgJob {
   int* iflag;  // iflag[kActive] == 0: the job's minor loop has exited, its kernels do nothing
   int enforce;
 };
-template <class T>
+template <class T, int NB>
 struct CgBatch {
-  CgJob<T> j[kMaxBatch];
+  CgJob<T> j[NB];
   size_t n;
 };
 
@@ -108,8 +108,8 @@ __device__ __forceinline__ T block_min_all(const double* __restrict__ partial, i
 }
 
 // per-block partials of p . Ap
-template <class T>
-__global__ __launch_bounds__(kT) void k_cg_pap(CgBatch<T> b) {
+template <class T, int NB>
+__global__ __launch_bounds__(kT) void k_cg_pap(CgBatch<T, NB> b) {
   const CgJob<T>& J = b.j[blockIdx.y];
   if (J.iflag[kActive] == 0) return;
   const V16<T>* __restrict__ p = reinterpret_cast<const V16<T>*>(J.p);
@@ -132,8 +132,8 @@ __device__ __forceinline__ T xn_of(double a, T p, T x) {
 
 // alpha = rr / (p . Ap) from k_cg_pap's np partials (every block adds them in the same order; block 0
 // stores p . Ap and alpha) ; xn = x + alpha p ; per-block minima of xn in the upper partials
-template <class T>
-__global__ __launch_bounds__(kT) void k_cg_xn(CgBatch<T> b, int np) {
+template <class T, int NB>
+__global__ __launch_bounds__(kT) void k_cg_xn(CgBatch<T, NB> b, int np) {
   const CgJob<T>& J = b.j[blockIdx.y];
   if (J.iflag[kActive] == 0) return;
   const double tot = block_total_all(J.partial, np);
@@ -164,8 +164,8 @@ __global__ __launch_bounds__(kT) void k_cg_xn(CgBatch<T> b, int np) {
 // positivity clip when enforce && min(xn) < 0 (the minimum of k_cg_xn's np per-block minima;
 // block 0 stores the flag, which predicates the clip pass's operator launches):
 // xn[xn<0] = 0 ; p = (xn - x) / alpha
-template <class T>
-__global__ __launch_bounds__(kT) void k_cg_clip(CgBatch<T> b, int np) {
+template <class T, int NB>
+__global__ __launch_bounds__(kT) void k_cg_clip(CgBatch<T, NB> b, int np) {
   const CgJob<T>& J = b.j[blockIdx.y];
   if (J.iflag[kActive] == 0) {  // the clip pass's operator launches are predicated on this flag
     if (blockIdx.x == 0 && threadIdx.x == 0) J.iflag[kClip] = 0;
@@ -218,17 +218,17 @@ struct RnJob {
   size_t n_snr;  // SNR elements: scales x plane (a multiple of 4)
   int nblk_snr;  // blocks and partials of the SNR pass (a function of n_snr only)
 };
-template <class T>
+template <class T, int NB>
 struct RnBatch {
-  RnJob<T> j[kMaxBatch];
+  RnJob<T> j[NB];
   size_t n;  // CG vector length
   int np;    // blocks (and partials) of the rn pass: cg_grid(n)
 };
 
 // rn = r - alpha Ap with per-block partials of rn . rn in blocks [0, np) (lower partials), and
 // R <- R - alpha Dcg with per-block partials of R . R in blocks [0, nblk_snr) (upper partials).
-template <class T>
-__global__ __launch_bounds__(kT) void k_cg_rn(RnBatch<T> b) {
+template <class T, int NB>
+__global__ __launch_bounds__(kT) void k_cg_rn(RnBatch<T, NB> b) {
   const RnJob<T>& J = b.j[blockIdx.y];
   if (J.iflag[kActive] == 0) return;
   const double a = J.scal[kAlpha];
@@ -271,8 +271,8 @@ __global__ __launch_bounds__(kT) void k_cg_rn(RnBatch<T> b) {
 
 // rnrn = rn . rn (from k_cg_rn's np partials) ; beta = rnrn / rr (block 0 stores both) ;
 // p = rn + beta p
-template <class T>
-__global__ __launch_bounds__(kT) void k_cg_p(CgBatch<T> b, int np) {
+template <class T, int NB>
+__global__ __launch_bounds__(kT) void k_cg_p(CgBatch<T, NB> b, int np) {
   const CgJob<T>& J = b.j[blockIdx.y];
   if (J.iflag[kActive] == 0) return;
   const double tot = block_total_all(J.partial, np);
@@ -298,20 +298,25 @@ __global__ __launch_bounds__(kT) void k_cg_p(CgBatch<T> b, int np) {
 // fires, the exit code; an exit clears the job's active flag, which turns its later queued
 // iterations into no-ops.  The host reads the outcome after the step and replays the iterate swaps
 // of the iterations that ran.
+struct CtlJob {
+  double* scal;
+  int* iflag;
+  const double* partial;  // the SNR partials
+  int np;
+  int miter;
+};
+template <int NB>
 struct CtlBatch {
-  double* scal[kMaxBatch];
-  int* iflag[kMaxBatch];
-  const double* partial[kMaxBatch];  // the SNR partials
-  long np[kMaxBatch];
-  int miter[kMaxBatch];
+  CtlJob j[NB];
 };
 
-__global__ __launch_bounds__(kT) void k_minor_ctl(CtlBatch b) {
-  const int j = blockIdx.x;
-  double* sc = b.scal[j];
-  int* fl = b.iflag[j];
+template <int NB>
+__global__ __launch_bounds__(kT) void k_minor_ctl(CtlBatch<NB> b) {
+  const CtlJob& J = b.j[blockIdx.x];
+  double* sc = J.scal;
+  int* fl = J.iflag;
   if (fl[kActive] == 0) return;
-  const double d2 = block_total(b.partial[j], (int)b.np[j]);
+  const double d2 = block_total(J.partial, J.np);
   if (threadIdx.x != 0) return;
   sc[kD2] = d2;
   const double snr = 20.0 * log10(sqrt(sc[kE2]) / sqrt(sc[kD2]));
@@ -324,7 +329,7 @@ __global__ __launch_bounds__(kT) void k_minor_ctl(CtlBatch b) {
     code = EXIT_ACCEPT;
   else if (niter > 2 && snr <= last)
     code = snr > 10.5 ? EXIT_FELL_OK : EXIT_FELL_LOW;
-  else if (niter >= b.miter[j])
+  else if (niter >= J.miter)
     code = EXIT_CAP;
   sc[kSnrLast] = last;
   sc[kSnrCur] = snr;
@@ -400,16 +405,31 @@ int cg_grid(size_t n) {
   return (int)(b < 1 ? 1 : (b > 1024 ? 1024 : b));
 }
 
-template <class T, class K>
-void launch_cg(K kernel, const CgBatch<T>& b, int nb, hipStream_t st) {
-  hipLaunchKernelGGL(kernel, dim3(cg_grid(b.n), nb), dim3(kT), 0, st, b);
+// The batch of a launch of one job, in the kernels' one-job argument form (see kMaxBatch).
+template <class T>
+CgBatch<T, 1> only_job(const CgBatch<T, kMaxBatch>& b) {
+  return CgBatch<T, 1>{{b.j[0]}, b.n};
+}
+
+// k1 and k: a kernel's forms for one job and for kMaxBatch
+template <class T>
+void launch_cg(void (*k1)(CgBatch<T, 1>), void (*k)(CgBatch<T, kMaxBatch>), const CgBatch<T, kMaxBatch>& b, int nb,
+               hipStream_t st) {
+  if (nb == 1)
+    hipLaunchKernelGGL(k1, dim3(cg_grid(b.n), 1), dim3(kT), 0, st, only_job(b));
+  else
+    hipLaunchKernelGGL(k, dim3(cg_grid(b.n), nb), dim3(kT), 0, st, b);
   PMS_LAUNCH_CHECK();
 }
 
 // a streaming kernel that also finishes the previous kernel's reduction (cg_grid(n) partials)
-template <class T, class K>
-void launch_cg_after(K kernel, const CgBatch<T>& b, int nb, hipStream_t st) {
-  hipLaunchKernelGGL(kernel, dim3(cg_grid(b.n), nb), dim3(kT), 0, st, b, cg_grid(b.n));
+template <class T>
+void launch_cg_after(void (*k1)(CgBatch<T, 1>, int), void (*k)(CgBatch<T, kMaxBatch>, int),
+                     const CgBatch<T, kMaxBatch>& b, int nb, hipStream_t st) {
+  if (nb == 1)
+    hipLaunchKernelGGL(k1, dim3(cg_grid(b.n), 1), dim3(kT), 0, st, only_job(b), cg_grid(b.n));
+  else
+    hipLaunchKernelGGL(k, dim3(cg_grid(b.n), nb), dim3(kT), 0, st, b, cg_grid(b.n));
   PMS_LAUNCH_CHECK();
 }
 
@@ -1403,11 +1423,11 @@ void Runner::enqueue_iterations_t(const std::vector<IterArgs>& its, const std::v
   const int nb = (int)ts.size();
   const int sub = its[0].sub, p_sub = its[0].p_sub;
   const size_t s2 = (size_t)sub * sub;
-  CgBatch<T> cb{};
+  CgBatch<T, kMaxBatch> cb{};
   cb.n = s2;
   std::vector<Task*> clip_ts;
   std::vector<IterArgs> clip_its;
-  CgBatch<T> clip_b{};
+  CgBatch<T, kMaxBatch> clip_b{};
   clip_b.n = s2;
   for (int i = 0; i < nb; ++i) {
     const IterArgs& a = its[i];
@@ -1422,18 +1442,18 @@ void Runner::enqueue_iterations_t(const std::vector<IterArgs>& its, const std::v
     }
   }
   apply_op<T>(ts, its, false);
-  launch_cg(k_cg_pap<T>, cb, nb, st_);
-  launch_cg_after(k_cg_xn<T>, cb, nb, st_);
+  launch_cg<T>(k_cg_pap<T, 1>, k_cg_pap<T, kMaxBatch>, cb, nb, st_);
+  launch_cg_after<T>(k_cg_xn<T, 1>, k_cg_xn<T, kMaxBatch>, cb, nb, st_);
   if (!clip_ts.empty()) {
-    launch_cg_after(k_cg_clip<T>, clip_b, (int)clip_ts.size(), st_);
+    launch_cg_after<T>(k_cg_clip<T, 1>, k_cg_clip<T, kMaxBatch>, clip_b, (int)clip_ts.size(), st_);
     apply_op<T>(clip_ts, clip_its, true);
   }
   // rn, and in the incremental form the SNR sums (main.py:413-424) in the same launch
-  RnBatch<T> rb{};
+  RnBatch<T, kMaxBatch> rb{};
   rb.n = s2;
   rb.np = cg_grid(s2);
   int gx = rb.np;
-  CtlBatch ctl{};
+  CtlBatch<kMaxBatch> ctl{};
   for (int i = 0; i < nb; ++i) {
     Job& J = *ts[i]->job();
     Planes<T>& B = J.pl<T>();
@@ -1443,15 +1463,14 @@ void Runner::enqueue_iterations_t(const std::vector<IterArgs>& its, const std::v
     rb.j[i] = RnJob<T>{(const T*)a.r, (const T*)a.ap, (T*)a.rn, snr_direct_ ? nullptr : B.Rs, B.Dcg, J.partial,
                        ts[i]->scal(), ts[i]->iflag(), n, nblk};
     if (!snr_direct_) gx = std::max(gx, nblk);
-    ctl.scal[i] = ts[i]->scal();
-    ctl.iflag[i] = ts[i]->iflag();
-    ctl.partial[i] = J.partial + kPartialHi;
-    ctl.np[i] = nblk;
-    ctl.miter[i] = ts[i]->spec.prm.minor_loop_miter;
+    ctl.j[i] = CtlJob{ts[i]->scal(), ts[i]->iflag(), J.partial + kPartialHi, nblk, ts[i]->spec.prm.minor_loop_miter};
   }
-  hipLaunchKernelGGL(k_cg_rn<T>, dim3(gx, nb), dim3(kT), 0, st_, rb);
+  if (nb == 1)
+    hipLaunchKernelGGL((k_cg_rn<T, 1>), dim3(gx, 1), dim3(kT), 0, st_, (RnBatch<T, 1>{{rb.j[0]}, rb.n, rb.np}));
+  else
+    hipLaunchKernelGGL((k_cg_rn<T, kMaxBatch>), dim3(gx, nb), dim3(kT), 0, st_, rb);
   PMS_LAUNCH_CHECK();
-  launch_cg_after(k_cg_p<T>, cb, nb, st_);
+  launch_cg_after<T>(k_cg_p<T, 1>, k_cg_p<T, kMaxBatch>, cb, nb, st_);
   if (snr_direct_) {
     // main.py:413-424 as written: convolve xn, decompose it against the extracted sources
     std::vector<typename EngineTypes<T>::Conv> fj;
@@ -1468,12 +1487,15 @@ void Runner::enqueue_iterations_t(const std::vector<IterArgs>& its, const std::v
     conv_batch(fj.data(), nb, sub, p_sub, st_);
     decompose_batch(dj.data(), nb, sub, sub, st_);
     for (int i = 0; i < nb; ++i) {
-      ctl.partial[i] = ts[i]->job()->partial;
-      ctl.np[i] = dj[i].np;
+      ctl.j[i].partial = ts[i]->job()->partial;
+      ctl.j[i].np = (int)dj[i].np;
     }
   }
   // exit rules of every job of the chunk (main.py:427-457)
-  hipLaunchKernelGGL(k_minor_ctl, dim3(nb), dim3(kT), 0, st_, ctl);
+  if (nb == 1)
+    hipLaunchKernelGGL(k_minor_ctl<1>, dim3(1), dim3(kT), 0, st_, (CtlBatch<1>{{ctl.j[0]}}));
+  else
+    hipLaunchKernelGGL(k_minor_ctl<kMaxBatch>, dim3(nb), dim3(kT), 0, st_, ctl);
   PMS_LAUNCH_CHECK();
 }
 

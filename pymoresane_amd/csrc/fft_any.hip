@@ -232,31 +232,31 @@ __device__ __forceinline__ void gfft_inverse(Cx<T>* sm, const GPlan& p, int TL, 
   }
 }
 
-template <class T>
+template <class T, int NB>
 struct GR2cBatch {
-  const void* src[kMaxBatch];
-  Cx<T>* T1[kMaxBatch];
-  const int* pred[kMaxBatch];
+  const void* src[NB];
+  Cx<T>* T1[NB];
+  const int* pred[NB];
 };
-template <class T>
+template <class T, int NB>
 struct GColBatch {
-  const Cx<T>* T1[kMaxBatch];
-  const Cx<T>* S[kMaxBatch];
-  Cx<T>* T2[kMaxBatch];
-  const int* pred[kMaxBatch];
+  const Cx<T>* T1[NB];
+  const Cx<T>* S[NB];
+  Cx<T>* T2[NB];
+  const int* pred[NB];
 };
-template <class T>
+template <class T, int NB>
 struct GC2rBatch {
-  const Cx<T>* T2[kMaxBatch];
-  T* out[kMaxBatch];
-  const int* pred[kMaxBatch];
+  const Cx<T>* T2[NB];
+  T* out[NB];
+  const int* pred[NB];
 };
 
 // ---- pass 1: rows r2c.  Frame row fr of the job: the image row (off == 0, q x q image at the
 // frame origin) or the PSF row of the centred, -P/2-rolled frame (off = q/2).  Output column-major:
 // T1[k * ldT + fr], k in [0, P/2].
-template <class T, class TIN>
-__global__ __launch_bounds__(kGThreads) void k_g_r2c(GR2cBatch<T> bt, GPlan pl, int P, int q, int off, int n_rows,
+template <class T, class TIN, int NB>
+__global__ __launch_bounds__(kGThreads) void k_g_r2c(GR2cBatch<T, NB> bt, GPlan pl, int P, int q, int off, int n_rows,
                                                      int ldT, int G, const Cx<T>* __restrict__ tw) {
   using C = Cx<T>;
   const int jb = blockIdx.y;
@@ -301,8 +301,8 @@ __global__ __launch_bounds__(kGThreads) void k_g_r2c(GR2cBatch<T> bt, GPlan pl, 
 // ---- pass 2: per frequency column k in [0, P/2]: the n_in stored rows (zero beyond) -> forward
 // P-point FFT.  SPEC: store the spectrum column (digit-reversed order).  Otherwise multiply by the
 // PSF column (same order), inverse FFT, store the first n_out rows: T2[k * n_out + i].
-template <class T, bool SPEC>
-__global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T> bt, GPlan pl, int n_in, int n_out, int G,
+template <class T, bool SPEC, int NB>
+__global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T, NB> bt, GPlan pl, int n_in, int n_out, int G,
                                                       const Cx<T>* __restrict__ tw) {
   using C = Cx<T>;
   const int jb = blockIdx.y;
@@ -339,8 +339,8 @@ __global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T> bt, GPlan pl,
 // ---- pass 3: per kept row r: Hermitian half spectrum T2[k * ldT + r], k in [0, P/2] -> the
 // P/2-point complex sequence whose inverse FFT interleaves the even and odd output samples, scaled
 // by 1/P^2; the first n columns are stored.
-template <class T>
-__global__ __launch_bounds__(kGThreads) void k_g_c2r(GC2rBatch<T> bt, GPlan pl, int P, int n, int ldT, int G, T scale,
+template <class T, int NB>
+__global__ __launch_bounds__(kGThreads) void k_g_c2r(GC2rBatch<T, NB> bt, GPlan pl, int P, int n, int ldT, int G, T scale,
                                                      const Cx<T>* __restrict__ tw) {
   using C = Cx<T>;
   const int jb = blockIdx.y;
@@ -447,11 +447,17 @@ void set_g_attrs() {
   static std::once_flag once;
   std::call_once(once, [] {
     const int lds_max = 160 * 1024;
-    (void)hipFuncSetAttribute((const void*)k_g_r2c<T, float>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void*)k_g_r2c<T, double>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void*)k_g_cols<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void*)k_g_cols<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-    (void)hipFuncSetAttribute((const void*)k_g_c2r<T>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+    auto allow = [&](const void* k) {
+      (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+    };
+    allow((const void*)k_g_r2c<T, float, 1>);
+    allow((const void*)k_g_r2c<T, double, 1>);
+    allow((const void*)k_g_r2c<T, T, kMaxBatch>);
+    allow((const void*)k_g_cols<T, true, 1>);
+    allow((const void*)k_g_cols<T, false, 1>);
+    allow((const void*)k_g_cols<T, false, kMaxBatch>);
+    allow((const void*)k_g_c2r<T, 1>);
+    allow((const void*)k_g_c2r<T, kMaxBatch>);
     (void)hipGetLastError();
   });
 }
@@ -467,41 +473,41 @@ void check_g_frame(int p) {
               "FFT frame side " + std::to_string(p) + " has a prime factor above 13");
 }
 
-template <class T, class TIN>
-void launch_r2c(const GR2cBatch<T>& bt, int nb, int p, int q, int off, int n_rows, int ldT,
+template <class T, class TIN, int NB>
+void launch_r2c(const GR2cBatch<T, NB>& bt, int nb, int p, int q, int off, int n_rows, int ldT,
                 const Cx<T>* tw, hipStream_t st) {
   using C = Cx<T>;
   GPlan pl;
   make_gplan(p / 2, &pl);
   const int G = groups_for(p / 2, sizeof(C));
   const size_t lds = (size_t)G * gspan(p / 2) * sizeof(C);
-  hipLaunchKernelGGL((k_g_r2c<T, TIN>), dim3(ceil_div(n_rows, G), nb), dim3(kGThreads), lds, st, bt, pl, p, q, off,
+  hipLaunchKernelGGL((k_g_r2c<T, TIN, NB>), dim3(ceil_div(n_rows, G), nb), dim3(kGThreads), lds, st, bt, pl, p, q, off,
                      n_rows, ldT, G, tw);
   PMS_LAUNCH_CHECK();
 }
 
-template <class T, bool SPEC>
-void launch_cols(const GColBatch<T>& bt, int nb, int p, int n_in, int n_out, const Cx<T>* tw,
+template <class T, bool SPEC, int NB>
+void launch_cols(const GColBatch<T, NB>& bt, int nb, int p, int n_in, int n_out, const Cx<T>* tw,
                  hipStream_t st) {
   using C = Cx<T>;
   GPlan pl;
   make_gplan(p, &pl);
   const int G = groups_for(p, sizeof(C));
   const size_t lds = (size_t)G * gspan(p) * sizeof(C);
-  hipLaunchKernelGGL((k_g_cols<T, SPEC>), dim3(ceil_div(p / 2 + 1, G), nb), dim3(kGThreads), lds, st, bt, pl, n_in,
+  hipLaunchKernelGGL((k_g_cols<T, SPEC, NB>), dim3(ceil_div(p / 2 + 1, G), nb), dim3(kGThreads), lds, st, bt, pl, n_in,
                      n_out, G, tw);
   PMS_LAUNCH_CHECK();
 }
 
-template <class T>
-void launch_c2r(const GC2rBatch<T>& bt, int nb, int p, int n, int ldT, const Cx<T>* tw, hipStream_t st) {
+template <class T, int NB>
+void launch_c2r(const GC2rBatch<T, NB>& bt, int nb, int p, int n, int ldT, const Cx<T>* tw, hipStream_t st) {
   using C = Cx<T>;
   GPlan pl;
   make_gplan(p / 2, &pl);
   const int G = groups_for(p / 2, sizeof(C));
   const size_t lds = (size_t)G * gspan(p / 2) * sizeof(C);
   const T scale = (T)(1.0 / ((double)p * (double)p));
-  hipLaunchKernelGGL(k_g_c2r<T>, dim3(ceil_div(n, G), nb), dim3(kGThreads), lds, st, bt, pl, p, n, ldT, G, scale, tw);
+  hipLaunchKernelGGL((k_g_c2r<T, NB>), dim3(ceil_div(n, G), nb), dim3(kGThreads), lds, st, bt, pl, p, n, ldT, G, scale, tw);
   PMS_LAUNCH_CHECK();
 }
 
@@ -533,15 +539,43 @@ void gfft_psf_spectrum(const TIN* psf, int q, int p, Cx<T>* spec, Cx<T>* work,
   }
   set_g_attrs<T>();
   const auto* tw = g_twiddles<T>(p);
-  GR2cBatch<T> rb{};
+  GR2cBatch<T, 1> rb{};
   rb.src[0] = psf;
   rb.T1[0] = work;
   launch_r2c<T, TIN>(rb, 1, p, q, q / 2, p, p, tw, st);
-  GColBatch<T> cb{};
+  GColBatch<T, 1> cb{};
   cb.T1[0] = work;
   cb.T2[0] = spec;
   launch_cols<T, true>(cb, 1, p, p, p, tw, st);
 }
+
+namespace {
+template <class T, int NB>
+void gfft_conv_jobs(const GConvJob<T>* jobs, int nb, int n, int p, const Cx<T>* tw, hipStream_t st) {
+  GR2cBatch<T, NB> rb{};
+  GColBatch<T, NB> cb{};
+  GC2rBatch<T, NB> ob{};
+  for (int k = 0; k < nb; ++k) {
+    const GConvJob<T>& j = jobs[k];
+    PMS_REQUIRE(j.in && j.spec && j.out && j.work, "fft_conv: NULL buffer");
+    auto* T1 = j.work;
+    auto* T2 = j.work + (size_t)(p / 2 + 1) * n;
+    rb.src[k] = j.in;
+    rb.T1[k] = T1;
+    rb.pred[k] = j.pred;
+    cb.T1[k] = T1;
+    cb.S[k] = j.spec;
+    cb.T2[k] = T2;
+    cb.pred[k] = j.pred;
+    ob.T2[k] = T2;
+    ob.out[k] = j.out;
+    ob.pred[k] = j.pred;
+  }
+  launch_r2c<T, T>(rb, nb, p, n, 0, n, n, tw, st);
+  launch_cols<T, false>(cb, nb, p, n, n, tw, st);
+  launch_c2r<T>(ob, nb, p, n, n, tw, st);
+}
+}  // namespace
 
 template <class T>
 void gfft_conv_batch(const GConvJob<T>* jobs, int count, int n, int p, hipStream_t st) {
@@ -555,31 +589,12 @@ void gfft_conv_batch(const GConvJob<T>* jobs, int count, int n, int p, hipStream
   }
   set_g_attrs<T>();
   const auto* tw = g_twiddles<T>(p);
-  const int L = p / 2;
   for (int j0 = 0; j0 < count; j0 += kMaxBatch) {
     const int nb = std::min(kMaxBatch, count - j0);
-    GR2cBatch<T> rb{};
-    GColBatch<T> cb{};
-    GC2rBatch<T> ob{};
-    for (int k = 0; k < nb; ++k) {
-      const GConvJob<T>& j = jobs[j0 + k];
-      PMS_REQUIRE(j.in && j.spec && j.out && j.work, "fft_conv: NULL buffer");
-      auto* T1 = j.work;
-      auto* T2 = j.work + (size_t)(L + 1) * n;
-      rb.src[k] = j.in;
-      rb.T1[k] = T1;
-      rb.pred[k] = j.pred;
-      cb.T1[k] = T1;
-      cb.S[k] = j.spec;
-      cb.T2[k] = T2;
-      cb.pred[k] = j.pred;
-      ob.T2[k] = T2;
-      ob.out[k] = j.out;
-      ob.pred[k] = j.pred;
-    }
-    launch_r2c<T, T>(rb, nb, p, n, 0, n, n, tw, st);
-    launch_cols<T, false>(cb, nb, p, n, n, tw, st);
-    launch_c2r<T>(ob, nb, p, n, n, tw, st);
+    if (nb == 1)
+      gfft_conv_jobs<T, 1>(jobs + j0, nb, n, p, tw, st);
+    else
+      gfft_conv_jobs<T, kMaxBatch>(jobs + j0, nb, n, p, tw, st);
   }
 }
 

@@ -251,31 +251,32 @@ __device__ __forceinline__ void mid_forward(C* sm, int L, int ns, int i0, int i1
   }
 }
 
-// Per-job pointers of a batched launch (grid y selects the job).
-template <class C>
+// Per-job pointers of a batched launch (grid y selects the job), for NB = 1 or kMaxBatch jobs: see
+// kMaxBatch on what the size of a launch's arguments costs.
+template <class C, int NB>
 struct R2cBatch {
-  const void* src[kMaxBatch];
-  C* T[kMaxBatch];
-  const int* pred[kMaxBatch];
+  const void* src[NB];
+  C* T[NB];
+  const int* pred[NB];
 };
-template <class C>
+template <class C, int NB>
 struct ColBatch {
-  const C* T1[kMaxBatch];
-  const C* S[kMaxBatch];
-  C* T2[kMaxBatch];
-  const int* pred[kMaxBatch];
+  const C* T1[NB];
+  const C* S[NB];
+  C* T2[NB];
+  const int* pred[NB];
 };
-template <class C>
+template <class C, int NB>
 struct C2rBatch {
-  const C* T2[kMaxBatch];
-  Rl<C>* out[kMaxBatch];
-  const int* pred[kMaxBatch];
+  const C* T2[NB];
+  Rl<C>* out[NB];
+  const int* pred[NB];
 };
 
 // ---- pass 1: rows r2c.  Group g of the block handles frame row fr; output T[k*ldT + fr], k in [0, P/2].
 // The frame row is a row of the centred, rolled PSF (off = q/2).
 template <class C, class TIN, int R0>
-__global__ __launch_bounds__(kThreads) void k_rows_r2c(R2cBatch<C> bt, int q, int off, int pm, int n_rows, int rb,
+__global__ __launch_bounds__(kThreads) void k_rows_r2c(R2cBatch<C, 1> bt, int q, int off, int pm, int n_rows, int rb,
                                                        int ldT, const C* __restrict__ tw) {
   const int jb = blockIdx.y;
   const int* pred = bt.pred[jb];
@@ -568,8 +569,8 @@ __device__ __forceinline__ int pos_of(int k) {
 }
 
 // ---- pass 1: rows r2c.  Block = RB frame rows; output T[k*ldT + row], k in [0, P/2].
-template <class C, int PG, bool LIN>
-__global__ __launch_bounds__((RowCfg<C, PG, LIN>::T)) void k_conv_r2c(R2cBatch<C> bt, int n_rows, int ldT,
+template <class C, int PG, bool LIN, int NB>
+__global__ __launch_bounds__((RowCfg<C, PG, LIN>::T)) void k_conv_r2c(R2cBatch<C, NB> bt, int n_rows, int ldT,
                                                                       const C* __restrict__ tw) {
   using G = RowCfg<C, PG, LIN>;
   constexpr int LG = PG - 1;
@@ -637,8 +638,9 @@ __global__ __launch_bounds__((RowCfg<C, PG, LIN>::T)) void k_conv_r2c(R2cBatch<C
 }
 
 // ---- pass 2: column convolution: forward FFT, product with the PSF column, inverse FFT.
-template <class C, int PG, bool LIN>
-__global__ __launch_bounds__((ColCfg<C, PG>::T)) void k_conv_cols(ColBatch<C> bt, int n_rows, const C* __restrict__ tw) {
+template <class C, int PG, bool LIN, int NB>
+__global__ __launch_bounds__((ColCfg<C, PG>::T)) void k_conv_cols(ColBatch<C, NB> bt, int n_rows,
+                                                               const C* __restrict__ tw) {
   using G = ColCfg<C, PG>;
   using Pl = Plan<PG>;
   constexpr int P = G::P, NT = G::NT, SP = span(P);
@@ -717,8 +719,8 @@ __global__ __launch_bounds__((ColCfg<C, PG>::T)) void k_conv_cols(ColBatch<C> bt
 }
 
 // ---- pass 3: rows c2r.  Block = RB kept rows; out[r * N + c].
-template <class C, int PG, bool LIN>
-__global__ __launch_bounds__((RowCfg<C, PG, LIN>::T)) void k_conv_c2r(C2rBatch<C> bt, int n_rows, int ldT, Rl<C> scale,
+template <class C, int PG, bool LIN, int NB>
+__global__ __launch_bounds__((RowCfg<C, PG, LIN>::T)) void k_conv_c2r(C2rBatch<C, NB> bt, int n_rows, int ldT, Rl<C> scale,
                                                                       const C* __restrict__ tw) {
   using G = RowCfg<C, PG, LIN>;
   constexpr int LG = PG - 1;
@@ -793,47 +795,53 @@ __global__ __launch_bounds__((RowCfg<C, PG, LIN>::T)) void k_conv_c2r(C2rBatch<C
   });
 }
 
-template <class C, int PG, bool LIN>
-void set_conv_attrs(int lds_max) {
-  (void)hipFuncSetAttribute((const void*)k_conv_r2c<C, PG, LIN>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-  (void)hipFuncSetAttribute((const void*)k_conv_cols<C, PG, LIN>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
-  (void)hipFuncSetAttribute((const void*)k_conv_c2r<C, PG, LIN>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+template <class C, int PG, bool LIN, int NB>
+void set_conv_attrs_nb(int lds_max) {
+  (void)hipFuncSetAttribute((const void*)k_conv_r2c<C, PG, LIN, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+  (void)hipFuncSetAttribute((const void*)k_conv_cols<C, PG, LIN, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+  (void)hipFuncSetAttribute((const void*)k_conv_c2r<C, PG, LIN, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
 }
 
 template <class C, int PG, bool LIN>
-void launch_conv(const R2cBatch<C>& rb, const ColBatch<C>& cb, const C2rBatch<C>& ob, int nb, int n, Rl<C> scale,
-                 const C* tw, hipStream_t st) {
+void set_conv_attrs(int lds_max) {
+  set_conv_attrs_nb<C, PG, LIN, 1>(lds_max);
+  set_conv_attrs_nb<C, PG, LIN, kMaxBatch>(lds_max);
+}
+
+template <class C, int PG, bool LIN, int NB>
+void launch_conv(const R2cBatch<C, NB>& rb, const ColBatch<C, NB>& cb, const C2rBatch<C, NB>& ob, int nb, int n,
+                 Rl<C> scale, const C* tw, hipStream_t st) {
   using R = RowCfg<C, PG, LIN>;
   using G = ColCfg<C, PG>;
-  hipLaunchKernelGGL((k_conv_r2c<C, PG, LIN>), dim3((n + R::RB - 1) / R::RB, nb), dim3(R::T), R::LDS, st, rb, n, n, tw);
+  hipLaunchKernelGGL((k_conv_r2c<C, PG, LIN, NB>), dim3((n + R::RB - 1) / R::RB, nb), dim3(R::T), R::LDS, st, rb, n, n, tw);
   PMS_LAUNCH_CHECK();
-  hipLaunchKernelGGL((k_conv_cols<C, PG, LIN>), dim3((G::P / 2 + 1 + G::CPB - 1) / G::CPB, nb), dim3(G::T), G::LDS, st,
+  hipLaunchKernelGGL((k_conv_cols<C, PG, LIN, NB>), dim3((G::P / 2 + 1 + G::CPB - 1) / G::CPB, nb), dim3(G::T), G::LDS, st,
                      cb, n, tw);
   PMS_LAUNCH_CHECK();
-  hipLaunchKernelGGL((k_conv_c2r<C, PG, LIN>), dim3((n + R::RB - 1) / R::RB, nb), dim3(R::T), R::LDS, st, ob, n, n,
+  hipLaunchKernelGGL((k_conv_c2r<C, PG, LIN, NB>), dim3((n + R::RB - 1) / R::RB, nb), dim3(R::T), R::LDS, st, ob, n, n,
                      scale, tw);
   PMS_LAUNCH_CHECK();
 }
 
-template <class C, bool LIN>
-void dispatch_conv(int pg, const R2cBatch<C>& rb, const ColBatch<C>& cb, const C2rBatch<C>& ob, int nb, int n,
-                   Rl<C> scale, const C* tw, hipStream_t st) {
+template <class C, bool LIN, int NB>
+void dispatch_conv(int pg, const R2cBatch<C, NB>& rb, const ColBatch<C, NB>& cb, const C2rBatch<C, NB>& ob, int nb,
+                   int n, Rl<C> scale, const C* tw, hipStream_t st) {
   switch (pg) {
-    case 2: launch_conv<C, 2, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 3: launch_conv<C, 3, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 4: launch_conv<C, 4, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 5: launch_conv<C, 5, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 6: launch_conv<C, 6, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 7: launch_conv<C, 7, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 8: launch_conv<C, 8, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 9: launch_conv<C, 9, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 10: launch_conv<C, 10, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 11: launch_conv<C, 11, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 12: launch_conv<C, 12, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
-    case 13: launch_conv<C, 13, LIN>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 2: launch_conv<C, 2, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 3: launch_conv<C, 3, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 4: launch_conv<C, 4, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 5: launch_conv<C, 5, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 6: launch_conv<C, 6, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 7: launch_conv<C, 7, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 8: launch_conv<C, 8, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 9: launch_conv<C, 9, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 10: launch_conv<C, 10, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 11: launch_conv<C, 11, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 12: launch_conv<C, 12, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
+    case 13: launch_conv<C, 13, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st); break;
     case 14:
       if constexpr (sizeof(Rl<C>) == 4) {  // one LDS transform holds a column: 8192 in float64
-        launch_conv<C, 14, LIN>(rb, cb, ob, nb, n, scale, tw, st);
+        launch_conv<C, 14, LIN, NB>(rb, cb, ob, nb, n, scale, tw, st);
         break;
       }
       [[fallthrough]];
@@ -949,7 +957,7 @@ template <class C, class TIN>
 void pow2_psf_spectrum(const TIN* psf, int q, int p, C* spec, C* work, const C* tw, hipStream_t st) {
   const int pm = ilog2(p);
   const int L = p / 2;
-  R2cBatch<C> rb{};
+  R2cBatch<C, 1> rb{};
   rb.src[0] = psf;
   rb.T[0] = work;
   const int rpb = rows_per_block<C>(L, p);
@@ -968,39 +976,47 @@ void pow2_psf_spectrum(const TIN* psf, int q, int p, C* spec, C* work, const C* 
   PMS_LAUNCH_CHECK();
 }
 
-// Jobs are independent: job j's blocks read and write only job j's buffers, so a batch gives each
-// job exactly the result of its own single-job call.
-template <class C, class JOB>
-void pow2_conv_batch(const JOB* jobs, int count, int n, int p, const C* tw, hipStream_t st) {
-  PMS_REQUIRE(p == n || p == 2 * n, "fft_conv: frame must be N (circular) or 2N (linear)");
+// nb <= NB jobs in one launch per pass.  Jobs are independent: job j's blocks read and write only job j's
+// buffers, so a batch gives each job exactly the result of its own single-job call.
+template <class C, int NB, class JOB>
+void pow2_conv_jobs(const JOB* jobs, int nb, int n, int p, const C* tw, hipStream_t st) {
   const int pm = ilog2(p);
   const int L = p / 2;
   const Rl<C> scale = (Rl<C>)1 / ((Rl<C>)p * (Rl<C>)p);
+  R2cBatch<C, NB> rb{};
+  ColBatch<C, NB> cb{};
+  C2rBatch<C, NB> ob{};
+  for (int k = 0; k < nb; ++k) {
+    const JOB& j = jobs[k];
+    PMS_REQUIRE(j.in && j.spec && j.out && j.work, "fft_conv: NULL buffer");
+    C* T1 = reinterpret_cast<C*>(j.work);
+    C* T2 = T1 + (size_t)(L + 1) * n;
+    rb.src[k] = j.in;
+    rb.T[k] = T1;
+    rb.pred[k] = j.pred;
+    cb.T1[k] = T1;
+    cb.S[k] = reinterpret_cast<const C*>(j.spec);
+    cb.T2[k] = T2;
+    cb.pred[k] = j.pred;
+    ob.T2[k] = T2;
+    ob.out[k] = j.out;
+    ob.pred[k] = j.pred;
+  }
+  if (p == 2 * n)
+    dispatch_conv<C, true, NB>(pm, rb, cb, ob, nb, n, scale, tw, st);
+  else
+    dispatch_conv<C, false, NB>(pm, rb, cb, ob, nb, n, scale, tw, st);
+}
+
+template <class C, class JOB>
+void pow2_conv_batch(const JOB* jobs, int count, int n, int p, const C* tw, hipStream_t st) {
+  PMS_REQUIRE(p == n || p == 2 * n, "fft_conv: frame must be N (circular) or 2N (linear)");
   for (int j0 = 0; j0 < count; j0 += kMaxBatch) {
     const int nb = std::min(kMaxBatch, count - j0);
-    R2cBatch<C> rb{};
-    ColBatch<C> cb{};
-    C2rBatch<C> ob{};
-    for (int k = 0; k < nb; ++k) {
-      const JOB& j = jobs[j0 + k];
-      PMS_REQUIRE(j.in && j.spec && j.out && j.work, "fft_conv: NULL buffer");
-      C* T1 = reinterpret_cast<C*>(j.work);
-      C* T2 = T1 + (size_t)(L + 1) * n;
-      rb.src[k] = j.in;
-      rb.T[k] = T1;
-      rb.pred[k] = j.pred;
-      cb.T1[k] = T1;
-      cb.S[k] = reinterpret_cast<const C*>(j.spec);
-      cb.T2[k] = T2;
-      cb.pred[k] = j.pred;
-      ob.T2[k] = T2;
-      ob.out[k] = j.out;
-      ob.pred[k] = j.pred;
-    }
-    if (p == 2 * n)
-      dispatch_conv<C, true>(pm, rb, cb, ob, nb, n, scale, tw, st);
+    if (nb == 1)
+      pow2_conv_jobs<C, 1>(jobs + j0, nb, n, p, tw, st);
     else
-      dispatch_conv<C, false>(pm, rb, cb, ob, nb, n, scale, tw, st);
+      pow2_conv_jobs<C, kMaxBatch>(jobs + j0, nb, n, p, tw, st);
   }
 }
 

@@ -65,14 +65,19 @@ struct ScaleJob {
 
 // One launch serves up to kMaxBatch jobs of the same shape and scale (grid y, or z for the
 // small-plane kernel, selects the job).
-struct ScaleParams {
-  ScaleJob job[kMaxBatch];
+struct ScaleDims {
   int h, w;               // plane shape (row-major, contiguous)
   int d;                  // dilation 2^s
   int q_log2, tj;         // comb: Q = 1<<q_log2 phases x TJ teeth (Q*TJ <= 256)
   int k_rows;             // output rows (in phase units) per workgroup walk
   int n_cg, n_tb, n_seg;  // grid decomposition
 };
+template <int NB>
+struct ScaleParamsN : ScaleDims {
+  using Dims = ScaleDims;
+  ScaleJob job[NB];
+};
+using ScaleParams = ScaleParamsN<kMaxBatch>;
 
 template <int MODE>
 struct ModeTraits;
@@ -95,8 +100,9 @@ struct ModeTraits<IUWT_RECOMP> {
 // Every load is issued before the first is used (at most 4 waves per SIMD, so the compiler may keep
 // all 81 values in registers instead of waiting row by row to save registers for occupancy that
 // these small grids never reach).
-template <int MODE>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 4))) void k_iuwt_small(ScaleParams sp) {
+template <int MODE, int NB>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 4))) void k_iuwt_small(
+    ScaleParamsN<NB> sp) {
   const ScaleJob a = sp.job[blockIdx.z];
   constexpr int H = ModeTraits<MODE>::H;
   constexpr int T = 2 * H + 1;
@@ -1214,12 +1220,20 @@ void dec2_batch(const Dec2Job* jobs, int count, int h, int w, int s, const Plan&
 // forms at the folded position.  Every plane is therefore bit-identical to two k_iuwt_small launches.
 constexpr int kTile2 = 16;  // tile side in lattice steps (one output pixel per thread)
 
-template <class J>
-struct Small2Params {
-  J job[kMaxBatch];  // Dec2Job or PairJob
+struct Small2Dims {
   int h, w, d;
-  int ntr, ntc;      // tiles per phase along rows and columns
+  int ntr, ntc;  // tiles per phase along rows and columns
 };
+template <class J>
+struct Small2 {
+  template <int NB>
+  struct Params : Small2Dims {
+    using Dims = Small2Dims;
+    J job[NB];  // Dec2Job or PairJob
+  };
+};
+template <class J>
+using Small2Params = typename Small2<J>::template Params<kMaxBatch>;
 
 // Folded plane index of lattice coordinates origin + step*(first + k), k in [0, n), for k = lane;
 // the index is stored with its mirror flag as ~index when the position lies on a mirrored period.
@@ -1276,8 +1290,8 @@ __device__ __forceinline__ float tap9(const float* v, int step) {
 // applied separably, row sums first (the one-scale kernel's order): pass 1 forms the 5-tap row sums
 // of C_s at every C_{s+1} column and the 9-tap row sums at the tile's columns, pass 2 the column sums
 // (C_{s+1} and w_s), pass 3 the row sums of C_{s+1} at spacing 2, pass 4 w_{s+1} and C_{s+2}.
-template <bool MASK, bool OUTC>
-__global__ __launch_bounds__(kThreads) void k_iuwt_small2_dec(Small2Params<Dec2Job> sp) {
+template <bool MASK, bool OUTC, int NB>
+__global__ __launch_bounds__(kThreads) void k_iuwt_small2_dec(Small2<Dec2Job>::Params<NB> sp) {
   constexpr int RS = kTile2 + 20, RP = RS + 1;  // staged C_s: lattice -10 .. 25 (rows padded)
   constexpr int IS = kTile2 + 16, IP = IS + 1;  // C_{s+1}: lattice -8 .. 23
   constexpr int N5 = RS * IS;                   // pass 1: 5-tap row sums, every staged row
@@ -1354,8 +1368,8 @@ __global__ __launch_bounds__(kThreads) void k_iuwt_small2_dec(Small2Params<Dec2J
 // Scales s+1 then s of a recomposition: R_s = h_s T + w_s with T = h_{s+1} R + w_{s+1}.  Pass 1 forms
 // the row sums of R at spacing 2 at every T column, pass 2 T, pass 3 the row sums of T at the tile's
 // columns, pass 4 R_s.
-template <bool MASK>
-__global__ __launch_bounds__(kThreads) void k_iuwt_small2_rec(Small2Params<PairJob> sp) {
+template <bool MASK, int NB>
+__global__ __launch_bounds__(kThreads) void k_iuwt_small2_rec(Small2<PairJob>::Params<NB> sp) {
   constexpr int RS = kTile2 + 12, RP = RS + 1;  // staged R: lattice -6 .. 21
   constexpr int TS = kTile2 + 4, TP = TS + 1;   // T: lattice -2 .. 17
   constexpr int N1 = RS * TS;                   // pass 1 sums
@@ -1431,8 +1445,7 @@ Small2Params<J> small2_params(int h, int w, int s) {
   return sp;
 }
 
-template <class J>
-dim3 small2_grid(const Small2Params<J>& sp, int nb) { return dim3(sp.d * sp.ntc, sp.d * sp.ntr, nb); }
+dim3 small2_grid(const Small2Dims& sp, int nb) { return dim3(sp.d * sp.ntc, sp.d * sp.ntr, nb); }
 
 // jobs[0..count) share shape and scale pair; masked and unmasked jobs, and jobs that keep C_{s+2}
 // and those that do not, go to separate launches
@@ -1444,12 +1457,15 @@ void small2_dec_batch(const Dec2Job* jobs, int count, int h, int w, int s, hipSt
     auto flush = [&]() {
       if (nb == 0) return;
       const dim3 g = small2_grid(sp, nb);
-      switch (kind) {
-        case 0: hipLaunchKernelGGL((k_iuwt_small2_dec<false, false>), g, dim3(kThreads), 0, st, sp); break;
-        case 1: hipLaunchKernelGGL((k_iuwt_small2_dec<true, false>), g, dim3(kThreads), 0, st, sp); break;
-        case 2: hipLaunchKernelGGL((k_iuwt_small2_dec<false, true>), g, dim3(kThreads), 0, st, sp); break;
-        default: hipLaunchKernelGGL((k_iuwt_small2_dec<true, true>), g, dim3(kThreads), 0, st, sp); break;
-      }
+      with_jobs<Small2<Dec2Job>::Params>(sp, nb, [&](const auto& p) {
+        constexpr int NB = sizeof(p.job) / sizeof(p.job[0]);
+        switch (kind) {
+          case 0: hipLaunchKernelGGL((k_iuwt_small2_dec<false, false, NB>), g, dim3(kThreads), 0, st, p); break;
+          case 1: hipLaunchKernelGGL((k_iuwt_small2_dec<true, false, NB>), g, dim3(kThreads), 0, st, p); break;
+          case 2: hipLaunchKernelGGL((k_iuwt_small2_dec<false, true, NB>), g, dim3(kThreads), 0, st, p); break;
+          default: hipLaunchKernelGGL((k_iuwt_small2_dec<true, true, NB>), g, dim3(kThreads), 0, st, p); break;
+        }
+      });
       PMS_LAUNCH_CHECK();
       nb = 0;
     };
@@ -1471,10 +1487,13 @@ void small2_rec_batch(const PairJob* jobs, int count, int h, int w, int s, hipSt
     auto flush = [&]() {
       if (nb == 0) return;
       const dim3 g = small2_grid(sp, nb);
-      if (masked)
-        hipLaunchKernelGGL(k_iuwt_small2_rec<true>, g, dim3(kThreads), 0, st, sp);
-      else
-        hipLaunchKernelGGL(k_iuwt_small2_rec<false>, g, dim3(kThreads), 0, st, sp);
+      with_jobs<Small2<PairJob>::Params>(sp, nb, [&](const auto& p) {
+        constexpr int NB = sizeof(p.job) / sizeof(p.job[0]);
+        if (masked)
+          hipLaunchKernelGGL((k_iuwt_small2_rec<true, NB>), g, dim3(kThreads), 0, st, p);
+        else
+          hipLaunchKernelGGL((k_iuwt_small2_rec<false, NB>), g, dim3(kThreads), 0, st, p);
+      });
       PMS_LAUNCH_CHECK();
       nb = 0;
     };
@@ -1598,12 +1617,15 @@ int iuwt_scale_batch(const IuwtScaleCall* calls, int count, hipStream_t st, bool
     for (int k = 0; k < nb; ++k) sp.job[k] = scale_job(calls[j0 + k]);
     const dim3 g2 = small_grid(c0.h, c0.w);
     const dim3 grid(g2.x, g2.y, nb);
-    if (c0.mode == IUWT_DECOMP)
-      hipLaunchKernelGGL(k_iuwt_small<IUWT_DECOMP>, grid, dim3(kThreads), 0, st, sp);
-    else if (c0.mode == IUWT_SMOOTH)
-      hipLaunchKernelGGL(k_iuwt_small<IUWT_SMOOTH>, grid, dim3(kThreads), 0, st, sp);
-    else
-      hipLaunchKernelGGL(k_iuwt_small<IUWT_RECOMP>, grid, dim3(kThreads), 0, st, sp);
+    with_jobs<ScaleParamsN>(sp, nb, [&](const auto& p) {
+      constexpr int NB = sizeof(p.job) / sizeof(p.job[0]);
+      if (c0.mode == IUWT_DECOMP)
+        hipLaunchKernelGGL((k_iuwt_small<IUWT_DECOMP, NB>), grid, dim3(kThreads), 0, st, p);
+      else if (c0.mode == IUWT_SMOOTH)
+        hipLaunchKernelGGL((k_iuwt_small<IUWT_SMOOTH, NB>), grid, dim3(kThreads), 0, st, p);
+      else
+        hipLaunchKernelGGL((k_iuwt_small<IUWT_RECOMP, NB>), grid, dim3(kThreads), 0, st, p);
+    });
     PMS_LAUNCH_CHECK();
     blocks = (int)(g2.x * g2.y);
   }

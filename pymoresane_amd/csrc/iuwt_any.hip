@@ -40,10 +40,16 @@ struct GenJob {
   const int* pred;
 };
 
-template <class T>
-struct GenParams {
-  GenJob<T> job[kMaxBatch];
+struct GenDims {
   int h, w, d;
+};
+template <class T>
+struct Gen {
+  template <int NB>
+  struct Params : GenDims {
+    using Dims = GenDims;
+    GenJob<T> job[NB];
+  };
 };
 
 // input index of the tap at offset off for output i on an axis of length n
@@ -52,8 +58,8 @@ __device__ __forceinline__ int tap_idx(int i, int off, int n) {
   return fold_idx(i + off, n);
 }
 
-template <class T, int MODE>
-__global__ __launch_bounds__(kGenThreads) void k_iuwt_gen(GenParams<T> sp) {
+template <class T, int MODE, int NB>
+__global__ __launch_bounds__(kGenThreads) void k_iuwt_gen(typename Gen<T>::template Params<NB> sp) {
   const GenJob<T> a = sp.job[blockIdx.z];
   if (a.pred && *a.pred == 0) return;
   const int w = sp.w, h = sp.h, d = sp.d;
@@ -117,13 +123,16 @@ template <class T, int MODE>
 void launch_gen(std::vector<GenJob<T>>& jobs, int h, int w, int d, hipStream_t st) {
   for (size_t j0 = 0; j0 < jobs.size(); j0 += kMaxBatch) {
     const int nb = (int)std::min(jobs.size() - j0, (size_t)kMaxBatch);
-    GenParams<T> sp{};
+    typename Gen<T>::template Params<kMaxBatch> sp{};
     for (int k = 0; k < nb; ++k) sp.job[k] = jobs[j0 + k];
     sp.h = h;
     sp.w = w;
     sp.d = d;
     const dim3 g2 = gen_grid(h, w);
-    hipLaunchKernelGGL((k_iuwt_gen<T, MODE>), dim3(g2.x, g2.y, nb), dim3(kGenThreads), 0, st, sp);
+    with_jobs<Gen<T>::template Params>(sp, nb, [&](const auto& p) {
+      constexpr int NB = sizeof(p.job) / sizeof(p.job[0]);
+      hipLaunchKernelGGL((k_iuwt_gen<T, MODE, NB>), dim3(g2.x, g2.y, nb), dim3(kGenThreads), 0, st, p);
+    });
     PMS_LAUNCH_CHECK();
   }
 }
