@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "iuwt_small2.h"
 #include "pms_internal.h"
 
 namespace pms {
@@ -194,12 +195,13 @@ int iuwt_gen_scale_batch(const IuwtScaleCallT<T>* calls, int count, hipStream_t 
 template int iuwt_gen_scale_batch<float>(const IuwtScaleCallT<float>*, int, hipStream_t);
 template int iuwt_gen_scale_batch<double>(const IuwtScaleCallT<double>*, int, hipStream_t);
 
-// float64 decomposition: scale by scale over all jobs (pre-smoothing below scale_adjust, then
-// decomposition), ping-ponging C through the job's two work planes.
+// float64 decomposition over all jobs: pre-smoothing below scale_adjust, then pairs of scales in one launch each where
+// both are within the side and no reference is reduced, the rest scale by scale; C ping-pongs
+// through the job's two work planes.
 void iuwt_decompose_batch(IuwtDecompJobT<double>* jobs, int count, int h, int w, hipStream_t st) {
   const size_t plane = (size_t)h * w;
   std::vector<const double*> cur(count);
-  std::vector<int> slot(count, 0);
+  std::vector<int> slot(count, 0), done(count, 0);  // scales below done are decomposed
   int smax = 0;
   for (int k = 0; k < count; ++k) {
     IuwtDecompJobT<double>& j = jobs[k];
@@ -210,11 +212,14 @@ void iuwt_decompose_batch(IuwtDecompJobT<double>* jobs, int count, int h, int w,
     smax = std::max(smax, j.scale_count);
   }
   std::vector<IuwtScaleCallT<double>> calls;
-  std::vector<int> who;
+  std::vector<int> who, pwho;
+  std::vector<Dec2JobT<double>> pairs;
   for (int s = 0; s < smax; ++s) {
     for (int mode : {IUWT_SMOOTH, IUWT_DECOMP}) {
       calls.clear();
       who.clear();
+      pairs.clear();
+      pwho.clear();
       for (int k = 0; k < count; ++k) {
         const IuwtDecompJobT<double>& j = jobs[k];
         double* ping = j.work + (size_t)slot[k] * plane;
@@ -229,8 +234,21 @@ void iuwt_decompose_batch(IuwtDecompJobT<double>* jobs, int count, int h, int w,
           if (s >= j.scale_adjust) continue;
           c.out_c = ping;
         } else {
-          if (s < j.scale_adjust || s >= j.scale_count) continue;
+          if (s < j.scale_adjust || s >= j.scale_count || s < done[k]) continue;
           const int kk = s - j.scale_adjust;
+          if (s + 1 < j.scale_count && j.detail && !j.ref && !iuwt_over_long(h, w, s + 1)) {
+            Dec2JobT<double> pj{};
+            pj.in = cur[k];
+            pj.out_c = s + 1 == j.scale_count - 1 ? j.smoothed : ping;
+            pj.out_w0 = j.detail + (size_t)kk * plane;
+            pj.out_w1 = pj.out_w0 + plane;
+            pj.mask0 = j.mask ? j.mask + (size_t)kk * plane : nullptr;
+            pj.mask1 = j.mask ? pj.mask0 + plane : nullptr;
+            pj.pred = j.pred;
+            pairs.push_back(pj);
+            pwho.push_back(k);
+            continue;
+          }
           const bool last = s == j.scale_count - 1;
           c.out_c = (last && j.smoothed) ? j.smoothed : ping;
           c.out_w = j.detail ? j.detail + (size_t)kk * plane : nullptr;
@@ -240,6 +258,16 @@ void iuwt_decompose_batch(IuwtDecompJobT<double>* jobs, int count, int h, int w,
         }
         calls.push_back(c);
         who.push_back(k);
+      }
+      if (!pairs.empty()) {
+        small2_dec_batch<double>(pairs.data(), (int)pairs.size(), h, w, s, st);
+        for (size_t i = 0; i < pwho.size(); ++i) {
+          const int k = pwho[i];
+          done[k] = s + 2;
+          if (s + 1 == jobs[k].scale_count - 1) continue;
+          cur[k] = pairs[i].out_c;
+          slot[k] ^= 1;
+        }
       }
       if (calls.empty()) continue;
       const int nb = iuwt_gen_scale_batch<double>(calls.data(), (int)calls.size(), st);
@@ -258,16 +286,22 @@ long iuwt_decompose_partials_f64(int h, int w, int scale_count, int scale_adjust
   return (long)(scale_count - scale_adjust) * iuwt_gen_blocks(h, w);
 }
 
-// float64 recomposition from the coarsest kept scale down (one launch per scale and job group)
+// float64 recomposition from the coarsest kept scale down: pairs of detail scales in one launch each
+// (from the finest up, so that an odd scale is left at the top) where both are within the side, one launch per
+// scale otherwise; jobs at the same step share launches.
 void iuwt_recompose_batch(const IuwtRecompJobT<double>* jobs, int count, int h, int w, hipStream_t st) {
   const size_t plane = (size_t)h * w;
+  enum { OP_RECOMP, OP_SMOOTH, OP_PAIR };
+  struct Op {
+    int kind, s;  // OP_PAIR covers scales s+1 then s
+  };
   struct State {
     const double* cur;
     int slot;
-    int s;  // next scale to apply (counts down to -1)
+    std::vector<Op> ops;
   };
   std::vector<State> state(count);
-  int smax = -1;
+  size_t rounds = 0;
   for (int k = 0; k < count; ++k) {
     const IuwtRecompJobT<double>& j = jobs[k];
     PMS_REQUIRE(j.nplanes >= 1 && j.scale_adjust >= 0, "recomposition needs at least one detail plane");
@@ -276,59 +310,73 @@ void iuwt_recompose_batch(const IuwtRecompJobT<double>* jobs, int count, int h, 
     State& sk = state[k];
     sk.cur = j.smoothed;
     sk.slot = 0;
-    sk.s = top - 1;
+    int s = top - 1;
     if (!j.smoothed) {
       // R starts at zero: the coarsest step is the (masked) detail plane itself
       const size_t off = (size_t)(top - 1 - j.scale_adjust) * plane;
-      double* dst = j.work;
-      if (top - 1 == 0) dst = j.out;  // one plane, no smoothing left
-      gen_masked_copy<double>(j.detail + off, j.mask ? j.mask + off : nullptr, dst, plane, j.pred, st);
-      sk.cur = dst;
-      sk.slot = 1;
-      sk.s = top - 2;
+      sk.cur = j.detail + off;
+      if (j.mask || top == 1) {  // a masked plane, or the result itself: one plane, no smoothing left
+        double* dst = top == 1 ? j.out : j.work;
+        gen_masked_copy<double>(j.detail + off, j.mask ? j.mask + off : nullptr, dst, plane, j.pred, st);
+        sk.cur = dst;
+        sk.slot = 1;
+      }
+      --s;
     }
-    smax = std::max(smax, sk.s);
+    bool odd_top = s >= j.scale_adjust && (s - j.scale_adjust + 1) % 2 == 1;
+    while (s >= 0) {
+      const bool pair = !odd_top && s - 1 >= j.scale_adjust && !iuwt_over_long(h, w, s);
+      odd_top = false;
+      sk.ops.push_back(pair ? Op{OP_PAIR, s - 1} : Op{s >= j.scale_adjust ? OP_RECOMP : OP_SMOOTH, s});
+      s -= pair ? 2 : 1;
+    }
+    rounds = std::max(rounds, sk.ops.size());
   }
   std::vector<IuwtScaleCallT<double>> calls;
-  std::vector<int> who;
-  for (int s = smax; s >= 0; --s) {
-    for (int mode : {IUWT_RECOMP, IUWT_SMOOTH}) {
+  std::vector<PairJobT<double>> pairs;
+  std::vector<char> issued(count);
+  for (size_t r = 0; r < rounds; ++r) {
+    std::fill(issued.begin(), issued.end(), 0);
+    for (int k0 = 0; k0 < count; ++k0) {
+      if (issued[k0] || r >= state[k0].ops.size()) continue;
+      const Op op = state[k0].ops[r];
       calls.clear();
-      who.clear();
-      for (int k = 0; k < count; ++k) {
-        const IuwtRecompJobT<double>& j = jobs[k];
+      pairs.clear();
+      for (int k = k0; k < count; ++k) {
         State& sk = state[k];
-        if (sk.s != s) continue;
-        const bool detail = s >= j.scale_adjust;
-        if ((mode == IUWT_RECOMP) != detail) continue;
-        IuwtScaleCallT<double> c{};
-        c.mode = mode;
-        c.in = sk.cur;
-        c.out_c = s == 0 ? j.out : j.work + (size_t)sk.slot * plane;
-        if (detail) {
-          const size_t off = (size_t)(s - j.scale_adjust) * plane;
-          c.w_in = j.detail + off;
-          c.mask = j.mask ? j.mask + off : nullptr;
+        if (issued[k] || r >= sk.ops.size() || sk.ops[r].kind != op.kind || sk.ops[r].s != op.s) continue;
+        const IuwtRecompJobT<double>& j = jobs[k];
+        double* out = r + 1 == sk.ops.size() ? j.out : j.work + (size_t)sk.slot * plane;
+        const size_t off = op.s >= j.scale_adjust ? (size_t)(op.s - j.scale_adjust) * plane : 0;
+        if (op.kind == OP_PAIR) {
+          pairs.push_back(PairJobT<double>{sk.cur, out, j.detail + off, j.detail + off + plane,
+                                           j.mask ? j.mask + off : nullptr, j.mask ? j.mask + off + plane : nullptr,
+                                           j.pred});
+        } else {
+          IuwtScaleCallT<double> c{};
+          c.mode = op.kind == OP_RECOMP ? IUWT_RECOMP : IUWT_SMOOTH;
+          c.in = sk.cur;
+          c.out_c = out;
+          if (op.kind == OP_RECOMP) {
+            c.w_in = j.detail + off;
+            c.mask = j.mask ? j.mask + off : nullptr;
+          }
+          c.h = h;
+          c.w = w;
+          c.scale = op.s;
+          c.pred = j.pred;
+          calls.push_back(c);
         }
-        c.h = h;
-        c.w = w;
-        c.scale = s;
-        c.pred = j.pred;
-        calls.push_back(c);
-        who.push_back(k);
-      }
-      if (calls.empty()) continue;
-      iuwt_gen_scale_batch<double>(calls.data(), (int)calls.size(), st);
-      for (size_t i = 0; i < who.size(); ++i) {
-        State& sk = state[who[i]];
-        sk.cur = calls[i].out_c;
+        issued[k] = 1;
+        sk.cur = out;
         sk.slot ^= 1;
-        sk.s -= 1;
       }
+      if (op.kind == OP_PAIR)
+        small2_rec_batch<double>(pairs.data(), (int)pairs.size(), h, w, op.s, st);
+      else
+        iuwt_gen_scale_batch<double>(calls.data(), (int)calls.size(), st);
     }
   }
-  // a job whose only plane was scale 0 with a smoothed base still needs its steps: covered above;
-  // a job with a smoothed base and nothing to apply cannot occur (nplanes >= 1)
 }
 
 }  // namespace pms
