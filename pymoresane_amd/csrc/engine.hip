@@ -475,16 +475,40 @@ void DeviceArena::release() {
   for (void* p : ptrs_) (void)hipFree(p);
   ptrs_.clear();
   bytes_ = 0;
+  planning_ = false;
+  planned_ = 0;
+  slab_ = nullptr;
+  slab_left_ = 0;
+}
+
+void* DeviceArena::allocate(size_t bytes) {
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e != hipSuccess) fail(PMS_ERR_ALLOC, "device allocation of " + std::to_string(bytes) + " bytes failed");
+  ptrs_.push_back(p);
+  bytes_ += bytes;
+  return p;
+}
+
+void DeviceArena::commit() {
+  planning_ = false;
+  slab_left_ = planned_;
+  planned_ = 0;
+  if (slab_left_) slab_ = (unsigned char*)allocate(slab_left_);
 }
 
 void* DeviceArena::alloc(size_t bytes) {
-  void* p = nullptr;
   const size_t b = ((bytes + 255) / 256) * 256;
   if (b == 0) return nullptr;
-  hipError_t e = hipMalloc(&p, b);
-  if (e != hipSuccess) fail(PMS_ERR_ALLOC, "device allocation of " + std::to_string(b) + " bytes failed");
-  ptrs_.push_back(p);
-  bytes_ += b;
+  if (planning_) {
+    planned_ += b;
+    return nullptr;
+  }
+  if (!slab_) return allocate(b);
+  PMS_REQUIRE(b <= slab_left_, "device buffer beyond its arena's plan");
+  void* p = slab_;
+  slab_ += b;
+  slab_left_ -= b;
   return p;
 }
 
@@ -653,17 +677,24 @@ bool Job::ensure(const Geometry& g, hipStream_t st) {
   if (have_ && fits(need, cap_)) return false;
   const JobSizes z = (have_ && cap_.f64 == need.f64) ? max_sizes(need, cap_) : need;
   arena_.release();
-  cap_ = z;
+  have_ = false;  // until every buffer is there: an allocation below may fail
   f = Planes<float>{};
   d = Planes<double>{};
-  if (g.f64)
-    carve(d, z, arena_);
-  else
-    carve(f, z, arena_);
-  M = (uint8_t*)arena_.alloc(z.mask);
-  mad_work = arena_.alloc(z.mad);
-  ext_work = arena_.alloc(z.ext);
-  partial = (double*)arena_.alloc(z.partial);
+  const auto cut = [&] {
+    if (g.f64)
+      carve(d, z, arena_);
+    else
+      carve(f, z, arena_);
+    M = (uint8_t*)arena_.alloc(z.mask);
+    mad_work = arena_.alloc(z.mad);
+    ext_work = arena_.alloc(z.ext);
+    partial = (double*)arena_.alloc(z.partial);
+  };
+  arena_.plan();
+  cut();
+  arena_.commit();
+  cut();
+  cap_ = z;
   have_ = true;
   // the by-scale copy lives in its own arena and survives a regrowth of the others
   f.cur_dirty = (float*)by_scale_ptr_;
