@@ -30,8 +30,9 @@
 // spacing 2 in the finer scale's frame), with results bit-identical to one
 // launch per scale.  Planes of at most 256^2 pixels, and planes of at most
 // 512^2 in launches of few of them, use direct-stencil kernels instead of the
-// walks, and pairs of scales there run as one launch (k_iuwt_small2_dec /
-// k_iuwt_small2_rec); every family gives the same bits.  An autotuner (end of this file) picks the
+// walks, and pairs of scales there run as one launch (iuwt_small2.h, and
+// iuwt_tile2.h where tiles fill the chip, which also takes the finer pairs of planes
+// up to some 3500^2); every family gives the same bits.  An autotuner (end of this file) picks the
 // walks' workgroup count and the recomposition pairing per call signature.
 #include <algorithm>
 #include <cmath>
@@ -41,7 +42,7 @@
 #include <string>
 #include <vector>
 
-#include "iuwt_small2.h"
+#include "iuwt_tile2.h"
 #include "pms_internal.h"
 
 namespace pms {
@@ -1227,6 +1228,19 @@ bool small2_applies(bool small, int h, int w, int s) {
   return small && !iuwt_over_long(h, w, s + 1) && env_int("PMS_IUWT_SMALL2", 1) != 0;
 }
 
+// Whether scales (s, s+1) of a plane above that range still run as one tile launch (iuwt_tile2.h; the same
+// planes again).  The tiles read and write every 2^s-th element, the walks whole runs, so the line lies at
+// fewer pixels (of the whole launch) for coarser pairs.  Measured, decomposition (recomposition) of one plane in us, walks
+// against tiles, each row with the finer pairs on tiles: pair (0,1): 1024^2 54 -> 46 (41 -> 39), 2048^2 112 -> 103 (79 -> 75),
+// 3000^2 180 -> 170 (147 -> 141), 4096^2 282 -> 285 (236 -> 237); pair (2,3): 1024^2 46 -> 38 (39 -> 33), 1600^2 76 -> 66
+// (53 -> 53), 2048^2 103 -> 98 (75 -> 76), 3000^2 170 -> 180 (141 -> 160); pair (4,5): 800^2 34 -> 43 (32 -> 30.5), 1024^2 38 -> 46
+// (33 -> 31), 1300^2 56 -> 77 (41 -> 51).
+bool tile2_range(int h, int w, int s, int jobs, bool recomp) {
+  const long px = (long)h * w * jobs;
+  const int top = px <= 1L << 20 ? (recomp ? 4 : 2) : px <= 1L << 22 ? 2 : px <= 3L << 22 ? 0 : -1;
+  return s <= top;
+}
+
 dim3 small_grid(int h, int w) { return dim3(ceil_div(w, 64), ceil_div(h, 4)); }
 
 static ScaleJob scale_job(const IuwtScaleCall& c) {
@@ -1373,7 +1387,7 @@ static void decompose_batch_impl(IuwtDecompJob* jobs, int count, int h, int w, b
       pairs.clear();
       pwho.clear();
       Plan pl;
-      const bool small_pair = mode == IUWT_DECOMP && small2_applies(small, h, w, s);
+      const bool small_pair = mode == IUWT_DECOMP && small2_applies(small || tile2_range(h, w, s, count, false), h, w, s);
       const bool pair_plan = small_pair || (!small && fuse == 1 && mode == IUWT_DECOMP && dec2_plan(h, w, s, &pl));
       for (int k = 0; k < count; ++k) {
         const IuwtDecompJob& j = jobs[k];
@@ -1417,7 +1431,7 @@ static void decompose_batch_impl(IuwtDecompJob* jobs, int count, int h, int w, b
       }
       if (!pairs.empty()) {
         if (small_pair)
-          small2_dec_batch<float>(pairs.data(), (int)pairs.size(), h, w, s, st);
+          pair_dec_batch<float>(pairs.data(), (int)pairs.size(), h, w, s, st);
         else
           dec2_batch(pairs.data(), (int)pairs.size(), h, w, s, pl, st);
         for (int k : pwho) {
@@ -1512,7 +1526,7 @@ static void recompose_batch_impl(const IuwtRecompJob* jobs, int count, int h, in
         --s;
         continue;
       }
-      if (pair && s - 1 >= j.scale_adjust && (small2_applies(small, h, w, s - 1) || (!small && recomp2_plan(h, w, s - 1, &pl)))) {
+      if (pair && s - 1 >= j.scale_adjust && (small2_applies(small || tile2_range(h, w, s - 1, count, true), h, w, s - 1) || (!small && recomp2_plan(h, w, s - 1, &pl)))) {
         sk.ops.push_back({OP_PAIR, s - 1});
         s -= 2;
       } else {
@@ -1573,8 +1587,8 @@ static void recompose_batch_impl(const IuwtRecompJob* jobs, int count, int h, in
       }
       if (op0.kind == OP_PAIR) {
         Plan pl;
-        if (small2_applies(small, h, w, op0.s)) {
-          small2_rec_batch<float>(pairs.data(), (int)pairs.size(), h, w, op0.s, st);
+        if (small2_applies(small || tile2_range(h, w, op0.s, count, true), h, w, op0.s)) {
+          pair_rec_batch<float>(pairs.data(), (int)pairs.size(), h, w, op0.s, st);
         } else {
           PMS_REQUIRE(recomp2_plan(h, w, op0.s, &pl), "two-scale recomposition plan changed");
           recomp2_batch(pairs.data(), (int)pairs.size(), h, w, op0.s, pl, st);
