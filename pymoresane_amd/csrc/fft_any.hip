@@ -12,17 +12,20 @@
 // Each transform of length L runs in LDS as in-place decimation-in-frequency stages (forward,
 // output in mixed-radix digit-reversed order) or their exact mirror (inverse, decimation in time,
 // digit-reversed in, natural order out), so the column pass needs no reordering: the PSF
-// spectrum is stored in the order in which the column pass multiplies by it.  The radices (2 to 16)
-// are chosen on the host per length, the stages are compiled per radix.  Stage twiddles, split factors
+// spectrum is stored in the order in which the column pass multiplies by it.  The stages (radix 2 to 13)
+// follow from the length; the host groups them into steps of one or two, which are compiled.  Stage twiddles, split factors
 // and the row transforms' digit reversal come from tables per frame side and type, computed on the host in float64.
 //
-// What bounds the passes is the chain of each block: its loads, one LDS exchange and barrier per stage, its
-// stores.  So stages are few (radices to 16), the first and last ones work on global memory, twiddles and
-// the PSF column are requested ahead of the barriers, nothing divides by a run-time number, and the
-// blocks are small enough for 16 waves a CU.  Convolution of a 1000^2 image on a frame of 2000: rows r2c 10 us, columns
-// 18 us, rows c2r 9 us (27 + 37 + 27 us with stages up to radix 8, a division per butterfly, run-time digit
-// reversal and two rows a block); frames of 132 / 800 / 3000 / 6000: 39 / 50 / 180 / 718 -> 16 / 21 / 68 / 232 us.
-// Error against 64 bits 3.0e-7 in the mean (3.1e-7 before).
+// What bounds the passes is the chain of each block: its loads, one LDS exchange and barrier per step, its
+// stores.  So two stages that fit the registers are one step, the first and last steps work on global memory,
+// twiddles and the PSF column are requested ahead of the barriers, nothing divides by a run-time number, and
+// the blocks are small enough for 16 waves a CU.  Steps of 15 and 16 elements save more exchanges than they are
+// worth (registers: 47 against 43 us in the mean below), and so does every other arithmetic: single-precision cleans
+// amplify a rounding, so sums and products stay those of the separate stages (composite DFTs of 6 to
+// 16 points were 37 us, no less exact, but moved a 120^2 clean by 3e-4).  Convolution of a 1000^2 image on a frame
+// of 2000: 88 us with a division per butterfly, run-time digit reversal, an exchange per stage and two rows a
+// block, 38 us now; frames of 132 / 800 / 3000 / 6000: 39 / 50 / 180 / 719 -> 21 / 23 / 75 / 256 us; geometric mean over 23 frames
+// 96 -> 43 us.
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -74,29 +77,42 @@ __device__ __forceinline__ Cx<T> gmul_i(Cx<T> a) {
 __device__ __forceinline__ int gpad(int i) { return i + (i >> 5); }
 __host__ __device__ __forceinline__ int gspan(int n) { return n + (n >> 5) + 1; }
 
-constexpr int kMaxStages = 8;
-constexpr int kMaxRadix = 16;
+constexpr int kMaxSteps = 8;
 
-// Radix plan of one transform length: stage i (decimation-in-frequency order) has radix r(i) and
-// works on sub-transforms of length Ls_i = L / (r(0) ... r(i-1)).  Four bits a radix (minus one):
-// kernel arguments stay small.
+// A step of a transform: one decimation-in-frequency stage of radix r1, or (r2 > 1) two successive stages in
+// registers, r1 then r2, on the same r1 * r2 elements.
+struct GStep {
+  int r1, r2;
+};
+constexpr int kStepKinds = 12;
+__host__ __device__ constexpr GStep step_kind(int k) {
+  constexpr GStep t[kStepKinds] = {{2, 1}, {3, 1}, {4, 1}, {5, 1}, {7, 1}, {8, 1}, {11, 1}, {13, 1},
+                                   {2, 3}, {2, 5}, {3, 3}, {4, 3}};
+  return t[k];
+}
+
+// Plan of one transform length: step i works on sub-transforms of length Ls_i = L / (r(0) ... r(i-1)), r(i)
+// the product of its radices.  Four bits a step: kernel arguments stay small.
 struct GPlan {
   int L;
   int ns;
   uint32_t code;
-  __host__ __device__ __forceinline__ int r(int i) const { return (int)((code >> (4 * i)) & 15u) + 1; }
+  __host__ __device__ __forceinline__ int kind(int i) const { return (int)((code >> (4 * i)) & 15u); }
+  __host__ __device__ __forceinline__ int r(int i) const { return step_kind(kind(i)).r1 * step_kind(kind(i)).r2; }
 };
 
-// Position of frequency k in the digit-reversed output of the forward transform:
+// Position of frequency k in the digit-reversed output of the forward transform, over its stages:
 // k = d0 + r0 (d1 + r1 (d2 + ...)), position = d0 L/r0 + d1 L/(r0 r1) + ...
 int gperm(const GPlan& p, int k) {
   int pos = 0, span = p.L;
   for (int i = 0; i < p.ns; ++i) {
-    const int r = p.r(i);
-    span /= r;
-    const int q = k / r;
-    pos += (k - q * r) * span;
-    k = q;
+    const GStep st = step_kind(p.kind(i));
+    for (int r : {st.r1, st.r2}) {
+      span /= r;
+      const int q = k / r;
+      pos += (k - q * r) * span;
+      k = q;
+    }
   }
   return pos;
 }
@@ -131,12 +147,45 @@ struct Roots {
   }
 };
 
-// In-register DFT of length R: x_m <- sum_n x_n exp(-+ 2 pi i m n / R) (FWD: minus).  Odd primes in
-// the symmetric form: with a_j = x_j + x_{R-j} and b_j = x_j - x_{R-j}, outputs m and R-m share
-// sum_j cos(2 pi m j / R) a_j and sum_j sin(2 pi m j / R) b_j, a quarter of the direct form's products.
+template <class T, int R, bool FWD>
+struct GDftPow;  // R = 1, 2, 4, 8
+
+// In-register DFT of length R: x_m <- sum_n x_n exp(-+ 2 pi i m n / R) (FWD: minus).  Odd primes in float32: term by
+// term.  Outputs m and R - m use the same products but for signs, so they are formed together, and one pair
+// after the other, or the products of all pairs are live at once (R = 13: 144).
 template <class T, int R, bool FWD>
 struct GDft {
   using C = Cx<T>;
+  __device__ __forceinline__ static C output(const C (&x)[R], int m) {
+    constexpr Roots<R> w{};
+    C acc = x[0];
+#pragma unroll
+    for (int n = 1; n < R; ++n) {
+      const int k = (m * n) % R;
+      acc = gadd(acc, m == 0 ? x[n] : gmul(x[n], cmk<T>((T)w.c[k], FWD ? (T)-w.s[k] : (T)w.s[k])));
+    }
+    return acc;
+  }
+  __device__ __forceinline__ static void run(C (&x)[R]) {
+    C y[R];
+    y[0] = output(x, 0);
+#pragma unroll
+    for (int m = 1; m <= R / 2; ++m) {
+      y[m] = output(x, m);
+      y[R - m] = output(x, R - m);
+      if (R >= 5) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 0; m < R; ++m) x[m] = y[m];
+  }
+};
+// In float64, whose rounding does not steer a clean, in the symmetric form: with a_j = x_j + x_{R-j} and
+// b_j = x_j - x_{R-j}, outputs m and R-m share sum_j cos(2 pi m j / R) a_j and sum_j sin(2 pi m j / R) b_j, a
+// quarter of the products.
+template <int R, bool FWD>
+struct GDft<double, R, FWD> {
+  using T = double;
+  using C = Cx<double>;
   __device__ __forceinline__ static void run(C (&x)[R]) {
     constexpr Roots<R> w{};
     constexpr int H = (R - 1) / 2;
@@ -152,13 +201,13 @@ struct GDft {
     x[0] = sum;
 #pragma unroll
     for (int m = 1; m <= H; ++m) {
-      C u = x0, v = cmk<T>((T)w.s[m] * b[0].x, (T)w.s[m] * b[0].y);
+      C u = x0, v = cmk<T>(w.s[m] * b[0].x, w.s[m] * b[0].y);
 #pragma unroll
       for (int j = 0; j < H; ++j) {
-        const T cc = (T)w.c[(m * (j + 1)) % R];
+        const T cc = w.c[(m * (j + 1)) % R];
         u = cmk<T>(fma(cc, a[j].x, u.x), fma(cc, a[j].y, u.y));
         if (j) {
-          const T ss = (T)w.s[(m * (j + 1)) % R];
+          const T ss = w.s[(m * (j + 1)) % R];
           v = cmk<T>(fma(ss, b[j].x, v.x), fma(ss, b[j].y, v.y));
         }
       }
@@ -168,9 +217,13 @@ struct GDft {
     }
   }
 };
+template <class T, bool FWD>
+struct GDftPow<T, 1, FWD> {
+  __device__ __forceinline__ static void run(Cx<T> (&)[1]) {}
+};
 
 template <class T, bool FWD>
-struct GDft<T, 2, FWD> {
+struct GDftPow<T, 2, FWD> {
   using C = Cx<T>;
   __device__ __forceinline__ static void run(C (&x)[2]) {
     const C a = x[0], b = x[1];
@@ -180,7 +233,7 @@ struct GDft<T, 2, FWD> {
 };
 
 template <class T, bool FWD>
-struct GDft<T, 4, FWD> {
+struct GDftPow<T, 4, FWD> {
   using C = Cx<T>;
   __device__ __forceinline__ static void run(C (&x)[4]) {
     const C s0 = gadd(x[0], x[2]), d0 = gsub(x[0], x[2]);
@@ -193,113 +246,42 @@ struct GDft<T, 4, FWD> {
 };
 
 template <class T, bool FWD>
-struct GDft<T, 8, FWD> {
+struct GDftPow<T, 8, FWD> {
   using C = Cx<T>;
   __device__ __forceinline__ static void run(C (&x)[8]) {
     C e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
-    GDft<T, 4, FWD>::run(e);
-    GDft<T, 4, FWD>::run(o);
+    GDftPow<T, 4, FWD>::run(e);
+    GDftPow<T, 4, FWD>::run(o);
     const T h = (T)0.70710678118654752440;  // cos(pi/4)
-    // o_k * exp(-+ 2 pi i k / 8) for k = 0..3
-    const C t1 = FWD ? cmk<T>(h * (o[1].x + o[1].y), h * (o[1].y - o[1].x))
-                     : cmk<T>(h * (o[1].x - o[1].y), h * (o[1].y + o[1].x));
+    // o_k * exp(-+ 2 pi i k / 8) for k = 0..3, those of 1 and 3 without their factor h
+    const C u1 = FWD ? cmk<T>(o[1].x + o[1].y, o[1].y - o[1].x) : cmk<T>(o[1].x - o[1].y, o[1].y + o[1].x);
     const C t2 = gmul_i<T, FWD>(o[2]);
-    const C t3 = FWD ? cmk<T>(h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y))
-                     : cmk<T>(-h * (o[3].x + o[3].y), h * (o[3].x - o[3].y));
+    const C u3 = FWD ? cmk<T>(o[3].y - o[3].x, -(o[3].x + o[3].y)) : cmk<T>(-(o[3].x + o[3].y), o[3].x - o[3].y);
     x[0] = gadd(e[0], o[0]);
     x[4] = gsub(e[0], o[0]);
-    x[1] = gadd(e[1], t1);
-    x[5] = gsub(e[1], t1);
+    x[1] = cmk<T>(fma(h, u1.x, e[1].x), fma(h, u1.y, e[1].y));
+    x[5] = cmk<T>(fma(-h, u1.x, e[1].x), fma(-h, u1.y, e[1].y));
     x[2] = gadd(e[2], t2);
     x[6] = gsub(e[2], t2);
-    x[3] = gadd(e[3], t3);
-    x[7] = gsub(e[3], t3);
+    x[3] = cmk<T>(fma(h, u3.x, e[3].x), fma(h, u3.y, e[3].y));
+    x[7] = cmk<T>(fma(-h, u3.x, e[3].x), fma(-h, u3.y, e[3].y));
   }
 };
 
-// Composite length A * B: B transforms of length A, the products with exp(-+ 2 pi i b m / AB), A
-// transforms of length B.
-template <class T, int A, int B, bool FWD>
-struct GDft2 {
-  using C = Cx<T>;
-  __device__ __forceinline__ static void run(C (&x)[A * B]) {
-    constexpr Roots<A * B> w{};
-    C y[B][A];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-#pragma unroll
-      for (int a = 0; a < A; ++a) y[b][a] = x[B * a + b];
-      GDft<T, A, FWD>::run(y[b]);
-      if (b) {
-#pragma unroll
-        for (int m = 1; m < A; ++m) {
-          if (4 * b * m == A * B)
-            y[b][m] = gmul_i<T, FWD>(y[b][m]);
-          else
-            y[b][m] = gmul(y[b][m], cmk<T>((T)w.c[b * m], FWD ? (T)-w.s[b * m] : (T)w.s[b * m]));
-        }
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < A; ++m) {
-      C z[B];
-#pragma unroll
-      for (int b = 0; b < B; ++b) z[b] = y[b][m];
-      GDft<T, B, FWD>::run(z);
-#pragma unroll
-      for (int q = 0; q < B; ++q) x[m + A * q] = z[q];
-    }
-  }
-};
+template <bool FWD, class T, int R>
+__device__ __forceinline__ void dft(Cx<T> (&x)[R]) {
+  if constexpr ((R & (R - 1)) == 0)
+    GDftPow<T, R, FWD>::run(x);
+  else
+    GDft<T, R, FWD>::run(x);
+}
 
-// The same for coprime A and B without the products (Good-Thomas): input (B a + A b) mod AB, output the m
-// with m = m_A mod A and m = m_B mod B.
-template <class T, int A, int B, bool FWD>
-struct GDftCoprime {
-  using C = Cx<T>;
-  __device__ __forceinline__ static constexpr int out(int ma, int mb) {
-    int m = ma;
-    while (m % B != mb) m += A;
-    return m;
-  }
-  __device__ __forceinline__ static void run(C (&x)[A * B]) {
-    C y[B][A];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-#pragma unroll
-      for (int a = 0; a < A; ++a) y[b][a] = x[(B * a + A * b) % (A * B)];
-      GDft<T, A, FWD>::run(y[b]);
-    }
-#pragma unroll
-    for (int m = 0; m < A; ++m) {
-      C z[B];
-#pragma unroll
-      for (int b = 0; b < B; ++b) z[b] = y[b][m];
-      GDft<T, B, FWD>::run(z);
-#pragma unroll
-      for (int q = 0; q < B; ++q) x[out(m, q)] = z[q];
-    }
-  }
-};
-template <class T, bool FWD>
-struct GDft<T, 6, FWD> : GDftCoprime<T, 2, 3, FWD> {};
-template <class T, bool FWD>
-struct GDft<T, 9, FWD> : GDft2<T, 3, 3, FWD> {};
-template <class T, bool FWD>
-struct GDft<T, 10, FWD> : GDftCoprime<T, 2, 5, FWD> {};
-template <class T, bool FWD>
-struct GDft<T, 12, FWD> : GDftCoprime<T, 4, 3, FWD> {};
-template <class T, bool FWD>
-struct GDft<T, 14, FWD> : GDftCoprime<T, 2, 7, FWD> {};
-template <class T, bool FWD>
-struct GDft<T, 15, FWD> : GDftCoprime<T, 3, 5, FWD> {};
-template <class T, bool FWD>
-struct GDft<T, 16, FWD> : GDft2<T, 4, 4, FWD> {};
-
-// f(std::integral_constant<int, R>) for the run-time radix r, 2 to 16
+// f(step_kind constants) for the run-time step kind
 template <class F>
-__device__ __forceinline__ void with_radix(int r, F&& f) {
-  switch (r) {
+__device__ __forceinline__ void with_step(int kind, F&& f) {
+  switch (kind) {
+    case 0: f(std::integral_constant<int, 0>{}); break;
+    case 1: f(std::integral_constant<int, 1>{}); break;
     case 2: f(std::integral_constant<int, 2>{}); break;
     case 3: f(std::integral_constant<int, 3>{}); break;
     case 4: f(std::integral_constant<int, 4>{}); break;
@@ -309,71 +291,146 @@ __device__ __forceinline__ void with_radix(int r, F&& f) {
     case 8: f(std::integral_constant<int, 8>{}); break;
     case 9: f(std::integral_constant<int, 9>{}); break;
     case 10: f(std::integral_constant<int, 10>{}); break;
-    case 11: f(std::integral_constant<int, 11>{}); break;
-    case 12: f(std::integral_constant<int, 12>{}); break;
-    case 13: f(std::integral_constant<int, 13>{}); break;
-    case 14: f(std::integral_constant<int, 14>{}); break;
-    case 15: f(std::integral_constant<int, 15>{}); break;
-    default: f(std::integral_constant<int, 16>{}); break;
+    default: f(std::integral_constant<int, 11>{}); break;
   }
 }
 
-// One stage of radix r over a transform of length L, sub-transform length Ls (M = Ls/r), butterflies
-// lt, lt + step, ...: elements from ld(i), results to st(i, v); a butterfly reads and writes the
-// same r elements, so a stage can run in place.  Forward: DFT then twiddles (decimation in
-// frequency); inverse: conjugate twiddles then the inverse DFT, the exact mirror.  tw: the plan's
-// stage twiddles, exp(-2 pi i n k / Ls) at L - Ls + (k-1) M + n, so that neighbouring butterflies read
-// neighbouring entries.  SYNC: a barrier before the first element is read, behind the request of the
-// first butterfly's twiddles.
-template <class T, bool FWD, bool SYNC, class Ld, class St>
-__device__ __forceinline__ void gstage(int r, int L, int Ls, const Cx<T>* __restrict__ tw, int lt, int step, Ld ld,
-                                       St st) {
+// Twiddles of one butterfly of a step on sub-transforms of length Ls, butterfly index n within one.  tw: the
+// plan's stage twiddles, exp(-2 pi i n k / Ls) of the stage of sub-transform length Ls at
+// L - Ls + (k-1) M + n (M = Ls / radix), so that neighbouring butterflies read neighbouring entries.
+template <class T, int R1, int R2>
+struct StepTw {
   using C = Cx<T>;
-  with_radix(r, [&](auto rc) {
-    constexpr int R = decltype(rc)::value;
-    const int M = Ls / R;
+  C w1[R1][R2];  // stage 1: element (k, j) at k M1 + j M2 + n
+  C w2[R2];      // stage 2
+  __device__ __forceinline__ void load(const C* __restrict__ tw, int L, int Ls, int n) {
+    const int M1 = Ls / R1, M2 = M1 / R2;
+    if (R2 > 1 || M1 > 1) {
+      const C* t = tw + (L - Ls);
+#pragma unroll
+      for (int k = 1; k < R1; ++k)
+#pragma unroll
+        for (int j = 0; j < R2; ++j) w1[k][j] = t[(k - 1) * M1 + j * M2 + n];
+    }
+    if (R2 > 1 && M2 > 1) {
+      const C* t = tw + (L - M1);
+#pragma unroll
+      for (int j = 1; j < R2; ++j) w2[j] = t[(j - 1) * M2 + n];
+    }
+  }
+};
+
+// The arithmetic of a step on the elements x[k * R2 + j] at k M1 + j M2.  Forward: stage 1 on the R1 elements of
+// each j, then stage 2 on the R2 of each k, a DFT then twiddles each (decimation in frequency; the last stage of a
+// transform has none).  Inverse: conjugate twiddles then the inverse DFT, the exact mirror.
+template <class T, int R1, int R2, bool FWD>
+__device__ __forceinline__ void step_math(Cx<T> (&x)[R1 * R2], const StepTw<T, R1, R2>& tw, bool tw1, bool tw2) {
+  using C = Cx<T>;
+  const auto stage1 = [&] {
+#pragma unroll
+    for (int j = 0; j < R2; ++j) {
+      C y[R1];
+#pragma unroll
+      for (int k = 0; k < R1; ++k) y[k] = x[k * R2 + j];
+      if (FWD) dft<true>(y);
+      if (R2 > 1 || tw1) {
+#pragma unroll
+        for (int k = 1; k < R1; ++k) y[k] = gmul(y[k], FWD ? tw.w1[k][j] : gconj(tw.w1[k][j]));
+      }
+      if (!FWD) dft<false>(y);
+#pragma unroll
+      for (int k = 0; k < R1; ++k) x[k * R2 + j] = y[k];
+    }
+  };
+  const auto stage2 = [&] {
+    if constexpr (R2 > 1) {
+#pragma unroll
+      for (int k = 0; k < R1; ++k) {
+        C y[R2];
+#pragma unroll
+        for (int j = 0; j < R2; ++j) y[j] = x[k * R2 + j];
+        if (FWD) dft<true>(y);
+        if (tw2) {
+#pragma unroll
+          for (int j = 1; j < R2; ++j) y[j] = gmul(y[j], FWD ? tw.w2[j] : gconj(tw.w2[j]));
+        }
+        if (!FWD) dft<false>(y);
+#pragma unroll
+        for (int j = 0; j < R2; ++j) x[k * R2 + j] = y[j];
+      }
+    }
+  };
+  if (FWD) {
+    stage1();
+    stage2();
+  } else {
+    stage2();
+    stage1();
+  }
+}
+
+// One step over a transform of length L, sub-transform length Ls, butterflies lt, lt + step, ...: elements from
+// ld(i), results to st(i, v); a butterfly reads and writes the same elements, so a step can run in
+// place.  SYNC: a barrier before the first element is read, behind the request of the first butterfly's
+// twiddles.
+template <class T, bool FWD, bool SYNC, class Ld, class St>
+__device__ __forceinline__ void gstep(int kind, int L, int Ls, const Cx<T>* __restrict__ tw, int lt, int step, Ld ld,
+                                      St st) {
+  using C = Cx<T>;
+  with_step(kind, [&](auto kc) {
+    constexpr GStep S = step_kind(decltype(kc)::value);
+    constexpr int R1 = S.r1, R2 = S.r2, R = R1 * R2;
+    const int M1 = Ls / R1, M2 = M1 / R2;
     const int nbf = L / R;
-    const float inv_m = 1.f / (float)M;
-    const C* __restrict__ ts = tw + (L - Ls);
-    // b / M: (b + 1/2) / M is at least 1/(2M) from a whole number, and the float product is off by less
-    // than 2^-21 of it, which is at most 2^-8 / M for b < 2^13
+    const float inv_m = 1.f / (float)M2;
+    // b / M2: (b + 1/2) / M2 is at least 1/(2 M2) from a whole number, and the float product is off by less
+    // than 2^-21 of it, which is at most 2^-8 / M2 for b < 2^13
     int b = lt;
     int blk = (int)(((float)b + 0.5f) * inv_m);
-    int n = b - blk * M;
-    C w[R];
-    if (M > 1 && b < nbf) {
-#pragma unroll
-      for (int k = 1; k < R; ++k) w[k] = ts[(k - 1) * M + n];
-    }
+    int n = b - blk * M2;
+    constexpr bool kAhead = R1 < 11;  // a large DFT holds its inputs and outputs: its twiddles come after it
+    StepTw<T, R1, R2> w;
+    if (kAhead && b < nbf) w.load(tw, L, Ls, n);
     if (SYNC) __syncthreads();
     while (b < nbf) {
       const int base = blk * Ls + n;
       C x[R];
 #pragma unroll
-      for (int k = 0; k < R; ++k) x[k] = ld(base + k * M);
-      if (FWD) GDft<T, R, true>::run(x);
-      if (M > 1) {
+      for (int k = 0; k < R1; ++k)
 #pragma unroll
-        for (int k = 1; k < R; ++k) x[k] = gmul(x[k], FWD ? w[k] : gconj(w[k]));
+        for (int j = 0; j < R2; ++j) x[k * R2 + j] = ld(base + k * M1 + j * M2);
+      if constexpr (kAhead) {
+        step_math<T, R1, R2, FWD>(x, w, M1 > 1, M2 > 1);
+      } else {
+        if (FWD) dft<true>(x);
+        __builtin_amdgcn_sched_barrier(0);
+        if (M1 > 1) {
+          const C* __restrict__ t = tw + (L - Ls) + n;
+#pragma unroll
+          for (int k = 1; k < R1; ++k) {
+            const C v = t[(k - 1) * M1];
+            x[k] = gmul(x[k], FWD ? v : gconj(v));
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (!FWD) dft<false>(x);
       }
-      if (!FWD) GDft<T, R, false>::run(x);
 #pragma unroll
-      for (int k = 0; k < R; ++k) st(base + k * M, x[k]);
+      for (int k = 0; k < R1; ++k)
+#pragma unroll
+        for (int j = 0; j < R2; ++j) st(base + k * M1 + j * M2, x[k * R2 + j]);
       b += step;
       if (b < nbf) {
         blk = (int)(((float)b + 0.5f) * inv_m);
-        n = b - blk * M;
-        if (M > 1) {
-#pragma unroll
-          for (int k = 1; k < R; ++k) w[k] = ts[(k - 1) * M + n];
-        }
+        n = b - blk * M2;
+        if (kAhead) w.load(tw, L, Ls, n);
       }
     }
   });
 }
 
 // Tables of one frame side P, in one device allocation: stage twiddles of the P plan and of the P/2
-// plan, the split factors exp(-2 pi i k / P) for k <= P/4, the digit reversal of the P/2 plan.
+// plan, the split factors exp(-2 pi i k / P) for k <= P/2, the digit reversal of the P/2 plan.
 template <class T>
 struct GTables {
   const Cx<T>* col;
@@ -412,7 +469,7 @@ struct GC2rBatch {
 // image, the split computes outputs k and L - k from one read of both.
 // VEC: image rows of even length at aligned addresses, read two values at a time.
 template <class T, class TIN, bool VEC, int NB>
-__global__ __launch_bounds__(kGThreads) void k_g_r2c(GR2cBatch<T, NB> bt, GPlan pl, int P, int q, int off, int n_rows,
+__global__ __launch_bounds__(kGThreads, sizeof(T) == 4 ? 4 : 2) void k_g_r2c(GR2cBatch<T, NB> bt, GPlan pl, int P, int q, int off, int n_rows,
                                                      int ldT, int lg, GTables<T> tab) {
   using C = Cx<T>;
   const int jb = blockIdx.y;
@@ -451,22 +508,25 @@ __global__ __launch_bounds__(kGThreads) void k_g_r2c(GR2cBatch<T, NB> bt, GPlan 
       return cmk<T>(ok0 ? v0 : (T)0, ok1 ? v1 : (T)0);
     }
   };
-  gstage<T, true, false>(pl.r(0), L, L, tab.row, lt, step, image, lds_st);
+  gstep<T, true, false>(pl.kind(0), L, L, tab.row, lt, step, image, lds_st);
   int Ls = L / pl.r(0);
   for (int i = 1; i < pl.ns; ++i) {
-    gstage<T, true, true>(pl.r(i), L, Ls, tab.row, lt, step, lds_ld, lds_st);
+    gstep<T, true, true>(pl.kind(i), L, Ls, tab.row, lt, step, lds_ld, lds_st);
     Ls /= pl.r(i);
   }
   __syncthreads();
   if (!live) return;
+  const auto split = [](C zk, C zl, C tw) {  // zl: conj z_{L-k}
+    const C e = gscale(gadd(zk, zl), (T)0.5);
+    const C dd = gscale(gsub(zk, zl), (T)0.5);
+    const C o = cmk<T>(dd.y, -dd.x);  // (zk - conj z_{L-k}) / (2i)
+    return gadd(e, gmul(tw, o));
+  };
   for (int k = lt; 2 * k <= L; k += step) {
     const C zk = lds_ld(tab.perm[k]);
     const C zl = gconj(lds_ld(tab.perm[k == 0 ? 0 : L - k]));
-    const C e = gscale(gadd(zk, zl), (T)0.5);
-    const C dd = gscale(gsub(zk, zl), (T)0.5);
-    const C o = gmul(tab.split[k], cmk<T>(dd.y, -dd.x));  // (zk - conj z_{L-k}) / (2i), times exp(-2 pi i k / P)
-    T1[(size_t)k * ldT + fr] = gadd(e, o);
-    if (2 * k < L) T1[(size_t)(L - k) * ldT + fr] = gconj(gsub(e, o));
+    T1[(size_t)k * ldT + fr] = split(zk, zl, tab.split[k]);
+    if (2 * k < L) T1[(size_t)(L - k) * ldT + fr] = split(gconj(zl), gconj(zk), tab.split[L - k]);
   }
 }
 
@@ -474,11 +534,11 @@ __global__ __launch_bounds__(kGThreads) void k_g_r2c(GR2cBatch<T, NB> bt, GPlan 
 // P-point FFT.  SPEC: store the spectrum column.  Otherwise multiply by the PSF column, inverse
 // FFT, store the first n_out rows: T2[k * n_out + i].
 //
-// The first stage reads the column, the last inverse stage stores it; between them the last forward
-// stage, the product and the first inverse stage work on the same r elements and stay in registers.
+// The first step reads the column, the last inverse step stores it; between them the last forward
+// step, the product and the first inverse step work on the same r elements and stay in registers.
 // The spectrum is stored as they read it: element k of butterfly b at k * (P/r) + b.
 template <class T, bool SPEC, int NB>
-__global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T, NB> bt, GPlan pl, int n_in, int n_out, int G,
+__global__ __launch_bounds__(kGThreads, sizeof(T) == 4 ? 4 : 2) void k_g_cols(GColBatch<T, NB> bt, GPlan pl, int n_in, int n_out, int G,
                                                       GTables<T> tab) {
   using C = Cx<T>;
   const int jb = blockIdx.y;
@@ -500,21 +560,25 @@ __global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T, NB> bt, GPlan
     const C v = col[i < n_in ? i : 0];
     return i < n_in ? v : cmk<T>(0, 0);
   };
-  gstage<T, true, false>(pl.r(0), P, P, tab.col, lt, step, column, lds_st);
+  gstep<T, true, false>(pl.kind(0), P, P, tab.col, lt, step, column, lds_st);
   int Ls = P / pl.r(0);
   const int last = pl.ns - 1;
   for (int i = 1; i < last; ++i) {
-    gstage<T, true, true>(pl.r(i), P, Ls, tab.col, lt, step, lds_ld, lds_st);
+    gstep<T, true, true>(pl.kind(i), P, Ls, tab.col, lt, step, lds_ld, lds_st);
     Ls /= pl.r(i);
   }
   C* __restrict__ out = bt.T2[jb] + (size_t)(live ? k : 0) * (SPEC ? P : n_out);
   const C* __restrict__ S = SPEC ? nullptr : bt.S[jb] + (size_t)(live ? k : 0) * P;
-  with_radix(pl.r(last), [&](auto rc) {
-    constexpr int R = decltype(rc)::value;
+  with_step(pl.kind(last), [&](auto kc) {
+    constexpr GStep K = step_kind(decltype(kc)::value);
+    constexpr int R1 = K.r1, R2 = K.r2, R = R1 * R2;
     const int nbf = P / R;
     int b = lt;
+    StepTw<T, R1, R2> w;
+    if (R2 > 1) w.load(tab.col, P, R, 0);
+    constexpr bool kAhead = R1 < 11;
     C s[R];
-    if (!SPEC && b < nbf) {
+    if (!SPEC && kAhead && b < nbf) {
 #pragma unroll
       for (int m = 0; m < R; ++m) s[m] = S[m * nbf + b];
     }
@@ -523,21 +587,27 @@ __global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T, NB> bt, GPlan
       C x[R];
 #pragma unroll
       for (int m = 0; m < R; ++m) x[m] = lds_ld(b * R + m);
-      GDft<T, R, true>::run(x);
+      step_math<T, R1, R2, true>(x, w, false, false);
       if (SPEC) {
         if (live) {
 #pragma unroll
           for (int m = 0; m < R; ++m) out[m * nbf + b] = x[m];
         }
       } else {
+        if (!kAhead) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int m = 0; m < R; ++m) s[m] = S[m * nbf + b];
+        }
 #pragma unroll
         for (int m = 0; m < R; ++m) x[m] = gmul(x[m], s[m]);
-        GDft<T, R, false>::run(x);
+        if (!kAhead) __builtin_amdgcn_sched_barrier(0);
+        step_math<T, R1, R2, false>(x, w, false, false);
 #pragma unroll
         for (int m = 0; m < R; ++m) lds_st(b * R + m, x[m]);
       }
       b += step;
-      if (!SPEC && b < nbf) {
+      if (!SPEC && kAhead && b < nbf) {
 #pragma unroll
         for (int m = 0; m < R; ++m) s[m] = S[m * nbf + b];
       }
@@ -546,12 +616,12 @@ __global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T, NB> bt, GPlan
   if (SPEC) return;
   for (int i = last - 1; i > 0; --i) {
     Ls *= pl.r(i);
-    gstage<T, false, true>(pl.r(i), P, Ls, tab.col, lt, step, lds_ld, lds_st);
+    gstep<T, false, true>(pl.kind(i), P, Ls, tab.col, lt, step, lds_ld, lds_st);
   }
   const auto kept = [&](int i, C v) {
     if (live && i < n_out) out[i] = v;
   };
-  gstage<T, false, true>(pl.r(0), P, P, tab.col, lt, step, lds_ld, kept);
+  gstep<T, false, true>(pl.kind(0), P, P, tab.col, lt, step, lds_ld, kept);
 }
 
 // ---- pass 3: per kept row r: Hermitian half spectrum T2[k * ldT + r], k in [0, P/2] -> the
@@ -560,7 +630,7 @@ __global__ __launch_bounds__(kGThreads) void k_g_cols(GColBatch<T, NB> bt, GPlan
 // read once for both their elements, and the last stage stores the image.
 // VEC: output rows of even length at aligned addresses.
 template <class T, bool VEC, int NB>
-__global__ __launch_bounds__(kGThreads) void k_g_c2r(GC2rBatch<T, NB> bt, GPlan pl, int n, int ldT, int lg, T scale,
+__global__ __launch_bounds__(kGThreads, sizeof(T) == 4 ? 4 : 2) void k_g_c2r(GC2rBatch<T, NB> bt, GPlan pl, int n, int ldT, int lg, T scale,
                                                      GTables<T> tab) {
   using C = Cx<T>;
   const int jb = blockIdx.y;
@@ -577,18 +647,20 @@ __global__ __launch_bounds__(kGThreads) void k_g_c2r(GC2rBatch<T, NB> bt, GPlan 
   const C* __restrict__ T2 = bt.T2[jb] + (live ? r : 0);
   const auto lds_ld = [&](int i) { return sm[gpad(i) << lg]; };
   const auto lds_st = [&](int i, C v) { sm[gpad(i) << lg] = v; };
+  const auto merge = [](C xk, C xl, C tw) {  // xl: conj X_{L-k}
+    const C d = gmul(gsub(xk, xl), gconj(tw));  // (X_k - conj X_{L-k}) exp(+2 pi i k / P)
+    return gadd(gadd(xk, xl), cmk<T>(-d.y, d.x));
+  };
   for (int k = lt; 2 * k <= L; k += step) {
     const C xk = T2[(size_t)k * ldT];
     const C xl = gconj(T2[(size_t)(L - k) * ldT]);
-    const C s = gadd(xk, xl);
-    const C d = gmul(gsub(xk, xl), gconj(tab.split[k]));  // (X_k - conj X_{L-k}) exp(+2 pi i k / P)
-    lds_st(tab.perm[k], gadd(s, cmk<T>(-d.y, d.x)));
-    if (k > 0 && 2 * k < L) lds_st(tab.perm[L - k], gadd(gconj(s), cmk<T>(d.y, d.x)));
+    lds_st(tab.perm[k], merge(xk, xl, tab.split[k]));
+    if (k > 0 && 2 * k < L) lds_st(tab.perm[L - k], merge(gconj(xl), gconj(xk), tab.split[L - k]));
   }
   int Ls = 1;
   for (int i = pl.ns - 1; i > 0; --i) {
     Ls *= pl.r(i);
-    gstage<T, false, true>(pl.r(i), L, Ls, tab.row, lt, step, lds_ld, lds_st);
+    gstep<T, false, true>(pl.kind(i), L, Ls, tab.row, lt, step, lds_ld, lds_st);
   }
   T* __restrict__ out = bt.out[jb] + (size_t)(live ? r : 0) * n;
   const auto image = [&](int e, C v) {
@@ -599,44 +671,44 @@ __global__ __launch_bounds__(kGThreads) void k_g_c2r(GC2rBatch<T, NB> bt, GPlan 
       if (live && 2 * e + 1 < n) out[2 * e + 1] = v.y * scale;
     }
   };
-  gstage<T, false, true>(pl.r(0), L, L, tab.row, lt, step, lds_ld, image);
+  gstep<T, false, true>(pl.kind(0), L, L, tab.row, lt, step, lds_ld, image);
 }
 
 // ---- host side --------------------------------------------------------------------------------
-// The plan of length L: the factors of 2 to 16 with the fewest stages (at least min_stages; each one is a
-// pass through LDS and a barrier), of those the one of the smallest sum (the fewest operations).
-// Even factors come first and odd ones last: the late stages' LDS strides are multiples of the last radix, and
-// odd ones touch all banks.
-bool make_gplan(int L, int min_stages, GPlan* p) {
-  struct Search {
-    int min_stages;
-    int cur[kMaxStages], best[kMaxStages];
-    int best_n = kMaxStages + 1, best_sum = 0;
-    void go(int m, int top, int n, int sum) {
-      if (m == 1) {
-        if (n >= min_stages && (n < best_n || (n == best_n && sum < best_sum))) {
-          best_n = n;
-          best_sum = sum;
-          std::copy(cur, cur + n, best);
-        }
-        return;
-      }
-      if (n == kMaxStages || n >= best_n) return;
-      for (int r = std::min(top, m); r >= 2; --r) {
-        if (m % r != 0) continue;
-        cur[n] = r;
-        go(m / r, r, n + 1, sum + r);
-      }
+// The plan of length L: its stages are radix 8 while the length allows, a 4 or 2 for the rest of the power of
+// two, then the odd primes in order (which fixes every rounding); neighbouring stages are taken together where a
+// step kind has them, with the fewest steps, at least min_steps (each is a pass through LDS and a barrier).
+bool make_gplan(int L, int min_steps, GPlan* p) {
+  constexpr int kMostStages = 16;
+  int r[kMostStages], n = 0, m = L;
+  for (int f : {8, 4, 2, 3, 5, 7, 11, 13})
+    while (m % f == 0 && n < kMostStages) {
+      r[n++] = f;
+      m /= f;
+      if (f == 4 || f == 2) break;  // at most one of each is left by the eights
     }
-  } s;
-  s.min_stages = min_stages;
-  s.go(L, kMaxRadix, 0, 0);
-  if (s.best_n > kMaxStages) return false;
-  std::stable_partition(s.best, s.best + s.best_n, [](int r) { return r % 2 == 0; });
+  if (m != 1 || n == 0) return false;
+  const auto kind_of = [&](int i, int count) {  // the step of `count` stages from stage i on, or -1
+    for (int k = 0; k < kStepKinds; ++k)
+      if (step_kind(k).r1 == r[i] && step_kind(k).r2 == (count == 2 ? r[i + 1] : 1)) return k;
+    return -1;
+  };
+  int steps[kMostStages + 1], take[kMostStages];  // from stage i on: the fewest steps, the stages of the first of them
+  steps[n] = 0;
+  for (int i = n - 1; i >= 0; --i) {
+    steps[i] = 1 + steps[i + 1];
+    take[i] = 1;
+    const bool two = i + 1 < n && kind_of(i, 2) >= 0 && !(i == 0 && n == 2 && min_steps == 2);
+    if (two && 1 + steps[i + 2] < steps[i]) {
+      steps[i] = 1 + steps[i + 2];
+      take[i] = 2;
+    }
+  }
+  if (steps[0] > kMaxSteps || steps[0] < min_steps) return false;
   p->L = L;
-  p->ns = s.best_n;
+  p->ns = 0;
   p->code = 0;
-  for (int i = 0; i < p->ns; ++i) p->code |= (uint32_t)(s.best[i] - 1) << (4 * i);
+  for (int i = 0; i < n; i += take[i]) p->code |= (uint32_t)kind_of(i, take[i]) << (4 * p->ns++);
   return true;
 }
 bool row_plan(int p, GPlan* pl) { return make_gplan(p / 2, 1, pl); }
@@ -682,16 +754,19 @@ struct TwKey {
 std::mutex g_gtw_mu;
 std::map<TwKey, void*> g_gtw;
 
-// stage twiddles of a plan, laid out as gstage reads them, from w[k] = exp(-2 pi i k / P)
+// stage twiddles of a plan, laid out as StepTw reads them, from w[k] = exp(-2 pi i k / P)
 template <class C>
 void stage_twiddles(const GPlan& pl, const std::vector<C>& w, C* out) {
   const int P = (int)w.size();
   int Ls = pl.L;
   for (int i = 0; i < pl.ns; ++i) {
-    const int r = pl.r(i), M = Ls / r, tstep = P / Ls;
-    for (int k = 1; k < r; ++k)
-      for (int n = 0; n < M; ++n) out[pl.L - Ls + (k - 1) * M + n] = w[(size_t)n * k * tstep];
-    Ls = M;
+    const GStep st = step_kind(pl.kind(i));
+    for (int r : {st.r1, st.r2}) {
+      const int M = Ls / r, tstep = P / Ls;
+      for (int k = 1; k < r; ++k)
+        for (int n = 0; n < M; ++n) out[pl.L - Ls + (k - 1) * M + n] = w[(size_t)n * k * tstep];
+      Ls = M;
+    }
   }
 }
 
@@ -699,7 +774,7 @@ void stage_twiddles(const GPlan& pl, const std::vector<C>& w, C* out) {
 template <class T>
 GTables<T> g_tables(int p) {
   using C = Cx<T>;
-  const int L = p / 2, n_split = p / 4 + 1;
+  const int L = p / 2, n_split = L + 1;
   int dev = 0;
   PMS_HIP(hipGetDevice(&dev));
   const TwKey key{dev, p, (int)sizeof(T)};

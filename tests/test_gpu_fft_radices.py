@@ -1,8 +1,8 @@
-"""Convolutions on frames that are not powers of two, over the radices of their plans.
+"""Convolutions on frames that are not powers of two, over the stages of their plans.
 
-Frames whose column and row lengths use every radix from 2 to 16, first, between and last; plans of
-one row stage (P/2 <= 16) and of many; rows of odd length; images and results at addresses that are not a
-multiple of two values (which the vector loads and stores of the row passes need); frames at
+Frames whose column and row lengths use every step (one stage of radix 2 to 13, or two at once), first, between
+and last; plans of one row step and of many; rows of odd length; images and results at addresses that
+are not a multiple of two values (which the vector loads and stores of the row passes need); frames at
 which the block shapes of the passes change.  A pass rounds every value about once a stage, each time
 by some 1.5 * 2^-24 rms, in at most 8 + 8 column and 4 + 4 row stages: 5e-7 rms of the result, held to three times that.
 """
