@@ -833,15 +833,20 @@ void set_g_attrs() {
   });
 }
 
+// Frames whose transforms there are kernels for: powers of two run on their own (fft_pow2.h), whatever
+// the steps below could make of them (4 and 8 are a single stage, which a column plan cannot be).
+bool has_kernels(int p) {
+  GPlan pl;
+  return is_pow2(p) || (col_plan(p, &pl) && row_plan(p, &pl));
+}
+
 template <class T>
 void check_g_frame(int p) {
-  GPlan pl;
   PMS_REQUIRE(p >= 4 && p % 2 == 0, "FFT frame side must be even and >= 4, got " + std::to_string(p));
   PMS_REQUIRE(p <= gfft_max_frame(sizeof(T)),
               "FFT frame side " + std::to_string(p) + " exceeds the " + std::to_string(gfft_max_frame(sizeof(T))) +
                   " that one LDS transform holds in " + (sizeof(T) == 8 ? "float64" : "float32"));
-  PMS_REQUIRE(col_plan(p, &pl) && row_plan(p, &pl),
-              "FFT frame side " + std::to_string(p) + " has a prime factor above 13");
+  PMS_REQUIRE(has_kernels(p), "FFT frame side " + std::to_string(p) + " has a prime factor above 13");
 }
 
 template <class T, class TIN, bool VEC, int NB>
@@ -883,8 +888,7 @@ void launch_c2r(const GC2rBatch<T, NB>& bt, int nb, int p, int n, int ldT, const
 int gfft_max_frame(size_t real_bytes) { return real_bytes == 8 ? 8192 : 16384; }
 
 bool gfft_frame_ok(int p, size_t real_bytes) {
-  GPlan pl;
-  return p >= 4 && p % 2 == 0 && p <= gfft_max_frame(real_bytes) && col_plan(p, &pl) && row_plan(p, &pl);
+  return p >= 4 && p % 2 == 0 && p <= gfft_max_frame(real_bytes) && has_kernels(p);
 }
 
 int gfft_perm(int k, int p) {
