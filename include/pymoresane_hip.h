@@ -61,13 +61,17 @@ size_t pms_iuwt_work_bytes(int h, int w);
 
 /* Detail planes for scales scale_adjust..scale_count-1 of `in` (h x w) into
  * detail_out ((scale_count-scale_adjust) planes); smoothed_out (h x w) may be
- * NULL.  Requires 2^scale_count <= min(h, w).
+ * NULL.  Requires 2^scale_count <= min(h, w).  No buffer may overlap another, but
+ * `in` may be smoothed_out or a detail plane other than the first when
+ * scale_count - scale_adjust >= 2 (it is used up before they are written).
  * Replaces iuwt.iuwt_decomposition (pymoresane/iuwt.py:17-41, gpu path 384-499). */
 int pms_iuwt_decompose(const float* in, int h, int w, int scale_count, int scale_adjust, float* detail_out,
                        float* smoothed_out, void* work, void* stream);
 
 /* Recompose n_planes detail planes (scales scale_adjust..) with optional
- * smoothed base (NULL = zeros) into out (h x w).
+ * smoothed base (NULL = zeros) into out (h x w).  No buffer may overlap another,
+ * but when n_planes >= 2 (3 without `smoothed`) out may be `smoothed` or a detail
+ * plane other than the first (those are used up before it is written).
  * Replaces iuwt.iuwt_recomposition (pymoresane/iuwt.py:43-64, gpu path 501-581). */
 int pms_iuwt_recompose(const float* detail, int n_planes, int h, int w, int scale_adjust, const float* smoothed,
                        float* out, void* work, void* stream);

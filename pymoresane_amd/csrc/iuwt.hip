@@ -1350,10 +1350,17 @@ long iuwt_decompose(const float* in, int h, int w, int scale_count, int scale_ad
   return j.np;
 }
 
+static bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
+  if (!a || !b) return false;
+  const char* pa = static_cast<const char*>(a);
+  const char* pb = static_cast<const char*>(b);
+  return pa < pb + nb && pb < pa + na;
+}
+
 // Scale by scale over all jobs: at scale s a job either pre-smooths (s < scale_adjust) or
 // decomposes (scale_adjust <= s < scale_count); jobs of the same kind share one launch.
 static void decompose_batch_impl(IuwtDecompJob* jobs, int count, int h, int w, bool small, hipStream_t st) {
-  const size_t plane = (size_t)h * w;
+  const size_t plane = (size_t)h * w, pb = plane * sizeof(float);
   struct State {
     const float* cur;
     int slot;
@@ -1405,10 +1412,16 @@ static void decompose_batch_impl(IuwtDecompJob* jobs, int count, int h, int w, b
         } else {
           if (s < j.scale_adjust || s >= j.scale_count || s < state[k].done) continue;
           const int kk = s - j.scale_adjust;
-          if (pair_plan && s + 1 < j.scale_count && kk % 2 == 0 && j.detail && !j.ref) {
+          // a pair reads its input around the pixels that it writes: a job whose input is the smoothed plane or
+          // the second detail plane takes one scale a launch, by which the input is used up before it is written
+          float* const out_c = (s + 1 == j.scale_count - 1) ? j.smoothed : ping;
+          const bool pair = pair_plan && s + 1 < j.scale_count && kk % 2 == 0 && j.detail && !j.ref &&
+                            !overlaps(state[k].cur, pb, out_c, pb) &&
+                            !overlaps(state[k].cur, pb, j.detail + (size_t)kk * plane, 2 * pb);
+          if (pair) {
             Dec2Job pj{};
             pj.in = state[k].cur;
-            pj.out_c = (s + 1 == j.scale_count - 1) ? j.smoothed : ping;
+            pj.out_c = out_c;
             pj.out_w0 = j.detail + (size_t)kk * plane;
             pj.out_w1 = j.detail + (size_t)(kk + 1) * plane;
             pj.mask0 = j.mask ? j.mask + (size_t)kk * plane : nullptr;
@@ -1480,7 +1493,7 @@ void iuwt_recompose(const float* detail, int nplanes, int h, int w, int scale_ad
 // job's r-th step, steps of the same kind and scale sharing one launch.  Without a smoothed base R
 // starts at zero, so a job's coarsest step is its (masked) detail plane itself.
 static void recompose_batch_impl(const IuwtRecompJob* jobs, int count, int h, int w, bool small, hipStream_t st) {
-  const size_t plane = (size_t)h * w;
+  const size_t plane = (size_t)h * w, pb = plane * sizeof(float);
   enum { OP_RECOMP, OP_SMOOTH, OP_PAIR };
   struct Op {
     int kind, s;  // OP_PAIR covers scales s+1 then s
@@ -1526,7 +1539,12 @@ static void recompose_batch_impl(const IuwtRecompJob* jobs, int count, int h, in
         --s;
         continue;
       }
-      if (pair && s - 1 >= j.scale_adjust && (small2_applies(small || tile2_range(h, w, s - 1, count, true), h, w, s - 1) || (!small && recomp2_plan(h, w, s - 1, &pl)))) {
+      // the last pair reads R and w_1 around the pixels of `out`: one scale a launch where those overlap
+      const bool own_out = s != 1 || !(overlaps(j.out, pb, j.detail + plane, pb) ||
+                                       (sk.ops.empty() && overlaps(j.out, pb, sk.cur, pb)));
+      if (pair && own_out && s - 1 >= j.scale_adjust &&
+          (small2_applies(small || tile2_range(h, w, s - 1, count, true), h, w, s - 1) ||
+           (!small && recomp2_plan(h, w, s - 1, &pl)))) {
         sk.ops.push_back({OP_PAIR, s - 1});
         s -= 2;
       } else {
@@ -1753,13 +1771,6 @@ std::vector<TuneParams> walk_candidates(int h, int w, bool recomp) {
   for (int p : pairs)
     for (int b : blocks) c.push_back(TuneParams{b, p});
   return c;
-}
-
-bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
-  if (!a || !b) return false;
-  const char* pa = static_cast<const char*>(a);
-  const char* pb = static_cast<const char*>(b);
-  return pa < pb + nb && pb < pa + na;
 }
 
 }  // namespace
