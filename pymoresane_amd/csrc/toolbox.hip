@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 #include "pms_internal.h"
 
@@ -371,18 +372,27 @@ __device__ __forceinline__ void store_stream(T* p, const Quad<T>& q) {
 //     either side.  One pass over the plane (k_mad_scan) counts the keys below the range, counts those in
 //     it in 64 bins and sets them aside (6 to 9% of the plane), and one block a plane (k_mad_pick) takes the
 //     bin of the median's rank and selects in it (from a list of that bin, k_mad_collect, on large planes).
+// An end of the range that many keys are equal to (blanked pixels, quantised values) is not a part of it: those keys
+// are only counted, so that the range holds what the sample says of it whatever the values (see MadRange::tied).
 // Nothing is estimated in the result: when the range misses the median's rank or more keys fall in it
-// than there is room for, k_mad_pick selects from the plane itself.  The result is the same key, and
-// for even counts the same pair of keys, as the radix select's.
+// than there is room for, k_mad_pick selects from the plane itself, with one block; the sample all but rules that
+// out.  The result is the same key, and for even counts the same pair of keys, as the radix select's.
 constexpr int kMT = 1024;            // threads of the one-block kernels
 constexpr int kMadOne = 32 * kMT;    // noise pixels that one block holds in registers
 constexpr int kMadBins = 64;         // bins of the range
 
+// tied: the sample's ends of the range are the keys lo - 1 and lo + range + 1, outside it and counted by themselves.
+// Such a range often starts at the smallest denormal (above zeros) and spans many binades, so its bins are of equal
+// width in value, not in key: bins of equal key width put half of it in one (seven 4096^2 planes with 48% zeros: 520 us).
 template <class K>
 struct alignas(16) MadRange {
   K lo, range;      // keys lo .. lo + range (inclusive)
   K least2;         // k_mad_collect: least key of the successor's bin
-  uint32_t shift;   // bin = (key - lo) >> shift, below kMadBins
+  uint32_t shift;   // bin = (key - lo) >> shift, below kMadBins; tied: bits of `range`, bin = tied_bin(key)
+  uint32_t tied;
+  float scale;      // tied: kMadBins / (value of the upper end - value of lo)
+  uint32_t at_lo;   // tied: keys equal to lo - 1
+  uint32_t at_hi;   // tied: keys equal to lo + range + 1
   uint32_t below;   // keys below lo
   uint32_t n;       // keys of the range set aside (counted beyond the room for them)
   uint32_t listed;  // k_mad_collect: keys of the median's bin (counted beyond the room for them)
@@ -402,6 +412,14 @@ __device__ __forceinline__ int bit_length(K v) {
     return v ? 64 - __clzll((long long)v) : 0;
   else
     return v ? 32 - __clz((int)v) : 0;
+}
+
+// Bin of a key of a tied range whose least value is `low`.  Each operation is monotonic and a NaN (an infinite or NaN
+// end) comes out alike for all keys, so the bins are in the keys' order whatever the scale.
+template <class T>
+__device__ __forceinline__ int tied_bin(typename MadKey<T>::K key, T low, float scale) {
+  const T x = (MadKey<T>::val(key) - low) * (T)scale;
+  return x < (T)(kMadBins - 1) ? (int)x : kMadBins - 1;
 }
 
 // Where a block finds ranks in the 2048 counts of h (LDS): the bin, the counts before it and its own.
@@ -604,30 +622,35 @@ __global__ __launch_bounds__(kMT) void k_mad_pivot(const T* __restrict__ planes,
   constexpr int kKeyBits = 8 * sizeof(K) - 1;
   __shared__ uint32_t h0[kBins], h1[kBins];
   __shared__ BinScratch scratch;
+  __shared__ K red[kMT / 64];
   __shared__ uint32_t taken;
   const int s = blockIdx.x, t = threadIdx.x;
   const T* x = planes + (size_t)s * plane;
   if (t < kMadBins) hist[(size_t)s * kMadBins + t] = 0;
   if (t == 0) taken = 0;
   const uint32_t stratum = area / (PT / 4 * kMT);  // at least 16 (area > kMadOne)
-  K key[PT];
-  uint32_t have = 0;
-  const bool vec = !MASKED && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const auto sample = [&](const T* from, K(&key)[PT]) {  // returns which of the keys are noise pixels'
+    uint32_t have = 0;
+    const bool vec = !MASKED && (reinterpret_cast<uintptr_t>(from) & 15) == 0;
 #pragma unroll
-  for (int i = 0; i < PT / 4; ++i) {
-    const uint32_t c = t + i * kMT;
-    const uint32_t at = c * stratum + ((c * 2654435761u) >> 8) % (stratum - 3);
-    if (vec) {
-      const Quad<T> q = reinterpret_cast<const Quad<T>*>(x)[at / 4];
+    for (int i = 0; i < PT / 4; ++i) {
+      const uint32_t c = t + i * kMT;
+      const uint32_t at = c * stratum + ((c * 2654435761u) >> 8) % (stratum - 3);
+      if (vec) {
+        const Quad<T> q = reinterpret_cast<const Quad<T>*>(from)[at / 4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) key[4 * i + k] = MadKey<T>::key(q.a[k]);
-      have |= 15u << (4 * i);
-      continue;
+        for (int k = 0; k < 4; ++k) key[4 * i + k] = MadKey<T>::key(q.a[k]);
+        have |= 15u << (4 * i);
+        continue;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (noise_key<T, MASKED>(from, w, inc, exc, at + k, &key[4 * i + k])) have |= 1u << (4 * i + k);
     }
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (noise_key<T, MASKED>(x, w, inc, exc, at + k, &key[4 * i + k])) have |= 1u << (4 * i + k);
-  }
+    return have;
+  };
+  K key[PT];
+  const uint32_t have = sample(x, key);
   __syncthreads();
   atomicAdd(&taken, (uint32_t)__popc(have));
   __syncthreads();
@@ -635,11 +658,12 @@ __global__ __launch_bounds__(kMT) void k_mad_pivot(const T* __restrict__ planes,
   const uint32_t half = (uint32_t)(4.f * sqrtf((float)m)) + 8;
   uint32_t r0 = m / 2 > half ? m / 2 - half : 0, r1 = m / 2 + half;
   const bool open0 = m / 2 <= half, open1 = r1 >= m;
-  // Digits of both ends: two, which is a range's width to better than a tenth, or three (a float32 key)
-  // where both ends share two, as where many keys are equal.
+  // Digits of both ends: two, which is a range's width to better than a tenth, and more while over 1/128 of the
+  // sample shares an end's digits and not its value: with the 1/15 of the sample between the ends (1/11 of 8192
+  // keys) the range then stays within the room for it, 1/8, once an end that many keys are equal to is not in it.
   K lo = 0, hi = 0;
-  int rest = kKeyBits;
-  for (int top = kKeyBits, pass = 0; top > 0 && (pass < 2 || (pass < 3 && lo == hi)); ++pass) {
+  uint32_t n_lo = 0, n_hi = 0;  // keys that share an end's digits
+  const auto digit = [&](const K(&q)[PT], uint32_t live, int top) {  // the one below bit `top`
     const int nd = min(11, top), shift = top - nd;
     const bool apart = lo != hi;
     clear_bins(h0);
@@ -647,10 +671,10 @@ __global__ __launch_bounds__(kMT) void k_mad_pivot(const T* __restrict__ planes,
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-      if (!((have >> i) & 1)) continue;
-      const uint32_t d = (uint32_t)(key[i] >> shift) & ((1u << nd) - 1);
-      if ((key[i] >> top) == (lo >> top)) atomicAdd(&h0[d], 1u);
-      if (apart && (key[i] >> top) == (hi >> top)) atomicAdd(&h1[d], 1u);
+      if (!((live >> i) & 1)) continue;
+      const uint32_t d = (uint32_t)(q[i] >> shift) & ((1u << nd) - 1);
+      if ((q[i] >> top) == (lo >> top)) atomicAdd(&h0[d], 1u);
+      if (apart && (q[i] >> top) == (hi >> top)) atomicAdd(&h1[d], 1u);
     }
     __syncthreads();
     BinHit a, b;
@@ -660,19 +684,55 @@ __global__ __launch_bounds__(kMT) void k_mad_pivot(const T* __restrict__ planes,
     hi |= (K)b.bin << shift;
     r0 -= a.before;
     r1 -= b.before;
-    top = shift;
-    rest = top;
+    n_lo = a.count;
+    n_hi = b.count;
+  };
+  int rest = kKeyBits;
+  for (; rest > kKeyBits - 22; rest -= 11) digit(key, have, rest);
+  const uint32_t few = m / 128;
+  if (n_lo > few || n_hi > few) {
+    // The sample is read again: kept in registers until here, it made the kernel 18 -> 22 us where nothing is tied.
+    const T* again = x;
+    asm volatile("" : "+s"(again));
+    K q[PT];
+    const uint32_t live = sample(again, q);
+    // are the keys that share an end's digits one value?
+    K least_lo = ~(K)0, high_lo = ~(K)0, least_hi = ~(K)0, high_hi = ~(K)0;  // high: complement of the greatest
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      if (!((live >> i) & 1)) continue;
+      const K prefix = q[i] >> rest;
+      if (prefix == (lo >> rest)) least_lo = min(least_lo, q[i]), high_lo = min(high_lo, ~q[i]);
+      if (prefix == (hi >> rest)) least_hi = min(least_hi, q[i]), high_hi = min(high_hi, ~q[i]);
+    }
+    least_lo = block_min_key(least_lo, red);
+    high_lo = ~block_min_key(high_lo, red);
+    least_hi = block_min_key(least_hi, red);
+    high_hi = ~block_min_key(high_hi, red);
+    if ((n_lo <= few || least_lo == high_lo) && (n_hi <= few || least_hi == high_hi)) {
+      lo = n_lo > few ? least_lo : lo;
+      hi = n_hi > few ? least_hi : hi | (((K)1 << rest) - 1);
+      rest = 0;
+    } else {
+      for (; rest > 0 && (n_lo > few || n_hi > few); rest = max(rest - 11, 0)) digit(q, live, rest);
+    }
   }
   if (t == 0) {
-    hi |= ((K)1 << rest) - 1;
     MadRange<K> z{};
+    if (rest == 0 && hi - lo >= 2 && !open0 && !open1) {
+      const K upper = hi--;
+      z.tied = 1;
+      ++lo;
+      z.scale = (float)kMadBins / (float)(MadKey<T>::val(upper) - MadKey<T>::val(lo));
+    }
+    hi |= ((K)1 << rest) - 1;
     if (open0) lo = 0;
     if (open1) hi = ((K)1 << kKeyBits) - 1;
     z.lo = lo;
     z.range = hi - lo;
     z.least2 = ~(K)0;
     const int bits = bit_length<K>(z.range);
-    z.shift = bits > 6 ? bits - 6 : 0;
+    z.shift = z.tied ? bits : bits > 6 ? bits - 6 : 0;
     st[s] = z;
   }
 }
@@ -681,8 +741,8 @@ __global__ __launch_bounds__(kMT) void k_mad_pivot(const T* __restrict__ planes,
 // counted, keys in it go to an LDS bin and to the wave's part of an LDS list (slots from a prefix sum
 // over the wave, no atomic), which the wave appends to the plane's buffer with one reservation when it fills
 // and at the end.  Bound: reading the
-// planes (137 us for seven of 4096^2, against 95 us for each of the radix select's three passes); what
-// stands above that is the prefix sums and bins.  A reservation for every few hundred keys of a wave made it
+// planes (104 us for seven of 4096^2, against 95 us for each of the radix select's three passes); what
+// stands above that is the prefix sums and bins.  A tied range has a form of its own, which counts the ends' keys too.  A reservation for every few hundred keys of a wave made it
 // 279 us: atomics on one address follow one another.
 template <class T, bool MASKED>
 __global__ __launch_bounds__(kT) void k_mad_scan(const T* __restrict__ planes, size_t plane, int w, Rect inc, Rect exc,
@@ -696,17 +756,17 @@ __global__ __launch_bounds__(kT) void k_mad_scan(const T* __restrict__ planes, s
   constexpr int kStage = 64 * G + 768;          // room for a large plane's share of a wave: one reservation a block
   __shared__ uint32_t h[kMadBins];
   __shared__ K stage[kT / 64][kStage];
-  __shared__ uint32_t counts[kT / 64], belows[kT / 64], base_all;
+  __shared__ uint32_t counts[kT / 64], belows[kT / 64], ends[2][kT / 64], base_all;
   const int s = blockIdx.y;
   MadRange<K>* S = st + s;
   const K lo = S->lo, range = S->range;
-  const uint32_t shift = S->shift;
+  const uint32_t shift = S->shift, tied = S->tied;
   K* out = aside + (size_t)s * room;
   if (threadIdx.x < kMadBins) h[threadIdx.x] = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63;
   K* mine = stage[threadIdx.x >> 6];
-  uint32_t below = 0;
+  uint32_t below = 0, at_lo = 0, at_hi = 0;
   int n = 0;  // keys in the wave's part, the same in all its lanes
   auto flush = [&] {
     __builtin_amdgcn_wave_barrier();  // the other lanes' LDS writes precede the reads below (one wave: in order)
@@ -718,103 +778,133 @@ __global__ __launch_bounds__(kT) void k_mad_scan(const T* __restrict__ planes, s
     n = 0;
     __builtin_amdgcn_wave_barrier();
   };
-  // `live`: which of the lane's keys are noise pixels; every lane of a wave takes every group
-  auto take = [&](const K (&key)[G], uint32_t live) {
-    uint32_t in = 0;
-#pragma unroll
-    for (int k = 0; k < G; ++k) {
-      below += (live >> k) & (key[k] < lo ? 1u : 0u);
-      in |= key[k] - lo <= range ? 1u << k : 0u;
-    }
-    in &= live;
-    uint32_t at = __popc(in);
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t v = __shfl_up(at, o, 64);
-      if (lane >= o) at += v;
-    }
-    const int total = __builtin_amdgcn_readlane((int)at, 63);
-    if (total == 0) return;
-    at += (uint32_t)n - __popc(in);
-#pragma unroll
-    for (int k = 0; k < G; ++k) {
-      if (!((in >> k) & 1)) continue;
-      atomicAdd(&h[(uint32_t)((key[k] - lo) >> shift)], 1u);
-      mine[at + __popc(in & ((1u << k) - 1))] = key[k];
-    }
-    if (shift != 0) n += total;  // otherwise a bin is one key and the bins say all
-    if (n > kStage - 64 * G) flush();
-  };
-  const T* x = planes + (size_t)s * plane;
-  const size_t thr = blockIdx.x * (size_t)kT + threadIdx.x, nthr = (size_t)gridDim.x * kT;
-  K key[G];
-  if constexpr (!MASKED) {
-    struct alignas(16) Vec {
-      T a[V];
-    };
-    const size_t nv = (reinterpret_cast<uintptr_t>(x) & 15) == 0 ? plane / V : 0;
-    const Vec* xv = reinterpret_cast<const Vec*>(x);
-    for (size_t i0 = thr - lane; i0 < nv; i0 += 2 * nthr) {  // the wave's first vector
-      uint32_t live = 0;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const size_t i = i0 + u * nthr + lane;
-        const Vec v = xv[min(i, nv - 1)];
-        live |= i < nv ? ((1u << V) - 1) << (u * V) : 0u;
-#pragma unroll
-        for (int k = 0; k < V; ++k) key[u * V + k] = MadKey<T>::key(v.a[k]);
-      }
-      take(key, live);
-    }
-    for (size_t i0 = nv * V + thr - lane; i0 < plane; i0 += G * nthr) {
-      uint32_t live = 0;
+  const T low = MadKey<T>::val(lo);
+  const float scale = S->scale;
+  const auto pass = [&](auto tc) {
+    constexpr bool TIED = decltype(tc)::value;
+    // `live`: which of the lane's keys are noise pixels; every lane of a wave takes every group
+    auto take = [&](const K (&key)[G], uint32_t live) {
+      uint32_t in = 0;
 #pragma unroll
       for (int k = 0; k < G; ++k) {
-        const size_t i = i0 + k * nthr + lane;
-        key[k] = MadKey<T>::key(x[min(i, plane - 1)]);
-        live |= i < plane ? 1u << k : 0u;
+        below += (live >> k) & (key[k] < lo ? 1u : 0u);
+        in |= key[k] - lo <= range ? 1u << k : 0u;
       }
-      take(key, live);
-    }
-  } else {
-    // a wave takes two rows by G / 2 columns a lane: no division per pixel
-    const int rstep = (int)(nthr >> 6);
-    for (int r = inc.r0 + (int)(thr >> 6); r < inc.r1; r += 2 * rstep) {
-      for (int c0 = inc.c0 + lane; c0 - lane < inc.c1; c0 += 32 * G) {
+      in &= live;
+      if constexpr (TIED) {
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+          at_lo += (live >> k) & (key[k] == lo - 1 ? 1u : 0u);
+          at_hi += (live >> k) & (key[k] == lo + range + 1 ? 1u : 0u);
+        }
+      }
+      uint32_t at = __popc(in);
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t v = __shfl_up(at, o, 64);
+        if (lane >= o) at += v;
+      }
+      const int total = __builtin_amdgcn_readlane((int)at, 63);
+      if (total == 0) return;
+      at += (uint32_t)n - __popc(in);
+#pragma unroll
+      for (int k = 0; k < G; ++k) {
+        if (!((in >> k) & 1)) continue;
+        if constexpr (TIED)
+          atomicAdd(&h[tied_bin<T>(key[k], low, scale)], 1u);
+        else
+          atomicAdd(&h[(uint32_t)((key[k] - lo) >> shift)], 1u);
+        mine[at + __popc(in & ((1u << k) - 1))] = key[k];
+      }
+      if (shift != 0) n += total;  // otherwise a bin is one key and the bins say all
+      if (n > kStage - 64 * G) flush();
+    };
+    const T* x = planes + (size_t)s * plane;
+    const size_t thr = blockIdx.x * (size_t)kT + threadIdx.x, nthr = (size_t)gridDim.x * kT;
+    K key[G];
+    if constexpr (!MASKED) {
+      struct alignas(16) Vec {
+        T a[V];
+      };
+      const size_t nv = (reinterpret_cast<uintptr_t>(x) & 15) == 0 ? plane / V : 0;
+      const Vec* xv = reinterpret_cast<const Vec*>(x);
+      for (size_t i0 = thr - lane; i0 < nv; i0 += 2 * nthr) {  // the wave's first vector
         uint32_t live = 0;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const int y = r + u * rstep;
-          const T* row = x + (size_t)min(y, inc.r1 - 1) * w;
-          const bool cut = y >= exc.r0 && y < exc.r1;
+          const size_t i = i0 + u * nthr + lane;
+          const Vec v = xv[min(i, nv - 1)];
+          live |= i < nv ? ((1u << V) - 1) << (u * V) : 0u;
 #pragma unroll
-          for (int k = 0; k < G / 2; ++k) {
-            const int c = c0 + 64 * k;
-            key[u * (G / 2) + k] = MadKey<T>::key(row[min(c, inc.c1 - 1)]);
-            if (y < inc.r1 && c < inc.c1 && !(cut && c >= exc.c0 && c < exc.c1)) live |= 1u << (u * (G / 2) + k);
-          }
+          for (int k = 0; k < V; ++k) key[u * V + k] = MadKey<T>::key(v.a[k]);
         }
         take(key, live);
       }
+      for (size_t i0 = nv * V + thr - lane; i0 < plane; i0 += G * nthr) {
+        uint32_t live = 0;
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+          const size_t i = i0 + k * nthr + lane;
+          key[k] = MadKey<T>::key(x[min(i, plane - 1)]);
+          live |= i < plane ? 1u << k : 0u;
+        }
+        take(key, live);
+      }
+    } else {
+      // a wave takes two rows by G / 2 columns a lane: no division per pixel
+      const int rstep = (int)(nthr >> 6);
+      for (int r = inc.r0 + (int)(thr >> 6); r < inc.r1; r += 2 * rstep) {
+        for (int c0 = inc.c0 + lane; c0 - lane < inc.c1; c0 += 32 * G) {
+          uint32_t live = 0;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int y = r + u * rstep;
+            const T* row = x + (size_t)min(y, inc.r1 - 1) * w;
+            const bool cut = y >= exc.r0 && y < exc.r1;
+#pragma unroll
+            for (int k = 0; k < G / 2; ++k) {
+              const int c = c0 + 64 * k;
+              key[u * (G / 2) + k] = MadKey<T>::key(row[min(c, inc.c1 - 1)]);
+              if (y < inc.r1 && c < inc.c1 && !(cut && c >= exc.c0 && c < exc.c1)) live |= 1u << (u * (G / 2) + k);
+            }
+          }
+          take(key, live);
+        }
+      }
     }
-  }
+  };
+  tied ? pass(std::true_type{}) : pass(std::false_type{});
   // the block's remainder in one reservation: atomics on one address cost more than the copy
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o, 64);
+  if (tied) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      at_lo += __shfl_xor(at_lo, o, 64);
+      at_hi += __shfl_xor(at_hi, o, 64);
+    }
+  }
   if (lane == 0) {
     counts[threadIdx.x >> 6] = (uint32_t)n;
     belows[threadIdx.x >> 6] = below;
+    ends[0][threadIdx.x >> 6] = at_lo;
+    ends[1][threadIdx.x >> 6] = at_hi;
   }
   __syncthreads();
-  uint32_t before = 0, all = 0, low = 0;
+  uint32_t before = 0, all = 0, less = 0;
   for (int k = 0; k < kT / 64; ++k) {
     before += k < (int)(threadIdx.x >> 6) ? counts[k] : 0;
     all += counts[k];
-    low += belows[k];
+    less += belows[k];
   }
   if (threadIdx.x == 0) {
     base_all = all ? atomicAdd(&S->n, all) : 0;
-    if (low) atomicAdd(&S->below, low);
+    if (less) atomicAdd(&S->below, less);
+  }
+  if (tied && threadIdx.x < 2) {
+    uint32_t v = 0;
+    for (int k = 0; k < kT / 64; ++k) v += ends[threadIdx.x][k];
+    if (v) atomicAdd(threadIdx.x ? &S->at_hi : &S->at_lo, v);
   }
   if (threadIdx.x < kMadBins && h[threadIdx.x])
     atomicAdd(&hist[(size_t)s * kMadBins + threadIdx.x], h[threadIdx.x]);
@@ -832,11 +922,13 @@ __device__ __forceinline__ void load_bins(uint32_t* h, const uint32_t* __restric
 }
 
 // Large planes: the keys of the median's bin and the least key of its successor's, by many blocks.
-template <class K>
-__global__ __launch_bounds__(kMT) void k_mad_collect(uint32_t count, MadRange<K>* __restrict__ st,
-                                                     const uint32_t* __restrict__ hist, const K* __restrict__ aside,
-                                                     size_t room, K* __restrict__ lists, size_t list_room,
+template <class T>
+__global__ __launch_bounds__(kMT) void k_mad_collect(uint32_t count, MadRange<typename MadKey<T>::K>* __restrict__ st,
+                                                     const uint32_t* __restrict__ hist,
+                                                     const typename MadKey<T>::K* __restrict__ aside, size_t room,
+                                                     typename MadKey<T>::K* __restrict__ lists, size_t list_room,
                                                      const int* pred) {
+  using K = typename MadKey<T>::K;
   if (pred_off(pred)) return;
   __shared__ uint32_t h[kBins];
   __shared__ BinScratch scratch;
@@ -846,7 +938,9 @@ __global__ __launch_bounds__(kMT) void k_mad_collect(uint32_t count, MadRange<K>
   const int s = blockIdx.y, t = threadIdx.x;
   MadRange<K>* S = st + s;
   const K lo = S->lo;
-  const uint32_t shift = S->shift, below = S->below, n = S->n, k = (count - 1) / 2;
+  const uint32_t shift = S->shift, tied = S->tied, below = S->below, n = S->n, k = (count - 1) / 2;
+  const T low = MadKey<T>::val(lo);
+  const float scale = S->scale;
   if (shift == 0 || n > room || k < below) return;
   load_bins(h, hist, s);
   BinHit b, b2;  // of ranks in the range; k_mad_pick finds out if they are not
@@ -866,7 +960,7 @@ __global__ __launch_bounds__(kMT) void k_mad_collect(uint32_t count, MadRange<K>
 #pragma unroll
     for (int e = 0; e < V; ++e) {
       if (i >= nv || i * V + e >= n) break;
-      const int bin = (int)((v.a[e] - lo) >> shift);
+      const int bin = tied ? tied_bin<T>(v.a[e], low, scale) : (int)((v.a[e] - lo) >> shift);
       if (bin == b.bin)
         stage[atomicAdd(&n_stage, 1u)] = v.a[e];
       else if (bin == b2.bin)
@@ -884,9 +978,10 @@ __global__ __launch_bounds__(kMT) void k_mad_collect(uint32_t count, MadRange<K>
   if (t == 0 && least2 != ~(K)0) atomicMin(&S->least2, least2);
 }
 
-// The median's rank in the bins, then digits of 11 bits of its bin's keys: from the list that
-// k_mad_collect left (lists, large planes), from the keys set aside, or from the plane where the range
-// missed the rank or its keys found no room.
+// The median's rank in the bins, then digits of 11 bits of its bin's keys: from the list that k_mad_collect left
+// (lists, large planes), from the keys set aside (the bin's gathered in LDS first where many digits are to come and
+// they fit), or from the plane where the range missed the rank or its keys found no room.  A rank on a tied range's end needs no digits, nor
+// does a tied range's bin of one value.
 template <class T, bool MASKED>
 __global__ __launch_bounds__(kMT) void k_mad_pick(const T* __restrict__ planes, size_t plane, int w, Rect inc, Rect exc,
                                                   uint32_t count,
@@ -897,69 +992,154 @@ __global__ __launch_bounds__(kMT) void k_mad_pick(const T* __restrict__ planes, 
                                                   double* __restrict__ thr, const int* pred) {
   using K = typename MadKey<T>::K;
   if (pred_off(pred)) return;
+  constexpr uint32_t kGather = 2048;
   __shared__ uint32_t h[kBins];
   __shared__ BinScratch scratch;
   __shared__ K red[kMT / 64];
+  __shared__ K gathered[kGather];
+  __shared__ uint32_t n_gathered;
   const int s = blockIdx.x, t = threadIdx.x;
   const T* x = planes + (size_t)s * plane;
   const MadRange<K> S = st[s];
+  const K* const mine = aside + (size_t)s * room;
   const bool even = (count & 1) == 0;
-  const uint32_t k = (count - 1) / 2;
+  const uint32_t k = (count - 1) / 2, k2 = k + (even ? 1 : 0);
   load_bins(h, hist, s);
   const BinHit last = find_bin(h, 0xffffffffu, scratch);
-  const uint32_t total = last.before + last.count;
-  const bool found = k >= S.below && k - S.below + (even ? 1 : 0) < total;
-  const bool listed = found && lists && S.n <= room && S.listed <= list_room;
+  // f(key) of n keys, eight loads in flight
+  const auto over = [&](const K* from, uint32_t n, auto f) {
+    for (uint32_t i0 = t; i0 < n; i0 += 8 * kMT) {
+      K q[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) q[u] = from[min(i0 + u * kMT, n - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (i0 + u * kMT < n) f(q[u]);
+    }
+  };
+  // ranks of the range: S.below to above; S.at_lo ranks before and S.at_hi after are a tied range's ends
+  const uint32_t above = S.below + last.before + last.count, end = above + S.at_hi;
+  if (k2 < end && (k >= above || (k < S.below && k >= S.below - S.at_lo))) {
+    const K v = k < S.below ? S.lo - 1 : S.lo + S.range + 1;
+    K hi = v;
+    if (k < S.below && k2 >= S.below) {  // the successor is the range's least key, or its upper end
+      K m = S.lo + S.range + 1;
+      if (above != S.below) {
+        if (S.shift == 0)
+          m = S.lo;  // the range is one key
+        else if (S.n <= room)
+          over(mine, S.n, [&](K key) { m = min(m, key); });
+        else
+          each_noise_key<T, MASKED>(x, plane, w, inc, exc, t, kMT, [&](K key) { m = key > v ? min(m, key) : m; });
+      }
+      hi = block_min_key(m, red);
+    }
+    if (t == 0) thr[s] = mad_of<T>(v, hi, even);
+    return;
+  }
+  const bool found = k >= S.below && k < above && k2 < end;
+  const bool set_aside = found && S.n <= room;
+  const bool listed = set_aside && lists && S.listed <= list_room;
+  const bool by_value = found && S.tied && S.shift != 0;
   // key - lo of every key that can be the median, and of at least all keys of the range up to its successor
   const K lo = found ? S.lo : 0;
+  const T low = MadKey<T>::val(S.lo);
   K v = 0;
   K least2 = ~(K)0;
   uint32_t rank = k, equal = 0;
   int top = 8 * (int)sizeof(K) - 1;
+  int bin = 0;
+  bool only_bin = listed;  // the keys are the median's bin's, the successor's least is least2
+  const K* from = listed ? lists + (size_t)s * list_room : mine;
+  uint32_t n_from = listed ? S.listed : S.n;
   if (found) {
     BinHit b, b2;
-    find_bins(h, k - S.below, k - S.below + (even ? 1 : 0), scratch, &b, &b2);
-    v = (K)b.bin << S.shift;
+    find_bins(h, k - S.below, k2 - S.below, scratch, &b, &b2);
+    bin = b.bin;
+    if (!S.tied) v = (K)bin << S.shift;
     rank = k - S.below - b.before;
     equal = b.count;
     top = (int)S.shift;
-    if (top == 0)
-      least2 = (K)b2.bin;
-    else if (listed && b2.bin != b.bin)
+    const auto bin_of = [&](K key) { return by_value ? tied_bin<T>(key, low, S.scale) : (int)((key - lo) >> S.shift); };
+    if (set_aside && !listed && top > 0 && equal <= kGather && (by_value || sizeof(K) == 8)) {
+      if (t == 0) n_gathered = 0;
+      __syncthreads();
+      K m = ~(K)0;
+      over(mine, S.n, [&](K key) {
+        const int at = bin_of(key);
+        if (at == bin)
+          gathered[atomicAdd(&n_gathered, 1u)] = key;
+        else if (at == b2.bin)
+          m = min(m, key);
+      });
+      least2 = block_min_key(m, red) - lo;
+      only_bin = true;
+      from = gathered;
+      n_from = equal;
+    } else if (listed && b2.bin != bin) {
       least2 = S.least2 - lo;
+    } else if (by_value && !listed) {
+      // many keys in the bin: one value, or digits
+      K m = ~(K)0, high = ~(K)0;  // the least key and the complement of the greatest
+      const auto ends = [&](K key) {
+        if (key < S.lo || key - S.lo > S.range || bin_of(key) != bin) return;
+        m = min(m, key);
+        high = min(high, ~key);
+      };
+      if (set_aside)
+        over(mine, S.n, ends);
+      else
+        each_noise_key<T, MASKED>(x, plane, w, inc, exc, t, kMT, ends);
+      m = block_min_key(m, red);
+      high = ~block_min_key(high, red);
+      if (m == high) {
+        v = m - lo;
+        top = 0;
+      }
+    }
+    if (k2 >= above)
+      least2 = S.range + 1;
+    else if (S.shift == 0)
+      least2 = (K)b2.bin;
   }
   auto each = [&](auto f) {
-    if (listed || (found && S.n <= room)) {
-      const K* from = listed ? lists + (size_t)s * list_room : aside + (size_t)s * room;
-      const uint32_t n = listed ? S.listed : S.n;
-      for (uint32_t i0 = t; i0 < n; i0 += 8 * kMT) {
-        K q[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) q[u] = from[min(i0 + u * kMT, n - 1)];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (i0 + u * kMT < n) f(q[u] - lo);
-      }
-    } else {
+    if (only_bin || set_aside)
+      over(from, n_from, [&](K key) { f(key - lo); });
+    else
       each_noise_key<T, MASKED>(x, plane, w, inc, exc, t, kMT, [&](K key) {
         if (!found || key - lo <= S.range) f(key - lo);
       });
+  };
+  const auto digits = [&](auto tc) {
+    while (top > 0) {
+      const int nd = min(11, top), shift = top - nd;
+      clear_bins(h);
+      __syncthreads();
+      each([&](K rel) {
+        if ((rel >> top) != (v >> top)) return;
+        const uint32_t d = (uint32_t)(rel >> shift) & ((1u << nd) - 1);
+        if constexpr (decltype(tc)::value) {
+          if (tied_bin<T>(rel + lo, low, S.scale) != bin) return;
+          // one addition for all lanes with the first one's digit: equal keys would be added one after the other
+          const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
+          const unsigned long long same = __ballot(d == first);
+          if (d != first)
+            atomicAdd(&h[d], 1u);
+          else if ((int)(t & 63) == __ffsll(same) - 1)
+            atomicAdd(&h[d], (uint32_t)__popcll(same));
+        } else {
+          atomicAdd(&h[d], 1u);
+        }
+      });
+      __syncthreads();
+      const BinHit b = find_bin(h, rank, scratch);
+      v |= (K)b.bin << shift;
+      rank -= b.before;
+      equal = b.count;
+      top = shift;
     }
   };
-  while (top > 0) {
-    const int nd = min(11, top), shift = top - nd;
-    clear_bins(h);
-    __syncthreads();
-    each([&](K rel) {
-      if ((rel >> top) == (v >> top)) atomicAdd(&h[(uint32_t)(rel >> shift) & ((1u << nd) - 1)], 1u);
-    });
-    __syncthreads();
-    const BinHit b = find_bin(h, rank, scratch);
-    v |= (K)b.bin << shift;
-    rank -= b.before;
-    equal = b.count;
-    top = shift;
-  }
+  by_value && !only_bin ? digits(std::true_type{}) : digits(std::false_type{});
   K hi = v;
   if (even && rank + 1 >= equal) {
     K m = least2;
@@ -1815,8 +1995,10 @@ void mad_thresholds_noalloc(const float* planes, int S, int h, int w, const Nois
 // The sample has 8192 keys below 2^20 noise pixels and 16384 above: a range of 8.8 and 6.3% of the
 // plane (32768: 4.4%, 35 instead of 20 us in k_mad_pivot for 4 us less in k_mad_scan).  From 2^20 pixels on the
 // median's bin is collected by many blocks: one block alone needs 45 us to look at what a 4096^2 plane sets
-// aside.  Seven 4096^2 planes take 190 us (340 us with the radix select), five 500^2 planes with an edge
-// mask 39 us (50 us), four 256^2 planes 26 us (33 us).
+// aside.  Seven 4096^2 planes take 160 us (285 us with the radix select), five 500^2 planes with an edge
+// mask 37 us (50 us), four 256^2 planes 26 us (33 us).  Seven planes with many equal keys (48 to 52% zeros, two values, 30
+// whole numbers, values within 1e-5 of one) take 132 to 260 us (277 to 810 us with the radix select; 1.1 to 22 ms with the
+// ends in the range and one block selecting from the plane), float64 ones 260 to 450 us (1.2 to 1.4 ms; 2.1 to 47 ms).
 template <class T, bool MASKED>
 static void mad_thresholds_t(const T* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
                              const int* pred, hipStream_t st) {
@@ -1849,7 +2031,7 @@ static void mad_thresholds_t(const T* planes, int S, int h, int w, const NoiseMa
                      aside, room, pred);
   PMS_LAUNCH_CHECK();
   if (large) {
-    hipLaunchKernelGGL((k_mad_collect<K>), dim3(32, S), dim3(kMT), 0, st, n, range, (const uint32_t*)hist,
+    hipLaunchKernelGGL((k_mad_collect<T>), dim3(32, S), dim3(kMT), 0, st, n, range, (const uint32_t*)hist,
                        (const K*)aside, room, lists, list_room, pred);
     PMS_LAUNCH_CHECK();
   }
