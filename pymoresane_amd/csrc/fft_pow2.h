@@ -21,8 +21,9 @@
 //   3. rows c2r   : per kept row: Hermitian pre-twiddle into a P/2-point
 //                   inverse FFT, scale 1/P^2, write the N kept columns.
 // Twiddles come from a device table exp(-2 pi i k / 2^14) computed on the
-// host in double precision; in-butterfly powers are formed by a balanced
-// product tree from one table value.
+// host in double precision (float64 entries from 80-bit angles); float32
+// in-butterfly powers are formed by a balanced product tree from one table
+// value, float64 ones by at most one product of table values (see Twiddles).
 #pragma once
 
 #include <algorithm>
@@ -92,15 +93,15 @@ __device__ __forceinline__ int pad(int i) { return i + (i >> 5); }
 // cos / sin of 2 pi j / 32 for j in [0, 16)
 struct Roots32 {
   static constexpr double c[16] = {
-      1.0, 0.98078528040323043, 0.92387953251128674, 0.83146961230254524,
-      0.70710678118654757, 0.55557023301960229, 0.38268343236508984, 0.19509032201612833,
-      0.0, -0.19509032201612819, -0.38268343236508973, -0.55557023301960196,
-      -0.70710678118654746, -0.83146961230254535, -0.92387953251128674, -0.98078528040323043};
+      1.0, 0.9807852804032304, 0.9238795325112867, 0.8314696123025452,
+      0.7071067811865476, 0.5555702330196022, 0.3826834323650898, 0.19509032201612828,
+      0.0, -0.19509032201612828, -0.3826834323650898, -0.5555702330196022,
+      -0.7071067811865476, -0.8314696123025452, -0.9238795325112867, -0.9807852804032304};
   static constexpr double s[16] = {
-      0.0, 0.19509032201612825, 0.38268343236508978, 0.55557023301960218,
-      0.70710678118654746, 0.83146961230254524, 0.92387953251128674, 0.98078528040323043,
-      1.0, 0.98078528040323043, 0.92387953251128674, 0.83146961230254546,
-      0.70710678118654757, 0.55557023301960218, 0.38268343236508989, 0.19509032201612861};
+      0.0, 0.19509032201612828, 0.3826834323650898, 0.5555702330196022,
+      0.7071067811865476, 0.8314696123025452, 0.9238795325112867, 0.9807852804032304,
+      1.0, 0.9807852804032304, 0.9238795325112867, 0.8314696123025452,
+      0.7071067811865476, 0.5555702330196022, 0.3826834323650898, 0.19509032201612828};
 };
 
 // t = o * exp(DIR * 2 pi i k / R), k < R/2 known at compile time after unrolling
@@ -138,14 +139,41 @@ struct Dft<C, 1, DIR> {
   __device__ __forceinline__ static void run(C (&)[1]) {}
 };
 
-// powers w^0 .. w^(R-1) by a balanced product tree
+// The twiddles w^1 .. w^(R-1) of a butterfly, w = tw[i].  float32: all from w by a balanced product tree.
+// float64: a power formed by squaring errs by its exponent's half in units of w's error, so w^1 .. w^3, w^4, w^8
+// and w^12 come from the table and the others are one product of those.
 template <class C, int R>
-__device__ __forceinline__ void powers(C w, C (&wk)[R]) {
-  wk[0] = mk<C>(1, 0);
-  if (R > 1) wk[1] = w;
+struct Twiddles {
+  static constexpr bool kTree = sizeof(Rl<C>) == 4;
+  static constexpr int N = kTree || R == 2 ? 1 : R == 4 ? 3 : R == 8 ? 4 : 6;
+  static constexpr int exponent(int j) { return j < 4 ? j + 1 : 4 * (j - 2); }
+  C w[N];
+  __device__ __forceinline__ void load(const C* __restrict__ tw, int i) {
 #pragma unroll
-  for (int k = 2; k < R; ++k) wk[k] = cmul(wk[k >> 1], wk[k - (k >> 1)]);
-}
+    for (int j = 0; j < N; ++j) w[j] = tw[exponent(j) * i];
+  }
+  __device__ __forceinline__ void none() {
+#pragma unroll
+    for (int j = 0; j < N; ++j) w[j] = mk<C>(1, 0);
+  }
+  template <bool CONJ>
+  __device__ __forceinline__ void powers(C (&wk)[R]) const {
+    const auto at = [&](int j) { return CONJ ? cconj(w[j]) : w[j]; };
+    wk[0] = mk<C>(1, 0);
+    wk[1] = at(0);
+#pragma unroll
+    for (int k = 2; k < R; ++k) {
+      if (kTree)
+        wk[k] = cmul(wk[k >> 1], wk[k - (k >> 1)]);
+      else if (k < 4)
+        wk[k] = at(k - 1);
+      else if (k % 4 == 0)
+        wk[k] = at(k / 4 + 2);
+      else
+        wk[k] = cmul(wk[k & ~3], wk[k & 3]);
+    }
+  }
+};
 
 // One in-place radix-R stage over an LDS array of length L, sub-transform
 // length Ls (M = Ls/R).  Forward = decimation in frequency; inverse runs the
@@ -167,14 +195,18 @@ __device__ __forceinline__ void fft_stage(C* sm, int L, int Ls, int lt, int nthr
       Dft<C, R, -1>::run(x);
       if (M > 1) {
         C wk[R];
-        powers<C, R>(tw[n * tw_step], wk);
+        Twiddles<C, R> w;
+        w.load(tw, n * tw_step);
+        w.template powers<false>(wk);
 #pragma unroll
         for (int k = 1; k < R; ++k) x[k] = cmul(x[k], wk[k]);
       }
     } else {
       if (M > 1) {
         C wk[R];
-        powers<C, R>(cconj(tw[n * tw_step]), wk);
+        Twiddles<C, R> w;
+        w.load(tw, n * tw_step);
+        w.template powers<true>(wk);
 #pragma unroll
         for (int k = 1; k < R; ++k) x[k] = cmul(x[k], wk[k]);
       }
@@ -231,7 +263,9 @@ __device__ __forceinline__ void stage0_load(C* sm, int L, int lt, int nthr, cons
         Dft<C, R0, -1>::run(x[u]);
         if (M0 > 1) {
           C wk[R0];
-          powers<C, R0>(tw[n * step], wk);
+          Twiddles<C, R0> w;
+          w.load(tw, n * step);
+          w.template powers<false>(wk);
 #pragma unroll
           for (int k = 1; k < R0; ++k) x[u][k] = cmul(x[u][k], wk[k]);
         }
@@ -389,7 +423,7 @@ struct StageTw {
   using Pl = Plan<LG>;
   static constexpr int PER = Pl::NBF > 0 ? (Pl::NBF + NT - 1) / NT : 1;
   static constexpr int NI = Pl::NS > 1 ? Pl::NS : 1;
-  C w[NI][PER];
+  Twiddles<C, 16> w[NI][PER];
   __device__ __forceinline__ void load(int lt, const C* __restrict__ gtw) {
     static_for<1, Pl::NS>([&](auto ic) {
       constexpr int I = decltype(ic)::value;
@@ -399,7 +433,10 @@ struct StageTw {
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
           const int b = lt + j * NT;
-          w[I][j] = (b < Pl::NBF) ? gtw[(b & (M - 1)) * (kFftMaxLen / Ls)] : mk<C>(1, 0);
+          if (b < Pl::NBF)
+            w[I][j].load(gtw, (b & (M - 1)) * (kFftMaxLen / Ls));
+          else
+            w[I][j].none();
         }
       }
     });
@@ -428,14 +465,14 @@ __device__ __forceinline__ void stage16(C* sm, int lt, const StageTw<C, LG, NT>&
       Dft<C, 16, -1>::run(x);
       if constexpr (M > 1) {
         C wk[16];
-        powers<C, 16>(tw.w[I][j], wk);
+        tw.w[I][j].template powers<false>(wk);
 #pragma unroll
         for (int k = 1; k < 16; ++k) x[k] = cmul(x[k], wk[k]);
       }
     } else {
       if constexpr (M > 1) {
         C wk[16];
-        powers<C, 16>(cconj(tw.w[I][j]), wk);
+        tw.w[I][j].template powers<true>(wk);
 #pragma unroll
         for (int k = 1; k < 16; ++k) x[k] = cmul(x[k], wk[k]);
       }
@@ -454,7 +491,7 @@ struct Stage0 {
   static constexpr int U = (Pl::M0 + NT - 1) / NT;
   static constexpr int KL = LIN ? (Pl::R0 / 2 > 0 ? Pl::R0 / 2 : 1) : Pl::R0;
   C x[U][Pl::R0];
-  C w[U];
+  Twiddles<C, Pl::R0> w[U];
   template <class Get>
   __device__ __forceinline__ void load(int lt, const C* __restrict__ gtw, Get get) {
 #pragma unroll
@@ -463,7 +500,12 @@ struct Stage0 {
       const bool ok = n < Pl::M0;
 #pragma unroll
       for (int k = 0; k < Pl::R0; ++k) x[u][k] = (ok && k < KL) ? get(n + k * Pl::M0) : mk<C>(0, 0);
-      if constexpr (Pl::M0 > 1) w[u] = ok ? gtw[n * (kFftMaxLen / Pl::L)] : mk<C>(1, 0);
+      if constexpr (Pl::M0 > 1) {
+        if (ok)
+          w[u].load(gtw, n * (kFftMaxLen / Pl::L));
+        else
+          w[u].none();
+      }
     }
   }
   // forward stage 0 from registers into LDS
@@ -475,7 +517,7 @@ struct Stage0 {
       Dft<C, Pl::R0, -1>::run(x[u]);
       if constexpr (Pl::M0 > 1) {
         C wk[Pl::R0];
-        powers<C, Pl::R0>(w[u], wk);
+        w[u].template powers<false>(wk);
 #pragma unroll
         for (int k = 1; k < Pl::R0; ++k) x[u][k] = cmul(x[u][k], wk[k]);
       }
@@ -497,7 +539,7 @@ struct Stage0 {
       for (int k = 0; k < Pl::R0; ++k) y[k] = s0[padc(k * Pl::M0)];
       if constexpr (Pl::M0 > 1) {
         C wk[Pl::R0];
-        powers<C, Pl::R0>(cconj(w[u]), wk);
+        w[u].template powers<true>(wk);
 #pragma unroll
         for (int k = 1; k < Pl::R0; ++k) y[k] = cmul(y[k], wk[k]);
       }
@@ -756,7 +798,10 @@ __global__ __launch_bounds__((RowCfg<C, PG, LIN>::T)) void k_conv_c2r(C2rBatch<C
 #pragma unroll
     for (int u = 0; u < Stage0<C, LG, NT, LIN>::U; ++u) {
       const int n = lt + u * NT;
-      s0.w[u] = (n < Plan<LG>::M0) ? tw[n * (kFftMaxLen / L)] : mk<C>(1, 0);
+      if (n < Plan<LG>::M0)
+        s0.w[u].load(tw, n * (kFftMaxLen / L));
+      else
+        s0.w[u].none();
     }
   }
   // Hermitian pre-twiddle: Z'[k] = (X[k] + conj X[L-k]) + i (X[k] - conj X[L-k]) conj(w^k), stored
@@ -921,7 +966,9 @@ struct Pow2Tables {
     if (ptr[device]) return ptr[device];
     std::vector<C> h(kFftMaxLen);
     for (int k = 0; k < kFftMaxLen; ++k) {
-      const double a = -2.0 * M_PI * (double)k / (double)kFftMaxLen;
+      // float64 entries from a wider angle, whose rounding would otherwise reach them
+      using A = std::conditional_t<sizeof(Rl<C>) == 8, long double, double>;
+      const A a = -2 * (A)M_PIl * (A)k / (A)kFftMaxLen;
       h[k].x = (Rl<C>)std::cos(a);
       h[k].y = (Rl<C>)std::sin(a);
     }
