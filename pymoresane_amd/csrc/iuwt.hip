@@ -1235,7 +1235,10 @@ bool small2_applies(bool small, int h, int w, int s) {
 // 3000^2 180 -> 170 (147 -> 141), 4096^2 282 -> 285 (236 -> 237); pair (2,3): 1024^2 46 -> 38 (39 -> 33), 1600^2 76 -> 66
 // (53 -> 53), 2048^2 103 -> 98 (75 -> 76), 3000^2 170 -> 180 (141 -> 160); pair (4,5): 800^2 34 -> 43 (32 -> 30.5), 1024^2 38 -> 46
 // (33 -> 31), 1300^2 56 -> 77 (41 -> 51).
+// PMS_IUWT_SMALL_LAUNCH=0 keeps planes above 256^2 on the walks, and PMS_IUWT_DEC2 or PMS_IUWT_PAIR, when set, say how
+// those take the scales of a decomposition or a recomposition: no tiles then (all read per call).
 bool tile2_range(int h, int w, int s, int jobs, bool recomp) {
+  if (env_int("PMS_IUWT_SMALL_LAUNCH", 1) == 0 || getenv(recomp ? "PMS_IUWT_PAIR" : "PMS_IUWT_DEC2")) return false;
   const long px = (long)h * w * jobs;
   const int top = px <= 1L << 20 ? (recomp ? 4 : 2) : px <= 1L << 22 ? 2 : px <= 3L << 22 ? 0 : -1;
   return s <= top;
@@ -1376,9 +1379,9 @@ static void decompose_batch_impl(IuwtDecompJob* jobs, int count, int h, int w, b
     j.np = 0;
     smax = std::max(smax, j.scale_count);
   }
-  // detail scales in pairs from the finest up where a two-scale launch applies (1), or one scale per
-  // launch (0): PMS_IUWT_DEC2 when set, else the autotuner's record, else the default (the planes are
-  // identical either way)
+  // on the row walks, detail scales in pairs from the finest up where a two-scale launch applies (1), or one
+  // scale per launch (0): PMS_IUWT_DEC2 when set, else the autotuner's record, else the default (the planes
+  // are identical either way)
   const int fuse = getenv("PMS_IUWT_DEC2") ? env_int("PMS_IUWT_DEC2", kDec2Default)
                                            : (t_active ? t_active->pair : kDec2Default);
   std::vector<IuwtScaleCall> calls;
