@@ -285,9 +285,15 @@ int pms_fft_convolve(const float* in, int n, int p, const void* spectrum, float*
 }
 
 // ------------------------------------------------------------------- threshold
+// the median's scratch, then the partial maxima of thresholding: an estimate on one stream and a thresholding on
+// another may share a workspace
+static size_t maxima_offset(int n_planes, int h, int w) {
+  return (mad_work_bytes(n_planes, (size_t)h * w, sizeof(float)) + 255) / 256 * 256;
+}
+
 size_t pms_threshold_work_bytes(int n_planes, int h, int w) {
   if (n_planes <= 0 || h <= 0 || w <= 0) return 0;
-  return std::max(mad_work_bytes(n_planes, (size_t)h * w, sizeof(float)), (size_t)n_planes * 256 * sizeof(float));
+  return maxima_offset(n_planes, h, w) + (size_t)n_planes * 256 * sizeof(float);
 }
 
 int pms_estimate_threshold(const float* planes, int n_planes, int h, int w, int edge_excl, int int_excl,
@@ -320,7 +326,8 @@ int pms_apply_threshold(const float* planes, int n_planes, int h, int w, const d
                         double sigma_level, float* out, void* work, void* stream) {
   return guarded([&] {
     PMS_REQUIRE(planes && thresholds && out && work, "NULL buffer");
-    apply_threshold(planes, out, n_planes, h, w, thresholds, sigma_level, nullptr, (float*)work, nullptr, S(stream));
+    float* pmax = (float*)((char*)work + maxima_offset(n_planes, h, w));
+    apply_threshold(planes, out, n_planes, h, w, thresholds, sigma_level, nullptr, pmax, nullptr, S(stream));
   });
 }
 
