@@ -2118,8 +2118,9 @@ static size_t ext_labels_offset(int S, int h, int wd) {
   return ext_bits_offset(S, h, wd) + ext_round((size_t)S * h * ccl_words(wd) * sizeof(u64));
 }
 
+// The words and tiles of a plane and of its transpose differ in number: room for either, as one workspace may serve both.
 size_t extract_work_bytes(int S, int h, int w) {
-  return ext_labels_offset(S, h, w) + (size_t)S * h * w * sizeof(int);
+  return std::max(ext_labels_offset(S, h, w), ext_labels_offset(S, w, h)) + (size_t)S * h * w * sizeof(int);
 }
 
 template <class T>
