@@ -77,7 +77,7 @@ Geometry make_geometry(int n, int psf_n, const MoresaneParams& prm, int scale_co
 
 // byte sizes of the per-job device buffers
 struct JobSizes {
-  size_t s2, S_s2, mask, iuwt, N2, spec_sub, spec_full, fft, psf, ext, mad, partial, pmax;
+  size_t s2, S_s2, mask, iuwt, N2, spec_sub, spec_full, fft, psf, detect, partial, pmax;
   bool f64;
 };
 
@@ -137,7 +137,7 @@ class Job {
   Planes<float> f{};
   Planes<double> d{};
   uint8_t* M = nullptr;
-  void *mad_work = nullptr, *ext_work = nullptr;
+  void* detect_work = nullptr;  // scratch of the noise estimate and of the source extraction, one after the other
   double* partial = nullptr;
 };
 

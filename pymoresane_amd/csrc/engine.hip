@@ -574,8 +574,7 @@ static JobSizes job_sizes(const Geometry& g, int S) {
                     fft_spectrum_elems(g.p_sub), fft_spectrum_elems(g.p_full)}) *
           2 * e;
   z.psf = (size_t)g.psf_n * g.psf_n * e;
-  z.ext = extract_work_bytes(S, g.sub, g.sub);
-  z.mad = mad_work_bytes(S, s2, e);
+  z.detect = std::max(extract_work_bytes(S, g.sub, g.sub), mad_work_bytes(S, s2, e));
   const long dec_partials = g.f64 ? iuwt_decompose_partials_f64(g.sub, g.sub, S, 0)
                                   : iuwt_decompose_partials(g.sub, g.sub, S, 0);
   z.partial = (size_t)std::max<long>({dec_partials, (long)reduce_grid(N2) * 2, (long)reduce_grid(s2) * S, 4096L}) *
@@ -587,8 +586,8 @@ static JobSizes job_sizes(const Geometry& g, int S) {
 static bool fits(const JobSizes& need, const JobSizes& have) {
   return need.f64 == have.f64 && need.s2 <= have.s2 && need.S_s2 <= have.S_s2 && need.mask <= have.mask &&
          need.iuwt <= have.iuwt && need.N2 <= have.N2 && need.spec_sub <= have.spec_sub &&
-         need.spec_full <= have.spec_full && need.fft <= have.fft && need.psf <= have.psf && need.ext <= have.ext && need.mad <= have.mad &&
-         need.partial <= have.partial && need.pmax <= have.pmax;
+         need.spec_full <= have.spec_full && need.fft <= have.fft && need.psf <= have.psf &&
+         need.detect <= have.detect && need.partial <= have.partial && need.pmax <= have.pmax;
 }
 
 static JobSizes max_sizes(const JobSizes& a, const JobSizes& b) {
@@ -603,8 +602,7 @@ static JobSizes max_sizes(const JobSizes& a, const JobSizes& b) {
   z.spec_full = std::max(a.spec_full, b.spec_full);
   z.fft = std::max(a.fft, b.fft);
   z.psf = std::max(a.psf, b.psf);
-  z.ext = std::max(a.ext, b.ext);
-  z.mad = std::max(a.mad, b.mad);
+  z.detect = std::max(a.detect, b.detect);
   z.partial = std::max(a.partial, b.partial);
   z.pmax = std::max(a.pmax, b.pmax);
   return z;
@@ -613,7 +611,7 @@ static JobSizes max_sizes(const JobSizes& a, const JobSizes& b) {
 size_t job_footprint_bytes(const Geometry& g) {
   const JobSizes z = job_sizes(g, std::max(g.S, (int)std::log2((double)g.n) - 1));
   const size_t by_scale = z.N2;  // moresane_by_scale's private dirty copy
-  return z.s2 * 10 + z.S_s2 * 4 + z.mask + z.iuwt + z.N2 * 3 + z.spec_sub + z.spec_full + z.fft + z.psf + z.ext + z.mad +
+  return z.s2 * 10 + z.S_s2 * 4 + z.mask + z.iuwt + z.N2 * 3 + z.spec_sub + z.spec_full + z.fft + z.psf + z.detect +
          z.partial + z.pmax + by_scale + 64 * 8 + 64 * 4 + 12 * 256;
 }
 
@@ -686,8 +684,7 @@ bool Job::ensure(const Geometry& g, hipStream_t st) {
     else
       carve(f, z, arena_);
     M = (uint8_t*)arena_.alloc(z.mask);
-    mad_work = arena_.alloc(z.mad);
-    ext_work = arena_.alloc(z.ext);
+    detect_work = arena_.alloc(z.detect);
     partial = (double*)arena_.alloc(z.partial);
   };
   arena_.plan();
@@ -779,7 +776,7 @@ void Task::enqueue_pre_t(hipStream_t st) {
       if (spec.mask) {
         // decomposition of dirty_sub * mask[sub] replaces the thresholded one (main.py:283-285)
         decompose1<T>(B.dirty_sub, sub, g_.S, B.D, B.iuwt_work, st);
-        mad_thresholds(B.D, g_.S, sub, sub, nm_, scal_ + kThr, J.mad_work, nullptr, st);
+        mad_thresholds(B.D, g_.S, sub, sub, nm_, scal_ + kThr, J.detect_work, nullptr, st);
         window_copy(spec.mask, g_.n, g_.lo, g_.lo, sub, (const T*)nullptr, B.cbuf, st);
         window_copy(B.dirty_sub, sub, 0, 0, sub, B.cbuf, B.rec, st);
         decompose1<T>(B.rec, sub, g_.S, B.D, B.iuwt_work, st);
@@ -791,7 +788,7 @@ void Task::enqueue_pre_t(hipStream_t st) {
         // decomposition can index them by scale
         const int adj = scale_adjust_;
         source_extract(B.D + (size_t)adj * s2, max_scale_ - adj, sub, sub, spec.prm.tolerance, spec.prm.neg_comp,
-                       J.M + (size_t)adj * s2, B.E + (size_t)adj * s2, nullptr, J.ext_work, nullptr, st);
+                       J.M + (size_t)adj * s2, B.E + (size_t)adj * s2, nullptr, J.detect_work, nullptr, st);
       }
       break;
     case UPDATE:
@@ -838,7 +835,7 @@ void Task::enqueue_post_t(hipStream_t st) {
   switch (phase_) {
     case DECOMP:
       // MAD thresholds, thresholding with the edge mask and normalised maxima (main.py:278-300)
-      if (!spec.mask) mad_thresholds(B.D, g_.S, sub, sub, nm_, scal_ + kThr, J.mad_work, nullptr, st);
+      if (!spec.mask) mad_thresholds(B.D, g_.S, sub, sub, nm_, scal_ + kThr, J.detect_work, nullptr, st);
       apply_threshold(B.D, B.D, g_.S, sub, sub, scal_ + kThr, prm.sigma_level,
                       borders_.empty() ? nullptr : iflag_ + kBorders, B.pmax, nullptr, st);
       max_final(B.pmax, threshold_grid(s2), g_.S, (T*)nullptr, scal_ + kEnergy, scal_ + kNsm, nullptr, st);
