@@ -2009,6 +2009,10 @@ static void mad_thresholds_t(const T* planes, int S, int h, int w, const NoiseMa
   const Rect exc{nm.exc_r0, nm.exc_r1, nm.exc_c0, nm.exc_c1};
   const size_t area = (size_t)(inc.r1 - inc.r0) * (inc.c1 - inc.c0);
   const uint32_t n = (uint32_t)nm.count;
+  if constexpr (sizeof(T) == 4) {
+    // 32-bit pixel numbers end here; the counts are of the pixels left in, which check_mad bounds
+    if (area >= (size_t)1 << 32) return mad_thresholds_noalloc(planes, S, h, w, nm, thr, work, pred, st);
+  }
   PMS_REQUIRE(area < ((size_t)1 << 32), "plane too large for the median");
   if (area <= (size_t)kMadOne) {
     auto one = area <= (size_t)8 * kMT ? k_mad_one<T, MASKED, 8> : k_mad_one<T, MASKED, 32>;
