@@ -740,10 +740,10 @@ __global__ __launch_bounds__(kMT) void k_mad_pivot(const T* __restrict__ planes,
 // The pass over the planes, eight keys (four float64) a thread at a time: keys below the range are
 // counted, keys in it go to an LDS bin and to the wave's part of an LDS list (slots from a prefix sum
 // over the wave, no atomic), which the wave appends to the plane's buffer with one reservation when it fills
-// and at the end.  Bound: reading the
-// planes (104 us for seven of 4096^2, against 95 us for each of the radix select's three passes); what
-// stands above that is the prefix sums and bins.  A tied range has a form of its own, which counts the ends' keys too.  A reservation for every few hundred keys of a wave made it
-// 279 us: atomics on one address follow one another.
+// and at the end.  Bound: reading the planes (104 us for seven of 4096^2, against 95 us for each of the radix
+// select's three passes); what stands above that is the prefix sums and bins.  A reservation for every few
+// hundred keys of a wave made it 279 us: atomics on one address follow one another.  A tied range has a form
+// of its own, which counts the ends' keys too.
 template <class T, bool MASKED>
 __global__ __launch_bounds__(kT) void k_mad_scan(const T* __restrict__ planes, size_t plane, int w, Rect inc, Rect exc,
                                                  MadRange<typename MadKey<T>::K>* __restrict__ st,
@@ -979,9 +979,9 @@ __global__ __launch_bounds__(kMT) void k_mad_collect(uint32_t count, MadRange<ty
 }
 
 // The median's rank in the bins, then digits of 11 bits of its bin's keys: from the list that k_mad_collect left
-// (lists, large planes), from the keys set aside (the bin's gathered in LDS first where many digits are to come and
-// they fit), or from the plane where the range missed the rank or its keys found no room.  A rank on a tied range's end needs no digits, nor
-// does a tied range's bin of one value.
+// (lists, large planes), from the keys set aside (the bin's gathered in LDS first where many digits are to come
+// and they fit), or from the plane where the range missed the rank or its keys found no room.  A rank on a tied
+// range's end needs no digits, nor does a tied range's bin of one value.
 template <class T, bool MASKED>
 __global__ __launch_bounds__(kMT) void k_mad_pick(const T* __restrict__ planes, size_t plane, int w, Rect inc, Rect exc,
                                                   uint32_t count,
@@ -1441,13 +1441,18 @@ __global__ __launch_bounds__(NT) void k_ccl_tile(const T* __restrict__ w, int* _
   }
 }
 
-// Second level: unions across tile borders, one thread per bit word (a word spans a tile's width), so
-// that pixels without a set neighbour across a border cost no label access.  On the rows that start a
-// tile every pixel looks at the row above; on the others only the word's first and last pixel look at
-// the neighbouring words, and not where the neighbour above or beside them makes the same union.  Unions
-// commute: the roots, each component's smallest index, do not depend on their order.  The last
-// block of a plane reduces the plane's tile maxima instead (smax).  Reading the labels of every tile
-// border took 502 us on seven 4096^2 planes: with 32-pixel tiles that is every line of them.
+// Second level: unions across tile borders, so that pixels without a set neighbour across a border cost no label
+// access.  On the rows that start a tile every pixel looks at the row above: a thread takes kCclPart pixels of a word
+// there (a thread with a whole word makes up to 64 unions one after the other, each a chain of memory latencies: five
+// 500 x 517 planes with 45% set pixels took 98 us, now 25).  On the others only the word's
+// first and last pixel look at the neighbouring words, one thread a word, and not where the neighbour above or beside
+// them makes the same union.  Unions commute: the roots, each component's smallest index, do not depend on
+// their order.  The last block of a plane reduces the plane's tile maxima instead (smax).  Reading the labels of
+// every tile border took 502 us on seven 4096^2 planes: with 32-pixel tiles that is every line of them.
+constexpr int kCclPart = 4;
+__host__ __device__ __forceinline__ unsigned ccl_border_items(int h, int wd) {  // words, then parts of the top rows' words
+  return (unsigned)ccl_words(wd) * ((unsigned)h + (unsigned)((h + kCclH - 1) / kCclH) * (kCclW / kCclPart));
+}
 template <class T>
 __global__ __launch_bounds__(kT) void k_ccl_border(int* __restrict__ lab, const u64* __restrict__ bits, int h, int wd,
                                                    const T* __restrict__ pmax, int n_pmax, T* __restrict__ smax,
@@ -1465,33 +1470,41 @@ __global__ __launch_bounds__(kT) void k_ccl_border(int* __restrict__ lab, const 
     return;
   }
   const unsigned nw = ccl_words(wd);
-  const unsigned n = (unsigned)h * nw;
+  const unsigned n = (unsigned)h * nw, items = ccl_border_items(h, wd);
   int* l = lab + (size_t)s * h * wd;
   const u64* b = bits + (size_t)s * n;
-  for (unsigned i = blockIdx.x * kT + threadIdx.x; i < n; i += (gridDim.x - 1) * kT) {
+  for (unsigned it = blockIdx.x * kT + threadIdx.x; it < items; it += (gridDim.x - 1) * kT) {
+    const bool top = it >= n;
+    unsigned i = it, part = 0;
+    if (top) {
+      const unsigned k = (it - n) / (kCclW / kCclPart);  // word k of the rows that start a tile
+      part = (it - n) % (kCclW / kCclPart);
+      i = k / nw * (kCclH * nw) + k % nw;
+    }
     const u64 m = b[i];
     if (m == 0) continue;
     const int r = (int)(i / nw), cw = (int)(i - (unsigned)r * nw);
+    if (!top && r % kCclH == 0) continue;
     const int me = r * wd + cw * kCclW;  // the word's first pixel
     const bool has_l = cw > 0, has_r = cw + 1 < (int)nw;
     const u64 lw = has_l ? b[i - 1] >> 63 : 0;  // the pixel left of the word
     const u64 u = r > 0 ? b[i - nw] : 0;
     const u64 ulw = r > 0 && has_l ? b[i - nw - 1] >> 63 : 0;
     const u64 urw = r > 0 && has_r ? b[i - nw + 1] & 1 : 0;
-    const bool top = r % kCclH == 0;
-    if ((lw & m & 1) && (top || !(u & ulw & 1))) ccl_union(l, me, me - 1);
+    if ((top ? part == 0 : !(u & ulw & 1)) && (lw & m & 1)) ccl_union(l, me, me - 1);
     if (top) {
+      const u64 mine = (((u64)1 << kCclPart) - 1) << (part * kCclPart);
       u64 up, upl, upr;
       ccl_rules(m, (m << 1) | lw, u, (u << 1) | ulw, (u >> 1) | (urw << 63), &up, &upl, &upr);
-      for (; up; up &= up - 1) {
+      for (up &= mine; up; up &= up - 1) {
         const int c = me + __ffsll(up) - 1;
         ccl_union(l, c, c - wd);
       }
-      for (; upl; upl &= upl - 1) {
+      for (upl &= mine; upl; upl &= upl - 1) {
         const int c = me + __ffsll(upl) - 1;
         ccl_union(l, c, c - wd - 1);
       }
-      for (; upr; upr &= upr - 1) {
+      for (upr &= mine; upr; upr &= upr - 1) {
         const int c = me + __ffsll(upr) - 1;
         ccl_union(l, c, c - wd + 1);
       }
@@ -1516,12 +1529,19 @@ __global__ __launch_bounds__(kT) void k_ccl_flatten(int* __restrict__ lab, const
 }
 
 // Roots of the set ones (bits `on`) of four pixels from px on, walked side by side so that a step costs
-// one memory latency for all of them; returns which of the roots carry the keep mark.
-__device__ __forceinline__ unsigned ccl_find4(const int* lab, int px, unsigned on, int (&root)[4]) {
+// one memory latency for all of them; returns which of the roots carry the keep mark.  From the third link on a walk
+// (HALVE) leaves each label pointing at its grandparent: the pixels of an object that winds through many tiles halve its
+// chain of tile roots for one another (other walks read either link; roots, which carry the marks, are not written).
+template <bool HALVE>
+__device__ __forceinline__ unsigned ccl_find4(int* lab, int px, unsigned on, int (&root)[4]) {
+  int child[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) root[k] = (on >> k) & 1 ? lab[px + k] & ~kMark : 0;
+  for (int k = 0; k < 4; ++k) {
+    root[k] = (on >> k) & 1 ? lab[px + k] & ~kMark : 0;
+    child[k] = px + k;
+  }
   unsigned marked = 0, more = on;
-  while (more) {
+  for (int link = 1; more; ++link) {
     int p[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) p[k] = (more >> k) & 1 ? lab[root[k]] : 0;
@@ -1531,11 +1551,48 @@ __device__ __forceinline__ unsigned ccl_find4(const int* lab, int px, unsigned o
       if ((p[k] & ~kMark) == root[k]) {
         more &= ~(1u << k);
         marked |= p[k] < 0 ? 1u << k : 0u;
+      } else if constexpr (HALVE) {
+        if (link >= 3) lab[child[k]] = p[k];
+        child[k] = root[k];
       }
       root[k] = p[k] & ~kMark;
     }
   }
   return marked;
+}
+
+// The first step of the keep rule of small stacks: links the set pixels of all scales (blockIdx.y) to their roots and
+// marks the roots of the coarsest one's objects that hold a seed pixel (value >= tol * max).  A chain of tile roots is then
+// walked here, for all scales at once, and not scale after scale in the steps that follow: the extraction on five 600^2
+// planes of vertical lines takes 61 us (116 without this step), of one object winding through every tile 93 us (166).
+template <class T>
+__global__ __launch_bounds__(kT) void k_keep_first(const T* __restrict__ w, int* __restrict__ lab,
+                                                   const u64* __restrict__ bits, int S, const T* __restrict__ smax,
+                                                   double tol, int neg_comp, int h, int wd, const int* pred) {
+  if (pred_off(pred)) return;
+  const int s = blockIdx.y;
+  const unsigned nq = (unsigned)(wd + 3) / 4;
+  const unsigned i = blockIdx.x * (unsigned)kT + threadIdx.x;
+  if (i >= (unsigned)h * nq) return;
+  const int r = (int)(i / nq), c = 4 * (int)(i - (unsigned)r * nq);
+  const unsigned on = (unsigned)(bits[((size_t)s * h + r) * ccl_words(wd) + (c >> 6)] >> (c & 63)) & 15u;
+  if (on == 0) return;
+  const size_t o = (size_t)s * h * wd;
+  const int px = r * wd + c;
+  int* l = lab + o;
+  const bool mark = s == S - 1;
+  T v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = mark && ((on >> k) & 1) ? w[o + px + k] : (T)0;
+  const double lim = mark ? tol * (double)smax[s] : 0.0;
+  int root[4];
+  (void)ccl_find4<true>(l, px, on, root);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (!((on >> k) & 1)) continue;
+    if (root[k] != px + k && l[px + k] != root[k]) l[px + k] = root[k];  // a root's own word is left: it takes the mark
+    if (mark && (double)(neg_comp ? (T)fabs(v[k]) : v[k]) >= lim) l[root[k]] = root[k] | kMark;
+  }
 }
 
 // One step of the per-scale keep rule, coarsest scale first, in one pass over the pixels: applies
@@ -1545,9 +1602,11 @@ __device__ __forceinline__ unsigned ccl_find4(const int* lab, int px, unsigned o
 // pixels of a row: their bits come from the scales' words, requested for all of them first, labels
 // and values are read at set pixels
 // alone, and VEC (sides and buffers that keep quads aligned) writes the four extracted values and the
-// four mask bytes as one store each.  Roots are found by walking from the tile's root, so no pass
-// compresses the labels beforehand (162 us on seven 4096^2 planes).  Bound: the two outputs' stores:
-// 31 us a scale at 4096^2 (64 us on label planes with separate flags; 33 us with one quad a thread).
+// four mask bytes as one store each, with U > 1 past the caches: the extraction of seven 4096^2 planes takes 477 us
+// (499 through them), of three 3000^2 planes 115 us (139), which a reader of the outputs pays back only there (191
+// and 190 us with one).  Roots are found by walking from the tile's root, so on large stacks no pass
+// compresses the labels beforehand (162 us on seven 4096^2 planes; k_keep_first does on small ones).  Bound: the two
+// outputs' stores: 31 us a scale at 4096^2 (64 us on label planes with separate flags; 33 us with one quad a thread).
 template <class T, bool VEC, int U>
 __global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, int* __restrict__ lab,
                                                   const u64* __restrict__ bits, int sa, int sm,
@@ -1559,7 +1618,7 @@ __global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, int* 
   const unsigned nq = (unsigned)(wd + 3) / 4;
   const size_t plane = (size_t)h * wd;
   const size_t oa = (size_t)(sa < 0 ? 0 : sa) * plane, om = (size_t)(sm < 0 ? 0 : sm) * plane;
-  const int* la = lab + oa;
+  int* la = lab + oa;
   int* lm = lab + om;
   const u64* ba = bits + (size_t)(sa < 0 ? 0 : sa) * h * nw;
   const u64* bm = bits + (size_t)(sm < 0 ? 0 : sm) * h * nw;
@@ -1588,7 +1647,7 @@ __global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, int* 
       Quad<T> e;
 #pragma unroll
       for (int k = 0; k < 4; ++k) e.a[k] = (on >> k) & 1 ? w[oa + px[u] + k] : (T)0;
-      kept = on ? ccl_find4(la, px[u], on, root) : 0u;
+      kept = on ? ccl_find4<U == 1>(la, px[u], on, root) : 0u;
 #pragma unroll
       for (int k = 0; k < 4; ++k) e.a[k] = (kept >> k) & 1 ? e.a[k] : (T)0;
       uint8_t* mo = mask + oa + px[u];
@@ -1623,7 +1682,7 @@ __global__ __launch_bounds__(kT) void k_keep_step(const T* __restrict__ w, int* 
       if (!((double)v >= lim)) seeds &= ~(1u << k);
     }
     if (!seeds) continue;
-    (void)ccl_find4(lm, px[u], seeds, root);
+    (void)ccl_find4<U == 1>(lm, px[u], seeds, root);
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       if ((seeds >> k) & 1) lm[root[k]] = root[k] | kMark;
@@ -2147,7 +2206,7 @@ static void source_extract_t(const T* w, int S, int h, int wd, double tol, int n
     hipLaunchKernelGGL((k_ccl_tile<T, 128>), dim3(tiles, S), dim3(128), 0, st, w, lab, bits, h, wd, neg_comp, pmax,
                        pred);
   PMS_LAUNCH_CHECK();
-  const int gb = std::min(ceil_div(h * ccl_words(wd), kT), 1024);
+  const int gb = (int)std::min<unsigned>((ccl_border_items(h, wd) + kT - 1) / kT, 1024);
   hipLaunchKernelGGL(k_ccl_border<T>, dim3(gb + 1, S), dim3(kT), 0, st, lab, (const u64*)bits, h, wd, (const T*)pmax,
                      tiles, smax, pred);
   PMS_LAUNCH_CHECK();
@@ -2160,7 +2219,16 @@ static void source_extract_t(const T* w, int S, int h, int wd, double tol, int n
   const unsigned per = kT * (four ? 4 : 1);
   auto keep = vec ? (four ? k_keep_step<T, true, 4> : k_keep_step<T, true, 1>)
                   : (four ? k_keep_step<T, false, 4> : k_keep_step<T, false, 1>);
-  for (int sa = S; sa >= 0; --sa) {
+  // On more tiles the walks of a step's pixels hide behind one another, and reading every label once more costs more than it
+  // saves: 1% set pixels on five 600^2 planes (950 tiles) 34 -> 32 us, on seven of 700^2 (1694) 46 -> 49, three of 1400^2
+  // (2904) 39 -> 44; lines and winding objects there 162 -> 95, 338 -> 153 and 152 -> 105, 191 -> 139.
+  const bool first = (size_t)tiles * S <= 2048;
+  if (first) {
+    hipLaunchKernelGGL(k_keep_first<T>, dim3((quads + kT - 1) / kT, S), dim3(kT), 0, st, w, lab, (const u64*)bits, S,
+                       (const T*)smax, tol, neg_comp, h, wd, pred);
+    PMS_LAUNCH_CHECK();
+  }
+  for (int sa = first ? S - 1 : S; sa >= 0; --sa) {
     hipLaunchKernelGGL(keep, dim3((quads + per - 1) / per), dim3(kT), 0, st, w, lab, (const u64*)bits,
                        sa < S ? sa : -1, sa - 1, (const T*)smax, tol, neg_comp, h, wd, mask, extracted, pred);
     PMS_LAUNCH_CHECK();
