@@ -1244,6 +1244,19 @@ bool tile2_range(int h, int w, int s, int jobs, bool recomp) {
   return s <= top;
 }
 
+// Tile size of a launch of `jobs` planes: 32 where that gives a tile to each CU and the phases fill their tiles at least half
+// as well as 16 x 16 ones do.  Pairs of one plane, decomposition (recomposition) with 16 and with 32: 512^2 (256 tiles) five scales
+// 20.6 -> 17.9 us (14.2 -> 13.6), 601 x 1000 (608 to 640 tiles) 34.0 -> 24.7 us (23.7 -> 19.3); 350^2 (121 to 144 tiles) 18.2 -> 17
+// (12.6 -> 13), 256^2 (64 tiles) 8.6 -> 11.4 us (7.0 -> 9.7).
+// A recomposition whose phases have at most 16 rows keeps 16 x 16: half the rows of a wider tile's column sums are idle there
+// (64 x 2048, five scales, 11.4 us with 16 and 12.4 with 32; 256 x 2048, seven, 28.6 and 31.3; the turned planes gain 5% from 32).
+bool tile2_fits(int h, int w, int s, int jobs, bool recomp) {
+  const int d = 1 << s, rows = ceil_div(h, d), cols = ceil_div(w, d);
+  const long small = (long)d * d * ceil_div(rows, kTile2) * ceil_div(cols, kTile2);
+  const long tiles = tile2_tiles(h, w, s);
+  return tiles * jobs >= 256 && 2 * tiles <= small && !(recomp && rows <= kTile2);
+}
+
 dim3 small_grid(int h, int w) { return dim3(ceil_div(w, 64), ceil_div(h, 4)); }
 
 static ScaleJob scale_job(const IuwtScaleCall& c) {

@@ -17,6 +17,9 @@
 #include "iuwt_small2.h"
 
 namespace pms {
+
+bool tile2_fits(int h, int w, int s, int jobs, bool recomp);  // iuwt.hip
+
 namespace {
 
 constexpr int kTile32 = 32;
@@ -443,26 +446,17 @@ void tile2_rec_batch(const PairJobT<T>* jobs, int count, int h, int w, int s, hi
   }
 }
 
-// Tile size of a launch of `jobs` planes: 32 where that gives a tile to each CU and the phases fill their tiles at least half
-// as well as 16 x 16 ones do.  Pairs of one plane, decomposition (recomposition) with 16 and with 32: 512^2 (256 tiles) five scales
-// 20.6 -> 17.9 us (14.2 -> 13.6), 601 x 1000 (608 to 640 tiles) 34.0 -> 24.7 us (23.7 -> 19.3); 350^2 (121 to 144 tiles) 18.2 -> 17
-// (12.6 -> 13), 256^2 (64 tiles) 8.6 -> 11.4 us (7.0 -> 9.7).
-inline bool tile2_fits(int h, int w, int s, int jobs) {
-  const int d = 1 << s;
-  const long small = (long)d * d * ceil_div(ceil_div(h, d), kTile2) * ceil_div(ceil_div(w, d), kTile2);
-  const long tiles = tile2_tiles(h, w, s);
-  return tiles * jobs >= 256 && 2 * tiles <= small;
-}
+// a pair's launch with the tile size that tile2_fits names (32 or 16)
 template <class T>
 void pair_dec_batch(const Dec2JobT<T>* jobs, int count, int h, int w, int s, hipStream_t st) {
-  if (tile2_fits(h, w, s, count))
+  if (tile2_fits(h, w, s, count, false))
     tile2_dec_batch<T>(jobs, count, h, w, s, st);
   else
     small2_dec_batch<T>(jobs, count, h, w, s, st);
 }
 template <class T>
 void pair_rec_batch(const PairJobT<T>* jobs, int count, int h, int w, int s, hipStream_t st) {
-  if (tile2_fits(h, w, s, count))
+  if (tile2_fits(h, w, s, count, true))
     tile2_rec_batch<T>(jobs, count, h, w, s, st);
   else
     small2_rec_batch<T>(jobs, count, h, w, s, st);
