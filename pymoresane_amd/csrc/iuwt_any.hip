@@ -195,8 +195,22 @@ int iuwt_gen_scale_batch(const IuwtScaleCallT<T>* calls, int count, hipStream_t 
 template int iuwt_gen_scale_batch<float>(const IuwtScaleCallT<float>*, int, hipStream_t);
 template int iuwt_gen_scale_batch<double>(const IuwtScaleCallT<double>*, int, hipStream_t);
 
+// Whether scales (s, s+1) of a float64 transform of `jobs` planes run as one launch.  Both have to be within the side, and
+// the phases of scale s long enough for the 16 x 16 tiles (a tile of a phase of 4 x 4 positions stages 36 x 36): at least
+// 16 positions in a decomposition, 32 in a recomposition, whose single scales are one launch each.  Launches of few pixels
+// last as long as their launches are many and pair more.  Decomposition (recomposition) of all scales, us, every pair
+// against this rule: 64^2 14 (12) either way, 256^2 46 -> 31 (32 -> 21), 512^2 75 -> 71 (52 -> 45), 1024^2 466 -> 206 (314 -> 128),
+// 2048^2 942 -> 819 (730 -> 562), 4096^2 8000 -> 3822 (5805 -> 2552); one scale a launch 36 (19), 51 (26), 102 (54), 290 (150),
+// 1201 (683), 5997 (3214).
+bool gen_pair_applies(int h, int w, int s, int jobs, bool recomp) {
+  if (iuwt_over_long(h, w, s + 1)) return false;
+  const long px = (long)h * w * jobs;
+  const int least = px <= 1L << 14 ? 1 : recomp && px > 1L << 16 ? 32 : 16;
+  return (std::min(h, w) >> s) >= least;
+}
+
 // float64 decomposition over all jobs: pre-smoothing below scale_adjust, then pairs of scales in one launch each where
-// both are within the side and no reference is reduced, the rest scale by scale; C ping-pongs
+// gen_pair_applies and no reference is reduced, the rest scale by scale; C ping-pongs
 // through the job's two work planes.
 void iuwt_decompose_batch(IuwtDecompJobT<double>* jobs, int count, int h, int w, hipStream_t st) {
   const size_t plane = (size_t)h * w;
@@ -236,7 +250,7 @@ void iuwt_decompose_batch(IuwtDecompJobT<double>* jobs, int count, int h, int w,
         } else {
           if (s < j.scale_adjust || s >= j.scale_count || s < done[k]) continue;
           const int kk = s - j.scale_adjust;
-          if (s + 1 < j.scale_count && j.detail && !j.ref && !iuwt_over_long(h, w, s + 1)) {
+          if (s + 1 < j.scale_count && j.detail && !j.ref && gen_pair_applies(h, w, s, count, false)) {
             Dec2JobT<double> pj{};
             pj.in = cur[k];
             pj.out_c = s + 1 == j.scale_count - 1 ? j.smoothed : ping;
@@ -287,7 +301,7 @@ long iuwt_decompose_partials_f64(int h, int w, int scale_count, int scale_adjust
 }
 
 // float64 recomposition from the coarsest kept scale down: pairs of detail scales in one launch each
-// (from the finest up, so that an odd scale is left at the top) where both are within the side, one launch per
+// (from the finest up, so that an odd scale is left at the top) where gen_pair_applies, one launch per
 // scale otherwise; jobs at the same step share launches.
 void iuwt_recompose_batch(const IuwtRecompJobT<double>* jobs, int count, int h, int w, hipStream_t st) {
   const size_t plane = (size_t)h * w;
@@ -325,7 +339,7 @@ void iuwt_recompose_batch(const IuwtRecompJobT<double>* jobs, int count, int h, 
     }
     bool odd_top = s >= j.scale_adjust && (s - j.scale_adjust + 1) % 2 == 1;
     while (s >= 0) {
-      const bool pair = !odd_top && s - 1 >= j.scale_adjust && !iuwt_over_long(h, w, s);
+      const bool pair = !odd_top && s - 1 >= j.scale_adjust && gen_pair_applies(h, w, s - 1, count, true);
       odd_top = false;
       sk.ops.push_back(pair ? Op{OP_PAIR, s - 1} : Op{s >= j.scale_adjust ? OP_RECOMP : OP_SMOOTH, s});
       s -= pair ? 2 : 1;
