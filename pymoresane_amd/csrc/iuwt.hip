@@ -1235,12 +1235,17 @@ bool small2_applies(bool small, int h, int w, int s) {
 // 3000^2 180 -> 170 (147 -> 141), 4096^2 282 -> 285 (236 -> 237); pair (2,3): 1024^2 46 -> 38 (39 -> 33), 1600^2 76 -> 66
 // (53 -> 53), 2048^2 103 -> 98 (75 -> 76), 3000^2 170 -> 180 (141 -> 160); pair (4,5): 800^2 34 -> 43 (32 -> 30.5), 1024^2 38 -> 46
 // (33 -> 31), 1300^2 56 -> 77 (41 -> 51).
+// Masked launches, whose tiles read one mask byte in every 2^s, leave them sooner: decompositions (recompositions) of four
+// scales, walks against pair (0,1) on tiles, 16 planes of 700^2 162 -> 142 us (76 -> 75), two of 2048^2 92 -> 96 (85 -> 75), 32 of
+// 600^2 217 -> 217 (116 -> 121), 3000^2 128 -> 121 (84 -> 90), twelve of 1024^2 138 -> 174 (124 -> 126), three of 2048^2 127 -> 175
+// (112 -> 121).
 // PMS_IUWT_SMALL_LAUNCH=0 keeps planes above 256^2 on the walks, and PMS_IUWT_DEC2 or PMS_IUWT_PAIR, when set, say how
 // those take the scales of a decomposition or a recomposition: no tiles then (all read per call).
-bool tile2_range(int h, int w, int s, int jobs, bool recomp) {
+bool tile2_range(int h, int w, int s, int jobs, bool masked, bool recomp) {
   if (env_int("PMS_IUWT_SMALL_LAUNCH", 1) == 0 || getenv(recomp ? "PMS_IUWT_PAIR" : "PMS_IUWT_DEC2")) return false;
   const long px = (long)h * w * jobs;
-  const int top = px <= 1L << 20 ? (recomp ? 4 : 2) : px <= 1L << 22 ? 2 : px <= 3L << 22 ? 0 : -1;
+  const long most = !masked ? 3L << 22 : recomp ? 1L << 23 : 15L << 19;
+  const int top = px <= 1L << 20 ? (recomp ? 4 : 2) : px <= 1L << 22 ? 2 : px <= most ? 0 : -1;
   return s <= top;
 }
 
@@ -1384,6 +1389,7 @@ static void decompose_batch_impl(IuwtDecompJob* jobs, int count, int h, int w, b
   };
   std::vector<State> state(count);
   int smax = 0;
+  const bool masked = std::any_of(jobs, jobs + count, [](const IuwtDecompJob& j) { return j.mask != nullptr; });
   for (int k = 0; k < count; ++k) {
     IuwtDecompJob& j = jobs[k];
     PMS_REQUIRE(j.scale_adjust >= 0 && j.scale_count > j.scale_adjust, "need scale_count > scale_adjust >= 0");
@@ -1410,7 +1416,7 @@ static void decompose_batch_impl(IuwtDecompJob* jobs, int count, int h, int w, b
       pairs.clear();
       pwho.clear();
       Plan pl;
-      const bool small_pair = mode == IUWT_DECOMP && small2_applies(small || tile2_range(h, w, s, count, false), h, w, s);
+      const bool small_pair = mode == IUWT_DECOMP && small2_applies(small || tile2_range(h, w, s, count, masked, false), h, w, s);
       const bool pair_plan = small_pair || (!small && fuse == 1 && mode == IUWT_DECOMP && dec2_plan(h, w, s, &pl));
       for (int k = 0; k < count; ++k) {
         const IuwtDecompJob& j = jobs[k];
@@ -1524,6 +1530,7 @@ static void recompose_batch_impl(const IuwtRecompJob* jobs, int count, int h, in
   // PMS_IUWT_PAIR=0 keeps every scale in its own launch, 1 pairs detail scales from the coarsest
   // down, 2 from the finest up (read per call, and it overrides the autotuner's record; the results
   // are identical)
+  const bool masked = std::any_of(jobs, jobs + count, [](const IuwtRecompJob& j) { return j.mask != nullptr; });
   const int pair = getenv("PMS_IUWT_PAIR") ? env_int("PMS_IUWT_PAIR", 2) : (t_active ? t_active->pair : 2);
   for (int k = 0; k < count; ++k) {
     const IuwtRecompJob& j = jobs[k];
@@ -1559,7 +1566,7 @@ static void recompose_batch_impl(const IuwtRecompJob* jobs, int count, int h, in
       const bool own_out = s != 1 || !(overlaps(j.out, pb, j.detail + plane, pb) ||
                                        (sk.ops.empty() && overlaps(j.out, pb, sk.cur, pb)));
       if (pair && own_out && s - 1 >= j.scale_adjust &&
-          (small2_applies(small || tile2_range(h, w, s - 1, count, true), h, w, s - 1) ||
+          (small2_applies(small || tile2_range(h, w, s - 1, count, masked, true), h, w, s - 1) ||
            (!small && recomp2_plan(h, w, s - 1, &pl)))) {
         sk.ops.push_back({OP_PAIR, s - 1});
         s -= 2;
@@ -1621,7 +1628,7 @@ static void recompose_batch_impl(const IuwtRecompJob* jobs, int count, int h, in
       }
       if (op0.kind == OP_PAIR) {
         Plan pl;
-        if (small2_applies(small || tile2_range(h, w, op0.s, count, true), h, w, op0.s)) {
+        if (small2_applies(small || tile2_range(h, w, op0.s, count, masked, true), h, w, op0.s)) {
           pair_rec_batch<float>(pairs.data(), (int)pairs.size(), h, w, op0.s, st);
         } else {
           PMS_REQUIRE(recomp2_plan(h, w, op0.s, &pl), "two-scale recomposition plan changed");
