@@ -116,7 +116,7 @@ class Job {
   Job(const Job&) = delete;
   Job& operator=(const Job&) = delete;
   // grow-only allocation for geometry g; returns true when buffers moved
-  bool ensure(const Geometry& g, hipStream_t st);
+  bool ensure(const Geometry& g);
   template <class T>
   T* by_scale_dirty(size_t n2);  // private copy of the dirty image for moresane_by_scale
   size_t device_bytes() const { return arena_.bytes() + by_scale_arena_.bytes(); }

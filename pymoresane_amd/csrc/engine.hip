@@ -668,7 +668,7 @@ static void carve(Planes<T>& P, const JobSizes& z, DeviceArena& arena) {
 }
 
 // Buffers grow to the largest geometry seen and are reused by smaller jobs of the same precision.
-bool Job::ensure(const Geometry& g, hipStream_t st) {
+bool Job::ensure(const Geometry& g) {
   const int S = std::max(g.S, (int)std::log2((double)g.n) - 1);
   const JobSizes need = job_sizes(g, S);
   geo_ = g;
@@ -886,7 +886,7 @@ void Task::enqueue_setup(hipStream_t st) {
   int sub = 0;
   Geometry g = make_geometry(prm.n, prm.psf_n, prm, scale_count_, &sub);
   Job& J = *job_;
-  if (J.ensure(g, st) || !x_) {
+  if (J.ensure(g) || !x_) {
     moved_ = true;
     Planes<T>& P = J.pl<T>();
     x_ = P.x;

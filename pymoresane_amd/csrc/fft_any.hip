@@ -818,7 +818,7 @@ void set_g_attrs() {
       (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
     };
     allow((const void*)k_g_r2c<T, float, false, 1>);
-    allow((const void*)k_g_r2c<T, double, false, 1>);
+    if constexpr (sizeof(T) == 8) allow((const void*)k_g_r2c<T, double, false, 1>);
     allow((const void*)k_g_r2c<T, T, true, 1>);
     allow((const void*)k_g_r2c<T, T, false, kMaxBatch>);
     allow((const void*)k_g_r2c<T, T, true, kMaxBatch>);

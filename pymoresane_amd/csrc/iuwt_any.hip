@@ -16,7 +16,8 @@
 // the vertical combination, as the row-walk kernels do).  A decomposition scale is two launches:
 // SMOOTH writes C, DETAIL reads C0 at the centre and C around it and writes w (optionally masked,
 // or reduced against a reference plane).  The float32 transforms (iuwt.hip) use this for the
-// scales beyond the row walks' range; the float64 transforms use it at every scale.
+// scales beyond the row walks' range; the float64 transforms, at the end of this file, run pairs of scales on
+// the kernels of iuwt_small2.h and the other scales on this one.
 #include <algorithm>
 #include <vector>
 

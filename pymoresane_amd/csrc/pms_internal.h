@@ -199,7 +199,7 @@ void iuwt_recompose_batch(const IuwtRecompJob* jobs, int count, int h, int w, hi
 // Direct-stencil IUWT (iuwt_any.hip) with the reference's exact tap semantics at every scale,
 // including scales whose taps are longer than the side (2^(s+1) > side: numpy's clipped slices
 // read the axis reversed, iuwt.py:166-187).  The float32 transforms above route such scales here;
-// the float64 transforms use it at every scale.  A decomposition scale is two launches (smooth,
+// the float64 transforms use it for the scales that do not run in pairs (iuwt_small2.h).  A decomposition scale is two launches (smooth,
 // then detail = C0 - smooth(C)), so its call needs out_c (a free work plane when not kept).
 bool iuwt_over_long(int h, int w, int scale);
 int iuwt_gen_blocks(int h, int w);  // partial sums per plane written by a reducing detail launch

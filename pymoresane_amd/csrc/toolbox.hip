@@ -3,10 +3,12 @@
 //
 // Semantics follow pymoresane/iuwt_toolbox.py:
 //   estimate_threshold (17-48) : median(|w| over the noise mask) / 0.6745,
-//                                exact: radix select on the float bits of |w|
+//                                exact: selection by the float bits of |w|
 //                                (non-negative floats order like unsigned ints),
-//                                np.median's mean of the two middle values for
-//                                even counts;
+//                                in one reading of the planes through a sampled
+//                                range of keys, or as a radix select where there
+//                                is no workspace for that; np.median's mean of
+//                                the two middle values for even counts;
 //   apply_threshold (50-75)    : w where |w| > sigma * t (strict), else 0;
 //   source_extraction (97-154) : 8-connected labels of non-zero pixels by
 //                                union-find with atomicMin links (every root is
@@ -129,19 +131,16 @@ struct MadKey<double> {
   __device__ static double val(K k) { return __longlong_as_double((long long)k); }
 };
 
-// per-plane select state (32 bytes for either key width)
-template <class K>
-struct alignas(16) SelStateT {
-  K prefix;          // fixed high bits of the target key
-  K hi_key;          // min key above the low median (for even counts)
+// per-plane select state of the radix select
+struct alignas(16) SelState {
+  uint32_t prefix;   // fixed high bits of the target key
+  uint32_t hi_key;   // min key above the low median (for even counts)
   uint32_t rank;     // remaining rank of the low median inside the prefix bucket
   uint32_t eq;       // count of keys equal to the final low median
-  uint32_t first;    // rank of the first key equal to the low median
   uint32_t n;        // number of keys
 };
 constexpr size_t kSelBytes = 32;
-static_assert(sizeof(SelStateT<uint32_t>) <= kSelBytes && sizeof(SelStateT<unsigned long long>) <= kSelBytes,
-              "select state exceeds its slot");
+static_assert(sizeof(SelState) <= kSelBytes, "select state exceeds its slot");
 
 constexpr int kBins = 2048;
 constexpr int kMaxPlanes = 16;  // plane stacks handled per call (scale counts up to 16)
@@ -150,25 +149,25 @@ constexpr int kMaxPlanes = 16;  // plane stacks handled per call (scale counts u
 // `above` set (the last digit), keys whose higher digits exceed the prefix are all larger than the
 // low median: the smallest of them goes to hi_key (atomic min), where the last select finds it if
 // the low median's bucket holds no larger key (the successor of even counts, without a pass of its own).
-template <class T, bool MASKED>
-__global__ __launch_bounds__(kT) void k_mad_hist(const T* __restrict__ planes, size_t plane, int w, Rect inc,
+template <bool MASKED>
+__global__ __launch_bounds__(kT) void k_mad_hist(const float* __restrict__ planes, size_t plane, int w, Rect inc,
                                                  Rect exc, int shift, int nbits, int prefix_shift, int above,
-                                                 SelStateT<typename MadKey<T>::K>* __restrict__ st,
-                                                 uint32_t* __restrict__ hist, const int* pred) {
-  using K = typename MadKey<T>::K;
+                                                 SelState* __restrict__ st, uint32_t* __restrict__ hist,
+                                                 const int* pred) {
+  using K = uint32_t;
   if (pred_off(pred)) return;
   __shared__ uint32_t h[kBins];
   const int s = blockIdx.y;
   for (int i = threadIdx.x; i < kBins; i += kT) h[i] = 0;
   __syncthreads();
-  const T* x = planes + (size_t)s * plane;
+  const float* x = planes + (size_t)s * plane;
   const K pre = st[s].prefix;
   const K dmask = ((K)1 << nbits) - 1;
   const K none = ~(K)0;
   K best = none;
-  auto add = [&](T v) {
-    const K key = MadKey<T>::key(v);
-    if (prefix_shift < (int)(8 * sizeof(K))) {
+  auto add = [&](float v) {
+    const K key = MadKey<float>::key(v);
+    if (prefix_shift < 32) {
       const K kp = key >> prefix_shift, pp = pre >> prefix_shift;
       if (kp != pp) {
         if (above && kp > pp && key < best) best = key;
@@ -178,10 +177,7 @@ __global__ __launch_bounds__(kT) void k_mad_hist(const T* __restrict__ planes, s
     atomicAdd(&h[(uint32_t)((key >> shift) & dmask)], 1u);
   };
   const size_t stride = (size_t)gridDim.x * kT;
-  bool vec = false;
-  if constexpr (!MASKED && sizeof(T) == 4) vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-  if constexpr (sizeof(T) == 4) {
-    if (vec) {
+  if (!MASKED && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
     // eight keys per thread and iteration, loaded as two float4 before any histogram update, so a
     // thread has two loads in flight instead of one per atomic (the counts do not depend on order)
     const float4* x4 = reinterpret_cast<const float4*>(x);
@@ -196,9 +192,7 @@ __global__ __launch_bounds__(kT) void k_mad_hist(const T* __restrict__ planes, s
       add(a.x), add(a.y), add(a.z), add(a.w);
     }
     for (size_t j = 4 * n4 + blockIdx.x * (size_t)kT + threadIdx.x; j < plane; j += stride) add(x[j]);
-    }
-  }
-  if (!vec) {
+  } else {
     for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < plane; i += stride) {
       if (MASKED) {
         const int r = (int)(i / w), c = (int)(i % w);
@@ -230,9 +224,9 @@ __global__ __launch_bounds__(kT) void k_mad_hist(const T* __restrict__ planes, s
 }
 
 // one block per plane: locate the bucket holding the target rank, extend the prefix, clear the histogram
-template <class K>
-__global__ __launch_bounds__(kT) void k_mad_select(SelStateT<K>* st, uint32_t* hist, int shift, int nbits, int last,
+__global__ __launch_bounds__(kT) void k_mad_select(SelState* st, uint32_t* hist, int shift, int nbits, int last,
                                                    const int* pred) {
+  using K = uint32_t;
   if (pred_off(pred)) return;
   const int s = blockIdx.x;
   uint32_t* gh = hist + (size_t)s * kBins;
@@ -240,7 +234,7 @@ __global__ __launch_bounds__(kT) void k_mad_select(SelStateT<K>* st, uint32_t* h
   __shared__ uint32_t part[kT];
   const int nb = 1 << nbits;
   const int per = kBins / kT;  // 8 bins per thread
-  const SelStateT<K> S0 = st[s];  // read by every thread before the barrier; one thread writes it after
+  const SelState S0 = st[s];  // read by every thread before the barrier; one thread writes it after
   uint32_t local = 0;
   for (int k = 0; k < per; ++k) {
     const int b = threadIdx.x * per + k;
@@ -266,10 +260,10 @@ __global__ __launch_bounds__(kT) void k_mad_select(SelStateT<K>* st, uint32_t* h
   // the thread whose range of ranks [exc, inc) holds the target rank finishes the search (the
   // last thread also takes a rank beyond the total, as the serial scan did)
   const bool mine = (S0.rank >= exc && S0.rank < inc) || (threadIdx.x == kT - 1 && S0.rank >= inc);
-  __shared__ SelStateT<K> s_state;
+  __shared__ SelState s_state;
   __shared__ int s_bin;
   if (mine) {
-    SelStateT<K> S = S0;
+    SelState S = S0;
     uint32_t run = exc;
     const int t = threadIdx.x;
     int b = t * per;
@@ -306,39 +300,37 @@ __global__ __launch_bounds__(kT) void k_mad_select(SelStateT<K>* st, uint32_t* h
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int k = 1; k < kT / 64; ++k) nxt = s_nxt[k] < nxt ? s_nxt[k] : nxt;
-    SelStateT<K> S = s_state;
+    SelState S = s_state;
     const K dm = (((K)1 << nbits) - 1) << shift;  // this digit's bits
     if (nxt < nb) S.hi_key = (S.prefix & ~dm) | ((K)nxt << shift);
     st[s] = S;
   }
 }
 
-template <class K>
-__global__ void k_mad_init(SelStateT<K>* st, int S, uint32_t n) {
+__global__ void k_mad_init(SelState* st, int S, uint32_t n) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= S) return;
-  SelStateT<K> z{};
+  SelState z{};
   z.n = n;
   z.rank = (n - 1) / 2;
   z.prefix = 0;
-  z.hi_key = ~(K)0;  // lowered by the last histogram pass and the last select
+  z.hi_key = ~0u;  // lowered by the last histogram pass and the last select
   st[s] = z;
 }
 
-template <class T>
-__global__ void k_mad_finish(const SelStateT<typename MadKey<T>::K>* st, int S, double* thr, const int* pred) {
+__global__ void k_mad_finish(const SelState* st, int S, double* thr, const int* pred) {
   if (pred_off(pred)) return;
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= S) return;
-  const SelStateT<typename MadKey<T>::K> z = st[s];
+  const SelState z = st[s];
   const uint32_t klo = (z.n - 1) / 2;
-  const T vlo = MadKey<T>::val(z.prefix);
+  const float vlo = MadKey<float>::val(z.prefix);
   double med = (double)vlo;
   if ((z.n & 1u) == 0) {
     // rank of the last key equal to vlo = first + eq - 1, first = klo - remaining rank
     const uint32_t first = klo - z.rank;
     const uint32_t lastr = first + z.eq - 1;
-    const T vhi = (klo + 1 <= lastr) ? vlo : MadKey<T>::val(z.hi_key);
+    const float vhi = (klo + 1 <= lastr) ? vlo : MadKey<float>::val(z.hi_key);
     med = ((double)vlo + (double)vhi) * 0.5;
   }
   thr[s] = med / 0.6745;
@@ -364,7 +356,8 @@ __device__ __forceinline__ void store_stream(T* p, const Quad<T>& q) {
 }
 
 // ---- median in one reading of the planes -------------------------------------------------------
-// The radix select above reads a plane once per digit.  With a workspace for it, a plane is read once:
+// The radix select above (float32, for callers without a workspace and planes of 2^32 pixels) reads a plane once per
+// digit.  With a workspace for it, a plane is read once:
 //   * planes of at most 32768 noise pixels are selected by one block with the keys in registers;
 //   * larger ones are sampled (k_mad_pivot: one block a plane, a radix select on the sample) for a range of
 //     keys [lo, lo + range] around the median.  The sample is groups of four neighbours; were the four
@@ -1150,7 +1143,8 @@ __global__ __launch_bounds__(kMT) void k_mad_pick(const T* __restrict__ planes, 
 }
 
 // ----------------------------------------------------------------------------- threshold + maxima
-// The same for planes whose quads are aligned: four quads in flight a thread, STREAM: the output goes past the caches
+// out = in where |in| > sigma * thr[s] (zero in the plane's border), and the outputs' maxima per block.
+// k_threshold4: planes whose quads are aligned, four quads in flight a thread, STREAM: the output goes past the caches
 // (launches that exceed them, see past_caches).  Bound: its bytes, 5.5 TB/s on seven 4096^2 planes: 171 us, 217 us one value at
 // a time through the caches; the noise estimate that reads the input planes next finds more of them cached (142 -> 113 us).
 template <class T, bool STREAM>
@@ -1198,6 +1192,7 @@ __global__ __launch_bounds__(kT) void k_threshold4(const T* __restrict__ in, T* 
   if (threadIdx.x == 0) pmax[(size_t)s * gridDim.x + blockIdx.x] = m;
 }
 
+// any other plane, a value at a time
 template <class T>
 __global__ __launch_bounds__(kT) void k_threshold(const T* __restrict__ in, T* __restrict__ out, size_t plane, int w,
                                                   const double* __restrict__ thr, double sigma,
@@ -1995,61 +1990,42 @@ static void mad_select_init(void* work, hipStream_t st) {
   fill_u32(hist, (size_t)kMaxPlanes * kBins, 0u, st);
 }
 
-// Exact median per plane: radix select over the key bits in digits of at most 11 bits, one
-// histogram pass and one select step per digit; for even counts the last pass and select also find
-// the successor of the low median.
 static void check_mad(int S, const NoiseMask& nm) {
   PMS_REQUIRE(nm.count > 0, "noise mask selects no pixels");
   PMS_REQUIRE(nm.count < (1L << 32), "plane too large for the median");
   PMS_REQUIRE(S >= 1 && S <= kMaxPlanes, "the median handles 1..16 planes per call");
 }
 
-// the form for a workspace of kNoAllocMadBytes
+// Exact median per plane for a workspace of kNoAllocMadBytes: radix select over the key bits in digits of at most
+// 11 bits (11/11/10), one histogram pass and one select step per digit; for even counts the last pass and select
+// also find the successor of the low median.
 void mad_thresholds_noalloc(const float* planes, int S, int h, int w, const NoiseMask& nm, double* thr, void* work,
                             const int* pred, hipStream_t st) {
-  using T = float;
-  using K = typename MadKey<T>::K;
   check_mad(S, nm);
   // the histograms hold the previous call's contents (the select state is rewritten by the first kernel)
   mad_select_init(work, st);
-  SelStateT<K>* sst = (SelStateT<K>*)work;
+  SelState* sst = (SelState*)work;
   uint32_t* hist = (uint32_t*)((char*)work + (size_t)kMaxPlanes * kSelBytes);
   const size_t plane = (size_t)h * w;
   Rect inc{nm.inc_r0, nm.inc_r1, nm.inc_c0, nm.inc_c1};
   Rect exc{nm.exc_r0, nm.exc_r1, nm.exc_c0, nm.exc_c1};
-  hipLaunchKernelGGL(k_mad_init<K>, dim3(ceil_div(S, 64)), dim3(64), 0, st, sst, S, (uint32_t)nm.count);
+  hipLaunchKernelGGL(k_mad_init, dim3(ceil_div(S, 64)), dim3(64), 0, st, sst, S, (uint32_t)nm.count);
   PMS_LAUNCH_CHECK();
   const int gx = std::min(ew_grid(plane), 512);
-  // digits of 11 bits from the top of the key word (its sign bit is always clear); the last digit
-  // takes what is left: 11/11/10 bits for float, 11 x 5 + 9 for double
-  constexpr int kKeyBits = 8 * sizeof(K);
-  constexpr int kPasses = (kKeyBits + 10) / 11;
-  int shifts[kPasses], bits[kPasses];
-  for (int pass = 0, top = kKeyBits; pass < kPasses; ++pass) {
-    bits[pass] = std::min(11, top);
-    top -= bits[pass];
-    shifts[pass] = top;
-  }
-  // even counts also need the smallest key above the low median: the last histogram pass and the
-  // last select find it on the way
+  constexpr int shifts[] = {21, 10, 0}, bits[] = {11, 11, 10};
   const int above = (nm.count & 1) == 0 ? 1 : 0;
-  for (int pass = 0; pass < kPasses; ++pass) {
-    const int pshift = (pass == 0) ? (int)(8 * sizeof(K)) : shifts[pass - 1];
-    const int ab = pass == kPasses - 1 ? above : 0;
-    if (nm.masked)
-      hipLaunchKernelGGL((k_mad_hist<T, true>), dim3(gx, S), dim3(kT), 0, st, planes, plane, w, inc, exc,
-                         shifts[pass], bits[pass], pshift, ab, sst, hist, pred);
-    else
-      hipLaunchKernelGGL((k_mad_hist<T, false>), dim3(gx, S), dim3(kT), 0, st, planes, plane, w, inc, exc,
-                         shifts[pass], bits[pass], pshift, ab, sst, hist, pred);
+  for (int pass = 0; pass < 3; ++pass) {
+    const int pshift = pass == 0 ? 32 : shifts[pass - 1], ab = pass == 2 ? above : 0;
+    hipLaunchKernelGGL((nm.masked ? k_mad_hist<true> : k_mad_hist<false>), dim3(gx, S), dim3(kT), 0, st, planes, plane, w,
+                       inc, exc, shifts[pass], bits[pass], pshift, ab, sst, hist, pred);
     PMS_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_mad_select<K>, dim3(S), dim3(kT), 0, st, sst, hist, shifts[pass], bits[pass],
-                       pass == kPasses - 1, pred);
+    hipLaunchKernelGGL(k_mad_select, dim3(S), dim3(kT), 0, st, sst, hist, shifts[pass], bits[pass], pass == 2, pred);
     PMS_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_mad_finish<T>, dim3(ceil_div(S, 64)), dim3(64), 0, st, (const SelStateT<K>*)sst, S, thr, pred);
+  hipLaunchKernelGGL(k_mad_finish, dim3(ceil_div(S, 64)), dim3(64), 0, st, (const SelState*)sst, S, thr, pred);
   PMS_LAUNCH_CHECK();
 }
+
 // Exact median per plane in one reading of it (k_mad_one, or k_mad_pivot / k_mad_scan / k_mad_pick).
 // The sample has 8192 keys below 2^20 noise pixels and 16384 above: a range of 8.8 and 6.3% of the
 // plane (32768: 4.4%, 35 instead of 20 us in k_mad_pivot for 4 us less in k_mad_scan).  From 2^20 pixels on the
